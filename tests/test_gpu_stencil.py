@@ -372,3 +372,24 @@ def test_pair_arithmetic_short_sequences_are_exact():
     out = (ctypes.c_uint64 * 4)()
     _lib.check(L.wrach_check_pair_arithmetic(0, out))
     assert list(out) == [0, 0, 805306370, 402653185]
+
+
+@pytest.mark.parametrize("row", [1, 3, 4, 5, 8, 9, 13, 31, 32, 33, 36])
+@pytest.mark.parametrize("n", [255, 257, 1000])
+def test_stencil_rows_at_the_edges_of_the_short_path(oracle, row, n):
+    """Rows of 3x3 cells at the sizes where the kernels change their path:
+    multiples of four and one past them (the steps a row is read in), more
+    pairs within reach than a lane's list holds, rows of 32 and 33 particles
+    (wavefronts that filter and that do not), last blocks of one lane and of
+    all but one, the last particles in the world's last cells; with and
+    without a tolerance, the statistics included."""
+    rng = np.random.default_rng(1000 * row + n)
+    groups = [(30, 5), (62, 30), (0, 0), (12, 31)]
+    parts = [np.stack([x + rng.uniform(0, 1.99, row), y + rng.uniform(0.0, 0.99, row)], 1) for x, y in groups]
+    rest = n - row * len(groups)
+    parts.append(np.stack([rng.uniform(0, 64, rest), rng.uniform(8, 32, rest)], 1))
+    pos = f32(np.concatenate(parts))
+    vel = f32(rng.normal(0, 0.05, (n, 2)))
+    cfg = WrachConfig(dimensions=(64, 32), cell_size=1)
+    run_stencil(oracle, cfg, pos, vel, 3, 3, every=1, label=f"rows of {row}")
+    run_stencil(oracle, cfg, pos, vel, 2, 3, tol=0.3, every=1, label=f"rows of {row}, tolerance", graph=False)

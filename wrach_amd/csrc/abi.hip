@@ -115,8 +115,10 @@ struct wrach_ctx {
     uint32_t passes = 0;
     float overlap_tol = 0.0f;
     uint32_t *scell = nullptr;   // frame-start cell of each particle (capacity entries)
-    uint32_t *swords = nullptr;  // wrach::kStencilWords words
+    uint32_t *swords = nullptr;  // wrach::kWordEntries words
     unsigned long long *ssums = nullptr;  // wrach::kStencilSumEntries entries
+    uint4 *srows = nullptr;   // each lane's rows and particle (capacity entries)
+    uint2 *srows2 = nullptr;
     uint32_t *sperm = nullptr;   // the separation kernels' lane order (capacity entries)
     uint32_t *scrowd = nullptr;  // the frame's crowded cells (crowd_cap entries)
     uint32_t crowd_cap = 0;
@@ -184,6 +186,8 @@ wrach::StencilArgs stencil_args(const wrach_ctx *c) {
     a.cell = c->scell;
     a.words = c->swords;
     a.sums = c->ssums;
+    a.rows = c->srows;
+    a.rows2 = c->srows2;
     if (c->sperm && c->scrowd) {
         a.perm = c->sperm;
         a.crowd = c->scrowd;
@@ -191,6 +195,9 @@ wrach::StencilArgs stencil_args(const wrach_ctx *c) {
     }
     return a;
 }
+
+// How a frame's stencil kernels after the first get their rows.
+uint32_t later_rows(const wrach_ctx *c) { return c->srows ? wrach::kRowsRecorded : wrach::kRowsOfCell; }
 
 // Mode S's passes: P0 = pos; pass k reads pos or pos_out (k even or odd)
 // and writes the other (pos_out is free until the collide kernel writes
@@ -206,13 +213,15 @@ int enqueue_stencil(wrach_ctx *c) {
     // overlap moves nothing, so each pass measures its own start and only
     // the end has a measure of its own.
     const bool check = c->overlap_tol > 0.0f;
-    a.first = 1;  // the frame's first kernel derives the cells
+    a.rows_from = wrach::kRowsOfPosition;  // the frame's first kernel derives the rows
+    a.record = c->srows && (check || passes > 1 || !c->quiet) ? 1 : 0;
     if (check) {
         a.pin = c->buf.pos;
         a.in_slot = 0;
         a.stat = 1;  // the overlap sums before the passes
         WRACH_HIP(wrach::launch_stencil_measure(c->fp, c->buf, a, c->stream));
-        a.first = 0;
+        a.rows_from = later_rows(c);
+        a.record = 0;
     }
     for (uint32_t k = 0; k < passes; ++k) {
         float2 *in = k % 2 == 0 ? c->buf.pos : c->buf.pos_out;
@@ -223,7 +232,8 @@ int enqueue_stencil(wrach_ctx *c) {
         a.check = check ? 1 : 0;
         a.stat = !check && k == 0 ? 1 : 0;
         WRACH_HIP(wrach::launch_stencil_move(c->fp, c->buf, a, c->stream));
-        a.first = 0;
+        a.rows_from = later_rows(c);
+        a.record = 0;
         if (check ? (k + 1 < passes || !c->quiet) : (k + 1 == passes && !c->quiet)) {
             a.pin = out;
             a.in_slot = k + 1;
@@ -297,7 +307,8 @@ int enqueue_learned(wrach_ctx *c) {
         }
     }
     a.tol = 0.0f;
-    a.first = 0;  // the cells came from the features
+    a.rows_from = wrach::kRowsOfCell;  // the cells came from the features
+    a.record = c->srows ? 1 : 0;
     for (uint32_t j = 0; j < plan.size(); ++j) {
         a.pin = plan[j].first;
         a.pout = plan[j].second;
@@ -306,6 +317,8 @@ int enqueue_learned(wrach_ctx *c) {
         a.stat = j == 0 ? 3 : 0;  // set 2: the warm start
         a.pin_alt = j == 1 ? X : nullptr;
         WRACH_HIP(wrach::launch_stencil_move(c->fp, c->buf, a, c->stream));
+        a.rows_from = later_rows(c);
+        a.record = 0;
     }
     if (cur != X) WRACH_HIP(wrach::launch_copy_pos(X, cur, c->fp.n, c->stream));
     if (!c->quiet) {
@@ -383,6 +396,8 @@ void release(wrach_ctx *c) {
     (void)hipFree(c->scell);
     (void)hipFree(c->swords);
     (void)hipFree(c->ssums);
+    (void)hipFree(c->srows);
+    (void)hipFree(c->srows2);
     (void)hipFree(c->sperm);
     (void)hipFree(c->scrowd);
     for (void *q : {(void *)c->lparams, (void *)c->lgrad, (void *)c->lm, (void *)c->lv, (void *)c->lw3,
@@ -1031,8 +1046,8 @@ int ensure_stencil(wrach_ctx *c) {
     }
     if (!c->swords) {
         uint32_t *words = nullptr;
-        WRACH_HIP(dmalloc(&words, wrach::kStencilWords));
-        WRACH_HIP(hipMemset(words, 0, wrach::kStencilWords * sizeof(uint32_t)));
+        WRACH_HIP(dmalloc(&words, wrach::kWordEntries));
+        WRACH_HIP(hipMemset(words, 0, wrach::kWordEntries * sizeof(uint32_t)));
         c->swords = words;
     }
     if (!c->ssums) {
@@ -1040,6 +1055,21 @@ int ensure_stencil(wrach_ctx *c) {
         WRACH_HIP(dmalloc(&sums, wrach::kStencilSumEntries));
         WRACH_HIP(hipMemset(sums, 0, wrach::kStencilSumEntries * sizeof(unsigned long long)));
         c->ssums = sums;
+    }
+    if (!c->srows) {
+        // Where there is no room for both the passes derive the rows again.
+        uint4 *rows = nullptr;
+        uint2 *rows2 = nullptr;
+        if (dmalloc(&rows, c->capacity ? c->capacity : 1) != hipSuccess ||
+            dmalloc(&rows2, c->capacity ? c->capacity : 1) != hipSuccess) {
+            (void)hipGetLastError();
+            (void)hipFree(rows);
+            (void)hipFree(rows2);
+            rows = nullptr;
+            rows2 = nullptr;
+        }
+        c->srows = rows;
+        c->srows2 = rows2;
     }
     if (!c->sperm) {
         uint32_t *perm = nullptr;
@@ -1103,7 +1133,7 @@ int wrach_set_solver(wrach_ctx *c, uint32_t mode, uint32_t max_passes, float ove
         const int rc = ensure_learned_frame(c);
         if (rc) return rc;
     }
-    if (c->swords) WRACH_HIP(hipMemset(c->swords, 0, wrach::kStencilWords * sizeof(uint32_t)));
+    if (c->swords) WRACH_HIP(hipMemset(c->swords, 0, wrach::kWordEntries * sizeof(uint32_t)));
     if (c->ssums) WRACH_HIP(hipMemset(c->ssums, 0, wrach::kStencilSumEntries * sizeof(unsigned long long)));
     free_graphs(c);  // captured with the previous solver
     c->solver = mode;
@@ -1116,7 +1146,7 @@ int wrach_set_solver(wrach_ctx *c, uint32_t mode, uint32_t max_passes, float ove
 
 int wrach_solver_stats(wrach_ctx *c, wrach_solver_report *out) {
     if (!c || !out) return fail(WRACH_E_INVALID, "null argument");
-    uint32_t w[wrach::kStencilWords] = {};
+    uint32_t w[wrach::kWordEntries] = {};
     std::vector<unsigned long long> sums(wrach::kStencilSumEntries, 0ull);
     if (c->swords && c->ssums) {
         WRACH_HIP(hipSetDevice(c->cfg.device));
@@ -1125,6 +1155,9 @@ int wrach_solver_stats(wrach_ctx *c, wrach_solver_report *out) {
         WRACH_HIP(hipMemcpy(sums.data(), c->ssums, sums.size() * sizeof(unsigned long long),
                             hipMemcpyDeviceToHost));
     }
+    for (uint32_t t = 1; t < wrach::kWordStripes; ++t)  // the largest over the stripes
+        for (uint32_t k = 0; k <= wrach::kMaxStencilPasses; ++k)
+            w[k] = std::max(w[k], w[t * wrach::kWordStride + k]);
     wrach_solver_report r{};
     std::memcpy(&r.max_overlap_before, &w[0], sizeof r.max_overlap_before);
     std::memcpy(&r.max_overlap_after, &w[c->passes], sizeof r.max_overlap_after);
@@ -2011,6 +2044,8 @@ int wrach_learn_sample(wrach_ctx *c, uint32_t target_passes, uint64_t *rows_tota
         // pos_out -> lbuf -> pos_out ...
         wrach::StencilArgs a = stencil_args(c);
         WRACH_HIP(wrach::launch_stencil_clear(c->fp, c->buf, a, c->buf.pos, c->stream));
+        a.rows_from = wrach::kRowsOfCell;
+        a.record = c->srows && target_passes > 1 ? 1 : 0;
         const float2 *in = c->buf.pos;
         for (uint32_t k = 0; k < target_passes; ++k) {
             float2 *out = k % 2 == 0 ? c->buf.pos_out : c->lbuf;
@@ -2018,6 +2053,8 @@ int wrach_learn_sample(wrach_ctx *c, uint32_t target_passes, uint64_t *rows_tota
             a.pout = out;
             a.in_slot = k;
             WRACH_HIP(wrach::launch_stencil_move(c->fp, c->buf, a, c->stream));
+            a.rows_from = later_rows(c);
+            a.record = 0;
             in = out;
         }
         WRACH_HIP(wrach::launch_learn_target(in, c->buf.pos, c->ttarget, (uint32_t)c->trows, n, c->stream));

@@ -233,6 +233,13 @@ hipError_t launch_upload_scatter(const UploadParams &u, const FrameBuffers &b, h
 // frame; the passes that ran are those whose start exceeded the tolerance.
 constexpr uint32_t kMaxStencilPasses = 64;
 constexpr uint32_t kStencilWords = kMaxStencilPasses + 4;
+// The words lie in kWordStripes copies on cache lines of their own: block b
+// raises the overlap words of stripe b % kWordStripes (the largest over the
+// stripes counts), the words that are no overlaps are stripe 0's.
+constexpr uint32_t kWordStripes = 16;
+constexpr uint32_t kWordStride = 96;
+static_assert(kStencilWords <= kWordStride && kWordStride % 32 == 0, "a stripe: whole 128-byte lines");
+constexpr uint32_t kWordEntries = kWordStripes * kWordStride;
 constexpr uint32_t kStencilBudget = 4096;  // most particles one lane visits in its 3x3 cells
 // Overlap sums (1 - d in 2^-24 units) and pair counts of the frame's first
 // and last measure (sets 0 and 1), and of the learned warm start's output
@@ -262,15 +269,24 @@ constexpr float kOverlapScale = 16777216.0f;  // 2^24
 // and skip more of their neighbours together.
 constexpr uint32_t kCrowdMin = 64;
 constexpr uint32_t kCrowdMax = 1024;
+constexpr uint32_t kRowsRecorded = 0, kRowsOfPosition = 1, kRowsOfCell = 2;
 struct StencilArgs {
     const float2 *pin;  // positions entering the kernel
     float2 *pout;       // a move's output
-    uint32_t *cell;     // each particle's cell at the frame's start
-    uint32_t *words;    // kStencilWords words
+    uint32_t *cell;     // each particle's cell at the frame's start (kRowsOfCell)
+    uint32_t *words;    // kWordEntries words
     unsigned long long *sums;  // kStencilSumEntries entries
     uint32_t stat;      // a measure: 0, or 1 / 2 to add its overlaps to the first / last sums
     uint32_t in_slot;   // a measure: the word it raises; a move: the word of its start
-    uint32_t first;     // the frame's first kernel: derives and writes `cell`
+    // A lane's particle and the rows of its 3x3 cells: kRowsOfPosition, the
+    // frame's first kernel derives them from its input; kRowsOfCell, from
+    // `cell`; kRowsRecorded, a kernel of the frame has recorded them (24
+    // bytes a lane, in lane order, when `record` is set; otherwise the first
+    // kernel writes `cell`).
+    uint32_t rows_from;
+    uint32_t record;
+    uint4 *rows;
+    uint2 *rows2;
     uint32_t check;     // a move: skip (copy) when the measured start is within tol
     float tol;          // a move runs while the overlap at its start exceeds this
     // A move after a learned warm start (else null): it reads pin_alt (the

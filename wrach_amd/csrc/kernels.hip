@@ -1923,22 +1923,44 @@ __global__ __launch_bounds__(256) void check_pair_arithmetic_kernel(unsigned lon
 // row cy - 1 .. cy + 1: the cells of one row are contiguous in the packed
 // layout, and [start(x0), start(x1 + 1)) covers columns x0..x1 (past the
 // row's last column, start(x1 + 1) is the next row's first cell, which
-// begins where the row ends).
+// begins where the row ends).  `own`: the start of cell (cx, cy) itself.
+// Every load is issued before the first is used (cell_start as a branch on
+// the chunk's flag made 12 dependent loads of the six offsets).
 __device__ __forceinline__ void stencil_rows(const FrameParams &p, const FrameBuffers &b,
                                              const Grid &g, int cx, int cy, uint32_t rs[3],
-                                             uint32_t re[3]) {
+                                             uint32_t re[3], uint32_t &own) {
     const int gx = (int)g.gx, gy = (int)g.gy;
-    const uint32_t base = g.base;
     const int x0 = cx > 0 ? cx - 1 : 0, x1 = cx + 1 < gx ? cx + 1 : gx - 1;
+    // Cells: [2t] the first of row t, [2t + 1] past its last, [6] the own one.
+    uint32_t c[7], at[7], live[7], pre[7];
+#pragma unroll
+    for (int t = 0; t < 3; ++t) {
+        int y = cy + t - 1;
+        y = y < 0 ? 0 : y < gy ? y : gy - 1;  // a row outside the world: loaded, not used
+        c[2 * t] = g.base + (uint32_t)(y * gx + x0);
+        c[2 * t + 1] = g.base + (uint32_t)(y * gx + x1 + 1);
+    }
+    c[6] = g.base + (uint32_t)(cy * gx + cx);
+#pragma unroll
+    for (int u = 0; u < 7; ++u) {
+        const uint32_t k = c[u] < p.ncell ? c[u] : p.ncell - 1;
+        live[u] = b.chunk_live[k >> kChunkShift];
+        pre[u] = b.chunk_prefix[k >> kChunkShift];
+        at[u] = b.idx[k + 1];
+    }
+#pragma unroll
+    for (int u = 0; u < 7; ++u) {
+        at[u] = live[u] ? at[u] : pre[u];
+        at[u] = c[u] < p.ncell && at[u] < p.n ? at[u] : p.n;
+    }
 #pragma unroll
     for (int t = 0; t < 3; ++t) {
         const int y = cy + t - 1;
-        rs[t] = re[t] = 0;
-        if (y < 0 || y >= gy) continue;  // the world's own rows only
-        rs[t] = cell_start(p, b, base + (uint32_t)(y * gx + x0));
-        re[t] = cell_start(p, b, base + (uint32_t)(y * gx + x1 + 1));
-        if (re[t] < rs[t]) re[t] = rs[t];
+        const bool in = y >= 0 && y < gy;  // the world's own rows only
+        rs[t] = in ? at[2 * t] : 0u;
+        re[t] = in && at[2 * t + 1] > at[2 * t] ? at[2 * t + 1] : rs[t];
     }
+    own = at[6];
 }
 
 // The grid of the world that holds packed particle i: the last world whose
@@ -1974,6 +1996,24 @@ __device__ __forceinline__ Grid particle_grid(const FrameParams &p, const FrameB
 // f is 0 or at least 2^-25 (normal), so F is exactly f * 2^30, and
 // dx * f * 2^30 rounds as dx * f does, scaled, unless dx * f is subnormal,
 // where both round to 0.
+constexpr float kReachSq = 1.00000011920928955078125f;  // 1 + 2^-23
+
+// ov and F of a pair within reach at squared distance sq.
+__device__ __forceinline__ void stencil_terms(float sq, float &ov, float &F) {
+    if (sq < 0x1p-96f) {  // d below 2^-48, or 0: the full sequences
+        float d = sqrtf(sq);
+        if (d == 0.0f) d = 0.0001f;
+        ov = 1.0f - d;
+        F = ((0.5f * ov) / d) * kStencilScale;
+        return;
+    }
+    const float d = sqrt_rn_above_2m96(sq);  // in [2^-48, 1]: never 0
+    ov = 1.0f - d;
+    // d is in [2^-48, 1]: overlap_force_rn's range, and the quotient is
+    // (0.5 * ov / d) * 2^30 exactly, as f is normal.
+    F = overlap_force_rn(d);
+}
+
 // `other`: j is not i (tested with the distance, so that the caller's load
 // of p_j need not wait for it).
 __device__ __forceinline__ bool stencil_reach(float dx, float dy, bool other, float &ov, float &F) {
@@ -1983,31 +2023,27 @@ __device__ __forceinline__ bool stencil_reach(float dx, float dy, bool other, fl
     // 1 and the root of the next float above it does not, so d <= 1 below.
     // Most neighbours of a crowded cell are out of reach; they skip the root
     // and the division with the same outcome.
-    if (!other | (sq > 1.00000011920928955078125f)) return false;
-    if (sq < 0x1p-96f) {  // d below 2^-48, or 0: the full sequences
-        float d = sqrtf(sq);
-        if (d == 0.0f) d = 0.0001f;
-        ov = 1.0f - d;
-        F = ((0.5f * ov) / d) * kStencilScale;
-        return true;
-    }
-    const float d = sqrt_rn_above_2m96(sq);  // in [2^-48, 1]: never 0
-    ov = 1.0f - d;
-    // d is in [2^-48, 1]: overlap_force_rn's range, and the quotient is
-    // (0.5 * ov / d) * 2^30 exactly, as f is normal.
-    F = overlap_force_rn(d);
+    if (!other | (sq > kReachSq)) return false;
+    stencil_terms(sq, ov, F);
     return true;
 }
 
-// One neighbour of particle i (`other`: not i itself) for stencil_particle.
-// ov is a multiple of 2^-24 in [0, 1], so a lane's sum of at most
-// kStencilBudget of them is a multiple of 2^-24 below 2^12: exact in a
-// double, and the sum times 2^24 an integer below 2^36.
+// The sums of a particle's pairs.  ov is a multiple of 2^-24 in [0, 1], so
+// a lane's sum of at most kStencilBudget of them is a multiple of 2^-24
+// below 2^12: exact in a double, and the sum times 2^24 an integer below
+// 2^36.
+struct PairSums {
+    double ax = 0.0, ay = 0.0;  // the terms, in 2^-30 units
+    double osum = 0.0;          // the overlaps
+    uint32_t worst = 0;         // the largest overlap's bits (overlaps lie in [0, 1])
+    uint32_t pairs = 0;
+};
+
+// One neighbour of particle i at (dx, dy) = p_i - p_j (`other`: not i
+// itself).
 template <bool MOVE, bool SUMS>
-__device__ __forceinline__ void stencil_visit(bool other, float xi, float yi, float2 q,
-                                              uint32_t &worst, uint32_t &pairs,
-                                              double &osum, double &ax, double &ay) {
-    const float dx = xi - q.x, dy = yi - q.y;
+__device__ __forceinline__ void stencil_visit(bool other, float dx, float dy, double &ax, double &ay,
+                                              double &osum, uint32_t &worst, uint32_t &pairs) {
     float ov, F;
     if (!stencil_reach(dx, dy, other, ov, F)) return;
     worst = max(worst, __float_as_uint(ov));
@@ -2019,36 +2055,130 @@ __device__ __forceinline__ void stencil_visit(bool other, float xi, float yi, fl
     }
 }
 
-// Particle i (in cell (cx, cy) at the frame's start) against the 3x3 cells
-// around it: the largest overlap, the number of overlapping pairs, with
-// MOVE the sum of its pair terms in 2^-30 units, and with SUMS the sum of
-// the overlaps in 2^-24 units.  Over kStencilBudget particles in those
-// cells: none of these (a bound on the work of one lane).
-template <bool MOVE, bool SUMS, bool HALF>
-__device__ __forceinline__ float stencil_particle(const FrameParams &p, const FrameBuffers &b,
-                                                  const float2 *pin, uint32_t i, uint32_t k,
-                                                  float xi, float yi, double &ax, double &ay,
-                                                  uint32_t &pairs, double &osum, bool &over) {
-    uint32_t rs[3], re[3];
-    const Grid g = grid_of(p, k);
-    uint32_t cx, cy;
-    cell_coords(g, k, cx, cy);
-    stencil_rows(p, b, g, (int)cx, (int)cy, rs, re);
-    const uint64_t total = (uint64_t)(re[0] - rs[0]) + (re[1] - rs[1]) + (re[2] - rs[2]);
-    if (total > kStencilBudget) {
-        over = true;
-        return 0.0f;
+// The same for a neighbour known to be within reach.
+template <bool MOVE, bool SUMS>
+__device__ __forceinline__ void stencil_hit(float dx, float dy, PairSums &s) {
+    float sq = dx * dx;
+    sq = sq + dy * dy;
+    float ov, F;
+    stencil_terms(sq, ov, F);
+    s.worst = max(s.worst, __float_as_uint(ov));
+    s.pairs += 1;
+    if (SUMS) s.osum += (double)ov;
+    if (MOVE) {
+        s.ax += (double)rintf(dx * F);
+        s.ay += (double)rintf(dy * F);
     }
-    uint32_t worst = 0;  // the largest overlap's bits (overlaps lie in [0, 1])
-    // HALF: each pair once.  A particle takes its pairs with the later
-    // particles of its own cell, with the cell to its right and with the
-    // three cells above; every other pair of its 3x3 cells is one of these
-    // seen from the other particle.
-    if (HALF) rs[1] = min(max(rs[1], cell_start(p, b, k)), re[1]);
+}
+
+// The 3x3 cells of a particle as the stencil kernels keep them: each row's
+// first particle and length, the lengths 0 over the budget.
+struct StencilRows {
+    uint32_t rs[3], len[3];
+    uint32_t half;  // rs[1] + half: the particle's own cell's start
+};
+
+// The rows of a particle in cell k.  More than kStencilBudget particles in
+// them: none, and `over` (a bound on the work of one lane).
+__device__ __forceinline__ StencilRows stencil_rows_of(const FrameParams &p, const FrameBuffers &b,
+                                                       uint32_t k, bool &over) {
+    StencilRows r;
+    const Grid g = grid_of(p, k);
+    uint32_t cx, cy, own, re[3];
+    cell_coords(g, k, cx, cy);
+    stencil_rows(p, b, g, (int)cx, (int)cy, r.rs, re, own);
+    const uint64_t total = (uint64_t)(re[0] - r.rs[0]) + (re[1] - r.rs[1]) + (re[2] - r.rs[2]);
+    over = total > kStencilBudget;
+#pragma unroll
+    for (int t = 0; t < 3; ++t) r.len[t] = over ? 0u : re[t] - r.rs[t];
+    r.half = over ? 0u : min(max(r.rs[1], own), re[1]) - r.rs[1];
+    return r;
+}
+
+// A wavefront none of whose rows holds more than kShortRow particles filters
+// first: four neighbours of each of the three rows at a time, their loads in
+// flight together, those within reach appended to the lane's list in LDS;
+// then every lane works off its list.  A loose world's lane has two or three
+// neighbours a row and about half of them within reach, and the pair
+// arithmetic (some 25 instructions) would otherwise run for every neighbour
+// that is within reach of any of the 64 lanes, the rows one after another to
+// the longest of each.  A pass over the 1M lattice is bound by these vector
+// instructions: 1,065 a wavefront and 35 us with a loop per row, 690 and 21 us
+// with the filter and recorded rows (the measure: 580 and 27 us, 373 and
+// 14 us).  Fuller wavefronts take each row by itself: lanes of one cell then
+// read the same neighbour together, and neighbours out of every lane's reach
+// are skipped together (the collapsed lattice, 820 us either way; a list of
+// them would only add to the pairs within reach, nearly all of the own
+// cell's).  kShortRow lies where the rows of a loose world end and those of a
+// pile (hundreds) begin.
+constexpr uint32_t kShortRow = 32;
+constexpr int kHitList = 9;  // entries a lane: 18 KiB a block, 8 blocks on a CU (24 KiB, 6 blocks: 26 us)
+
+template <bool MOVE, bool SUMS>
+__device__ __forceinline__ void stencil_hits(const float2 *list, uint32_t &hits, PairSums &s) {
+    for (uint32_t h = 0; __ballot(h < hits) != 0; ++h) {
+        if (h < hits) {
+            const float2 d = list[h * 256];
+            stencil_hit<MOVE, SUMS>(d.x, d.y, s);
+        }
+    }
+    hits = 0;
+}
+
+// The short rows of a wavefront: filter, then the list.
+template <bool MOVE, bool SUMS, bool HALF>
+__device__ __forceinline__ void stencil_short(const float2 *pin, uint32_t i, float xi, float yi,
+                                              StencilRows r, float2 *list, PairSums &s) {
+    if (HALF) {
+        const uint32_t from = min(max(r.rs[1], i + 1), r.rs[1] + r.len[1]);
+        r.len[1] -= from - r.rs[1];
+        r.rs[1] = from;
+    }
+    const uint32_t longest = max(max(r.len[0], r.len[1]), r.len[2]);
+    uint32_t hits = 0;
+    for (uint32_t o = 0; __ballot(o < longest) != 0; o += 4) {
+        // Past a row's end these are other particles, or up to three
+        // entries past the last one (dmalloc's slack).
+        float2 q[3][4];
+#pragma unroll
+        for (int t = HALF ? 1 : 0; t < 3; ++t) {
+            if (o < r.len[t]) {
+                const float2 *qp = pin + (r.rs[t] + o);
+#pragma unroll
+                for (int v = 0; v < 4; ++v) q[t][v] = qp[v];
+            }
+        }
+#pragma unroll
+        for (int t = HALF ? 1 : 0; t < 3; ++t) {
+            if (__ballot(o < r.len[t]) == 0) continue;
+            if (__ballot(hits > (uint32_t)kHitList - 4) != 0) stencil_hits<MOVE, SUMS>(list, hits, s);
+#pragma unroll
+            for (int v = 0; v < 4; ++v) {
+                const float dx = xi - q[t][v].x, dy = yi - q[t][v].y;
+                float sq = dx * dx;
+                sq = sq + dy * dy;
+                bool in = o + v < r.len[t];
+                if (t == 1 && !HALF) in = in & (r.rs[1] + o + v != i);
+                if (in & !(sq > kReachSq)) {
+                    list[hits * 256] = make_float2(dx, dy);
+                    ++hits;
+                }
+            }
+        }
+    }
+    stencil_hits<MOVE, SUMS>(list, hits, s);
+}
+
+// Any rows, one row after another, four neighbours a step, all loaded before
+// the first is used.
+template <bool MOVE, bool SUMS, bool HALF>
+__device__ __forceinline__ void stencil_long(const float2 *pin, uint32_t i, float xi, float yi,
+                                             const uint32_t (&rs)[3], const uint32_t (&re)[3],
+                                             double &ax, double &ay, double &osum, uint32_t &worst,
+                                             uint32_t &pairs) {
     for (int t = HALF ? 1 : 0; t < 3; ++t) {
         uint32_t j = rs[t];
         const uint32_t e = re[t];
-        // Four neighbours a step, all loaded before the first is used.
         for (; j + 4 <= e; j += 4) {
             // One address, four loads at constant offsets from it.
             const float2 *qp = pin + j;
@@ -2057,13 +2187,45 @@ __device__ __forceinline__ float stencil_particle(const FrameParams &p, const Fr
             for (int u = 0; u < 4; ++u) q[u] = qp[u];
 #pragma unroll
             for (int u = 0; u < 4; ++u)
-                stencil_visit<MOVE, SUMS>(HALF && t == 1 ? j + u > i : j + u != i, xi, yi, q[u], worst, pairs,
-                                          osum, ax, ay);
+                stencil_visit<MOVE, SUMS>(HALF && t == 1 ? j + u > i : j + u != i, xi - q[u].x, yi - q[u].y, ax, ay,
+                                          osum, worst, pairs);
         }
-        for (; j < e; ++j)
-            stencil_visit<MOVE, SUMS>(HALF && t == 1 ? j > i : j != i, xi, yi, pin[j], worst, pairs, osum, ax, ay);
+        for (; j < e; ++j) {
+            const float2 q = pin[j];
+            stencil_visit<MOVE, SUMS>(HALF && t == 1 ? j > i : j != i, xi - q.x, yi - q.y, ax, ay, osum, worst, pairs);
+        }
     }
-    return __uint_as_float(worst);
+}
+
+// Particle i at (xi, yi) against the particles of its rows: the number of
+// overlapping pairs and the largest overlap, with MOVE the sum of its pair
+// terms, and with SUMS the sum of the overlaps.  (A lane without a particle
+// has empty rows.)  HALF: each pair once -- the later particles of its own
+// cell, the cell to its right and the three cells above; every other pair of
+// its 3x3 cells is one of these seen from the other particle.
+template <bool MOVE, bool SUMS, bool HALF>
+__device__ __forceinline__ PairSums stencil_particle(const float2 *pin, uint32_t i, float xi, float yi,
+                                                     StencilRows r, float2 *list) {
+    if (HALF) {
+        r.len[0] = 0;
+        r.rs[1] += r.half;
+        r.len[1] -= r.half;
+    }
+    PairSums s;
+    if (__ballot(max(max(r.len[0], r.len[1]), r.len[2]) > kShortRow) == 0) {
+        stencil_short<MOVE, SUMS, HALF>(pin, i, xi, yi, r, list, s);
+        return s;
+    }
+    double ax = 0.0, ay = 0.0, osum = 0.0;
+    uint32_t worst = 0, pairs = 0;
+    const uint32_t re[3] = {r.rs[0] + r.len[0], r.rs[1] + r.len[1], r.rs[2] + r.len[2]};
+    stencil_long<MOVE, SUMS, HALF>(pin, i, xi, yi, r.rs, re, ax, ay, osum, worst, pairs);
+    s.ax = ax;
+    s.ay = ay;
+    s.osum = osum;
+    s.worst = worst;
+    s.pairs = pairs;
+    return s;
 }
 
 __device__ __forceinline__ float wave_max(float v) {
@@ -2072,50 +2234,115 @@ __device__ __forceinline__ float wave_max(float v) {
     return v;
 }
 
-// Raises *w to the block's largest v -- one atomic per block, and none when
-// the word already holds as much (every block hitting one word serialises)
-// -- and, with sums, adds the block's overlap sum and pair count to its
+// Reductions of a wavefront into lane 63 by DPP moves (one instruction a
+// step; a shuffle takes three): lanes without a source add or compare 0.
+template <int CTRL, int ROWS>
+__device__ __forceinline__ uint32_t dpp0(uint32_t v) {
+    return (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, CTRL, ROWS, 0xf, false);
+}
+
+__device__ __forceinline__ uint32_t wave63_max(uint32_t v) {
+    v = max(v, dpp0<0x111, 0xf>(v));  // row_shr:1, :2, :4, :8
+    v = max(v, dpp0<0x112, 0xf>(v));
+    v = max(v, dpp0<0x114, 0xf>(v));
+    v = max(v, dpp0<0x118, 0xf>(v));
+    v = max(v, dpp0<0x142, 0xa>(v));  // row_bcast:15 into rows 1 and 3
+    return max(v, dpp0<0x143, 0xc>(v));  // row_bcast:31 into rows 2 and 3
+}
+
+__device__ __forceinline__ uint32_t wave63_sum(uint32_t v) {
+    v += dpp0<0x111, 0xf>(v);
+    v += dpp0<0x112, 0xf>(v);
+    v += dpp0<0x114, 0xf>(v);
+    v += dpp0<0x118, 0xf>(v);
+    v += dpp0<0x142, 0xa>(v);
+    return v + dpp0<0x143, 0xc>(v);
+}
+
+// Raises word `slot` of the block's stripe to the block's largest overlap
+// (its bits) -- one atomic per block that nothing waits for; with one word
+// for every block they serialised, and reading it first to skip them kept
+// each block resident for a memory round trip -- and, with sums, adds
+// `sides` times the block's
+// overlap sum (a lane's below 2^36 units of 2^-24) and pair count to its
 // slot (blockIdx % kStencilSumSlots) of them.
-__device__ __forceinline__ void block_report(uint32_t *w, float v, unsigned long long *sums,
-                                             unsigned long long osum, unsigned long long ocnt) {
-    __shared__ float s_max[4];
-    __shared__ unsigned long long s_sum[4], s_cnt[4];
-    v = wave_max(v);
-#pragma unroll
-    for (int o = 32; o > 0; o >>= 1) {
-        osum += __shfl_xor(osum, o, 64);
-        ocnt += __shfl_xor(ocnt, o, 64);
+__device__ __forceinline__ void block_report(uint32_t *words, uint32_t slot, const PairSums &s, unsigned long long *sums,
+                                             unsigned long long sides) {
+    __shared__ uint32_t s_max[4], s_cnt[4];
+    __shared__ unsigned long long s_sum[4];
+    const uint32_t wave = threadIdx.x >> 6, lane = lane_id();
+    const uint32_t worst = wave63_max(s.worst);
+    uint32_t cnt = 0, lo = 0, hi = 0;
+    if (sums) {  // the whole grid alike
+        const unsigned long long o = (unsigned long long)(s.osum * (double)kOverlapScale);
+        cnt = wave63_sum(s.pairs);
+        lo = wave63_sum((uint32_t)o & 0xffffffu);
+        hi = wave63_sum((uint32_t)(o >> 24));
     }
-    if (lane_id() == 0) {
-        s_max[threadIdx.x >> 6] = v;
-        s_sum[threadIdx.x >> 6] = osum;
-        s_cnt[threadIdx.x >> 6] = ocnt;
+    if (lane == 63) {
+        s_max[wave] = worst;
+        s_cnt[wave] = cnt;
+        s_sum[wave] = ((unsigned long long)hi << 24) + lo;
     }
     __syncthreads();
     if (threadIdx.x == 0) {
-        const float m = fmaxf(fmaxf(s_max[0], s_max[1]), fmaxf(s_max[2], s_max[3]));
-        if (m > 0.0f && __float_as_uint(m) > __hip_atomic_load(w, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT))
-            atomicMax(w, __float_as_uint(m));
-        const unsigned long long cnt = s_cnt[0] + s_cnt[1] + s_cnt[2] + s_cnt[3];
-        if (sums && cnt) {
-            unsigned long long *slot = sums + (blockIdx.x % kStencilSumSlots) * kStencilSumStride;
-            atomicAdd(slot, s_sum[0] + s_sum[1] + s_sum[2] + s_sum[3]);
-            atomicAdd(slot + 1, cnt);
+        const uint32_t m = max(max(s_max[0], s_max[1]), max(s_max[2], s_max[3]));
+        if (m) atomicMax(&words[(blockIdx.x % kWordStripes) * kWordStride + slot], m);
+        const unsigned long long n = (unsigned long long)s_cnt[0] + s_cnt[1] + s_cnt[2] + s_cnt[3];
+        if (sums && n) {
+            unsigned long long *to = sums + (blockIdx.x % kStencilSumSlots) * kStencilSumStride;
+            atomicAdd(to, sides * (s_sum[0] + s_sum[1] + s_sum[2] + s_sum[3]));
+            atomicAdd(to + 1, sides * n);
         }
     }
 }
 
-// The largest overlap at positions a.pin, raised into a.words[a.in_slot]
-// (non-negative floats order as their bits).  a.first: the frame-start
-// positions, whose cells every pass of the frame uses.
-// Particle i's cell at the frame's start: derived from its position by the
-// frame's first stencil kernel (a.first), which records it; read after.
-__device__ __forceinline__ uint32_t stencil_cell(const FrameParams &p, const FrameBuffers &b,
-                                                 const StencilArgs &a, uint32_t i, float2 q) {
-    if (!a.first) return a.cell[i];
-    const uint32_t k = cell_key(p, particle_grid(p, b, i), q.x, q.y);
-    a.cell[i] = k;
-    return k;
+// The particle of this lane and its rows.  The frame's first stencil kernel
+// takes the particle from the lane order (StencilArgs::perm) and its cell
+// from its position or from a.cell, and records both for the kernels that
+// follow: a particle's 3x3 cells are the frame start's in every pass, and
+// deriving the rows (a division, 21 loads and their selection) was a fifth of
+// a loose pass's instructions.  Without room for the record (a.record 0) the
+// first kernel leaves the cell.  A lane without a particle gets i >= p.n, or
+// empty rows.
+__device__ __forceinline__ StencilRows stencil_lane(const FrameParams &p, const FrameBuffers &b,
+                                                    const StencilArgs &a, uint32_t &i, float2 &q) {
+    StencilRows r;
+#pragma unroll
+    for (int t = 0; t < 3; ++t) r.rs[t] = r.len[t] = 0;
+    r.half = 0;
+    q = make_float2(0.0f, 0.0f);
+    const uint32_t t = blockIdx.x * 256 + threadIdx.x;
+    i = t;
+    if (t >= p.n) return r;
+    if (a.rows_from == kRowsRecorded) {
+        const uint4 v = a.rows[t];
+        const uint2 w = a.rows2[t];
+        i = w.y;
+        q = a.pin[i];
+        r.rs[0] = v.x;
+        r.rs[1] = v.y;
+        r.rs[2] = v.z;
+        r.len[0] = v.w & 0xffffu;
+        r.half = v.w >> 16;
+        r.len[1] = w.x & 0xffffu;
+        r.len[2] = w.x >> 16;
+        return r;
+    }
+    i = a.perm ? a.perm[t] : t;
+    q = a.pin[i];
+    const uint32_t k = a.rows_from == kRowsOfCell ? a.cell[i] : cell_key(p, particle_grid(p, b, i), q.x, q.y);
+    if (k < p.ncell) {
+        bool over;
+        r = stencil_rows_of(p, b, k, over);
+        if (over) atomicOr(&a.words[kOverBudgetWord], 1u);
+    }
+    if (a.rows_from == kRowsOfPosition && !a.record) a.cell[i] = k;
+    if (a.record) {
+        a.rows[t] = make_uint4(r.rs[0], r.rs[1], r.rs[2], r.len[0] | (r.half << 16));
+        a.rows2[t] = make_uint2(r.len[1] | (r.len[2] << 16), i);
+    }
+    return r;
 }
 
 __device__ __forceinline__ unsigned long long *stencil_sums(const StencilArgs &a) {
@@ -2146,36 +2373,28 @@ __device__ __forceinline__ bool warm_rejected(const StencilArgs &a) {
     return s_rej != 0;
 }
 
-// The particle of lane t (see StencilArgs::perm).
-__device__ __forceinline__ uint32_t lane_particle(const FrameParams &p, const StencilArgs &a, uint32_t t) {
-    return a.perm && t < p.n ? a.perm[t] : t;
+// The largest overlap at positions a.pin, raised into a.words[a.in_slot]
+// (non-negative floats order as their bits).
+__global__ __launch_bounds__(256, 8) void stencil_measure_kernel(FrameParams p, FrameBuffers b,
+                                                              StencilArgs a) {
+    __shared__ float2 s_list[kHitList * 256];
+    uint32_t i;
+    float2 q;
+    const StencilRows r = stencil_lane(p, b, a, i, q);
+    const bool half = a.half && a.words[kOverBudgetWord] == 0;  // the whole grid alike
+    float2 *list = s_list + threadIdx.x;
+    const PairSums s = half ? (a.stat ? stencil_particle<false, true, true>(a.pin, i, q.x, q.y, r, list)
+                                      : stencil_particle<false, false, true>(a.pin, i, q.x, q.y, r, list))
+                            : (a.stat ? stencil_particle<false, true, false>(a.pin, i, q.x, q.y, r, list)
+                                      : stencil_particle<false, false, false>(a.pin, i, q.x, q.y, r, list));
+    block_report(a.words, a.in_slot, s, stencil_sums(a), half ? 2ull : 1ull);
 }
 
-__global__ __launch_bounds__(256) void stencil_measure_kernel(FrameParams p, FrameBuffers b,
-                                                              StencilArgs a) {
-    const uint32_t i = lane_particle(p, a, blockIdx.x * 256 + threadIdx.x);
-    float worst = 0.0f;
-    uint32_t pairs = 0;
-    double osum = 0.0;  // overlaps: multiples of 2^-24, at most kStencilBudget of them
-    bool over = false;
-    const bool half = a.half && a.words[kOverBudgetWord] == 0;  // the whole grid alike
-    if (i < p.n) {
-        const float2 q = a.pin[i];
-        const uint32_t k = stencil_cell(p, b, a, i, q);
-        double ax = 0.0, ay = 0.0;
-        if (k < p.ncell) {
-            if (half)
-                worst = a.stat ? stencil_particle<false, true, true>(p, b, a.pin, i, k, q.x, q.y, ax, ay, pairs, osum, over)
-                               : stencil_particle<false, false, true>(p, b, a.pin, i, k, q.x, q.y, ax, ay, pairs, osum, over);
-            else
-                worst = a.stat ? stencil_particle<false, true, false>(p, b, a.pin, i, k, q.x, q.y, ax, ay, pairs, osum, over)
-                               : stencil_particle<false, false, false>(p, b, a.pin, i, k, q.x, q.y, ax, ay, pairs, osum, over);
-        }
-    }
-    if (over) atomicOr(&a.words[kOverBudgetWord], 1u);
-    const unsigned long long sides = half ? 2ull : 1ull;  // each pair seen once or from both sides
-    block_report(&a.words[a.in_slot], worst, stencil_sums(a),
-                 sides * (unsigned long long)(osum * (double)kOverlapScale), sides * pairs);
+// Whether the largest overlap recorded in word `slot` exceeds tol (overlaps
+// lie in [0, 1]: the stripes' bits order as the floats).
+__device__ __forceinline__ bool overlap_above(const uint32_t *words, uint32_t slot, float tol) {
+    const uint32_t v = words[(lane_id() % kWordStripes) * kWordStride + slot];
+    return __ballot(__uint_as_float(v) > tol) != 0;
 }
 
 // One pass: a.pin -> a.pout.  With a.check it runs only while the
@@ -2184,48 +2403,40 @@ __global__ __launch_bounds__(256) void stencil_measure_kernel(FrameParams p, Fra
 // way it raises a.words[a.in_slot] to the largest overlap of its input, so
 // that a frame without a check (tolerance 0, where a pass over no overlap
 // moves nothing) needs no measure between passes.
-__global__ __launch_bounds__(256) void stencil_move_kernel(FrameParams p, FrameBuffers b,
+__global__ __launch_bounds__(256, 7) void stencil_move_kernel(FrameParams p, FrameBuffers b,
                                                            StencilArgs a) {
-    const uint32_t i = lane_particle(p, a, blockIdx.x * 256 + threadIdx.x);
-    if (a.check && !(__uint_as_float(a.words[a.in_slot]) > a.tol)) {
-        if (i < p.n) a.pout[i] = a.pin[i];
+    __shared__ float2 s_list[kHitList * 256];
+    if (a.check && !overlap_above(a.words, a.in_slot, a.tol)) {
+        const uint32_t t = blockIdx.x * 256 + threadIdx.x;
+        if (t < p.n) a.pout[t] = a.pin[t];
         return;  // the whole grid: no barrier follows
     }
-    float worst = 0.0f;
-    double ax = 0.0, ay = 0.0;  // integers: the sums of the terms in 2^-30 units
-    uint32_t pairs = 0;
-    double osum = 0.0;  // overlaps: multiples of 2^-24, at most kStencilBudget of them
-    bool over = false;
-    float2 q = make_float2(0.0f, 0.0f);
     if (a.pin_alt) {
         const bool rej = warm_rejected(a);
         if (blockIdx.x == 0 && threadIdx.x == 0) a.words[kFallbackWord] = rej ? 1u : 0u;
         if (rej) a.pin = a.pin_alt;  // a copy of the arguments: the whole grid decides alike
     }
-    if (i < p.n) {
-        q = a.pin[i];
-        const uint32_t k = stencil_cell(p, b, a, i, q);
-        if (k < p.ncell)
-            worst = a.stat ? stencil_particle<true, true, false>(p, b, a.pin, i, k, q.x, q.y, ax, ay, pairs, osum, over)
-                           : stencil_particle<true, false, false>(p, b, a.pin, i, k, q.x, q.y, ax, ay, pairs, osum, over);
-    }
-    if (over) atomicOr(&a.words[kOverBudgetWord], 1u);
-    block_report(&a.words[a.in_slot], worst, stencil_sums(a),
-                 (unsigned long long)(osum * (double)kOverlapScale), pairs);
+    uint32_t i;
+    float2 q;
+    const StencilRows r = stencil_lane(p, b, a, i, q);
+    float2 *list = s_list + threadIdx.x;
+    const PairSums s = a.stat ? stencil_particle<true, true, false>(a.pin, i, q.x, q.y, r, list)
+                              : stencil_particle<true, false, false>(a.pin, i, q.x, q.y, r, list);
+    block_report(a.words, a.in_slot, s, stencil_sums(a), 1ull);
     if (i >= p.n) return;
     // The mean of the pair corrections (constraint averaging): a particle
     // moves at most 0.5 per pass.
-    float dx = (float)ax * kStencilUnit;  // the integer rounded once to f32
-    float dy = (float)ay * kStencilUnit;
-    if (pairs > 1) {
-        dx = dx / (float)pairs;
-        dy = dy / (float)pairs;
+    float dx = (float)s.ax * kStencilUnit;  // the integer rounded once to f32
+    float dy = (float)s.ay * kStencilUnit;
+    if (s.pairs > 1) {
+        dx = dx / (float)s.pairs;
+        dy = dy / (float)s.pairs;
     }
     a.pout[i] = make_float2(q.x + dx, q.y + dy);
 }
 
 __global__ __launch_bounds__(256) void stencil_clear_kernel(uint32_t *w, unsigned long long *sums) {
-    for (uint32_t i = threadIdx.x; i < kStencilWords; i += 256) w[i] = 0;
+    for (uint32_t i = threadIdx.x; i < kWordEntries; i += 256) w[i] = 0;
     for (uint32_t i = threadIdx.x; i < kStencilSumSets * kStencilSumSlots; i += 256) {
         sums[i * kStencilSumStride] = 0;
         sums[i * kStencilSumStride + 1] = 0;
