@@ -132,6 +132,14 @@ def test_gradient_matches_the_oracle(n):
     assert not bad, bad
 
 
+@pytest.mark.parametrize("n", [128, 704, 2112, 5376, 16448])
+def test_gradient_over_batches_of_uneven_chunks(n):
+    """The weight gradients' chunks of 32, 64 and 96 rows, a shorter last one,
+    chunk counts that are no multiple of 8, and column sums over a last
+    round of fewer than 256 rows: the tolerances of the batch test above."""
+    test_gradient_matches_the_oracle(n)
+
+
 def test_adam_is_bit_exact():
     params = _params(6)
     r = np.random.Generator(np.random.PCG64(7))

@@ -141,7 +141,7 @@ struct wrach_ctx {
     size_t tsel_cap = 0;
     uint32_t tbsz = 0;
     uint16_t *txt = nullptr, *ta1t = nullptr, *tdz1t = nullptr, *tdz2t = nullptr;
-    float *ta2t = nullptr, *tdyt = nullptr, *tsq = nullptr, *tpart1 = nullptr, *tpart2 = nullptr;
+    float *ta2t = nullptr, *tdyt = nullptr, *tsq = nullptr, *tpart = nullptr, *tcols = nullptr;
     float *tloss = nullptr;  // one loss per step of a training call
     size_t tloss_cap = 0;
 };
@@ -404,7 +404,7 @@ void release(wrach_ctx *c) {
                     (void *)c->lfrag, (void *)c->lfeat, (void *)c->lbuf, (void *)c->tfeat,
                     (void *)c->ttarget, (void *)c->tsel, (void *)c->txt, (void *)c->ta1t,
                     (void *)c->tdz1t, (void *)c->tdz2t, (void *)c->ta2t, (void *)c->tdyt, (void *)c->tsq,
-                    (void *)c->tpart1, (void *)c->tpart2, (void *)c->tloss})
+                    (void *)c->tpart, (void *)c->tcols, (void *)c->tloss})
         (void)hipFree(q);
     if (c->stream) (void)hipStreamDestroy(c->stream);
     delete c;
@@ -1766,13 +1766,13 @@ int ensure_learn(wrach_ctx *c) {
 int ensure_batch(wrach_ctx *c, uint32_t bsz) {
     if (c->tbsz >= bsz) return WRACH_OK;
     for (void *q : {(void *)c->txt, (void *)c->ta1t, (void *)c->tdz1t, (void *)c->tdz2t, (void *)c->ta2t,
-                    (void *)c->tdyt, (void *)c->tsq, (void *)c->tpart1, (void *)c->tpart2})
+                    (void *)c->tdyt, (void *)c->tsq, (void *)c->tpart, (void *)c->tcols})
         (void)hipFree(q);
     c->txt = c->ta1t = c->tdz1t = c->tdz2t = nullptr;
-    c->ta2t = c->tdyt = c->tsq = c->tpart1 = c->tpart2 = nullptr;
+    c->ta2t = c->tdyt = c->tsq = c->tpart = c->tcols = nullptr;
     c->tbsz = 0;
     const size_t b = bsz;
-    const size_t chunks = b / 32;  // the most k chunks a GEMM uses
+    const size_t chunks = b / 32;  // the most k chunks a batch uses
     WRACH_HIP(dmalloc(&c->txt, (size_t)wrach::kFeat * b));
     WRACH_HIP(dmalloc(&c->ta1t, (size_t)wrach::kHid * b));
     WRACH_HIP(dmalloc(&c->tdz1t, (size_t)wrach::kHid * b));
@@ -1780,29 +1780,30 @@ int ensure_batch(wrach_ctx *c, uint32_t bsz) {
     WRACH_HIP(dmalloc(&c->ta2t, (size_t)wrach::kHid * b));
     WRACH_HIP(dmalloc(&c->tdyt, 2 * b));
     WRACH_HIP(dmalloc(&c->tsq, b / 16));
-    WRACH_HIP(dmalloc(&c->tpart1, (size_t)wrach::kFeat * wrach::kHid * std::min<size_t>(chunks, 64)));
-    WRACH_HIP(dmalloc(&c->tpart2, (size_t)wrach::kHid * wrach::kHid * std::min<size_t>(chunks, 64)));
+    WRACH_HIP(dmalloc(&c->tpart, (size_t)wrach::kWeights * std::min<size_t>(chunks, 64)));
+    WRACH_HIP(dmalloc(&c->tcols, wrach::kCols));
     c->tbsz = bsz;
     return WRACH_OK;
 }
 
-// k chunk of the weight GEMMs over a batch of bsz rows (a multiple of 64):
+// k chunk of the weight gradients over a batch of bsz rows (a multiple of 64):
 // at most 64 chunks, each a multiple of 32, the last one possibly shorter.
 uint32_t gemm_chunk(uint32_t bsz) {
     const uint32_t chunks = std::min<uint32_t>(64u, bsz / 32u);
     return (bsz / chunks + 31u) / 32u * 32u;
 }
 
-// One training step on the batch rows sel[0..bsz) of (feat, target):
-// gradient into lgrad, the loss into *loss_dev (if not null).
+// The gradient's parts over the batch rows sel[0..bsz) of (feat, target).
 int enqueue_gradient(wrach_ctx *c, const uint16_t *feat, const float2 *target, const uint32_t *sel,
-                     uint32_t bsz, float *loss_dev) {
+                     uint32_t bsz) {
     wrach::TrainArgs t{};
     t.feat = feat;
     t.target = target;
     t.sel = sel;
     t.bsz = bsz;
     t.inv_bsz = 1.0f / (float)bsz;
+    t.kc = gemm_chunk(bsz);
+    t.chunks = (bsz + t.kc - 1) / t.kc;
     t.xt = c->txt;
     t.a1t = c->ta1t;
     t.dz1t = c->tdz1t;
@@ -1810,31 +1811,39 @@ int enqueue_gradient(wrach_ctx *c, const uint16_t *feat, const float2 *target, c
     t.a2t = c->ta2t;
     t.dyt = c->tdyt;
     t.sqerr = c->tsq;
-    WRACH_HIP(wrach::launch_learn_rows(mlp_weights(c), t, c->stream));
-    const uint32_t kc = gemm_chunk(bsz), chunks = (bsz + kc - 1) / kc;
-    WRACH_HIP(wrach::launch_learn_gemm_nt(c->txt, c->tdz1t, wrach::kFeat, wrach::kHid, bsz, kc, chunks,
-                                          c->tpart1, c->stream));
-    WRACH_HIP(wrach::launch_learn_gemm_nt(c->ta1t, c->tdz2t, wrach::kHid, wrach::kHid, bsz, kc, chunks,
-                                          c->tpart2, c->stream));
-    WRACH_HIP(wrach::launch_learn_reduce(t, c->tpart1, c->tpart2, chunks, c->lgrad, loss_dev, c->stream));
+    t.part = c->tpart;
+    t.cols = c->tcols;
+    WRACH_HIP(wrach::launch_learn_grad(mlp_weights(c), t, c->stream));
     return WRACH_OK;
 }
 
-int enqueue_adam(wrach_ctx *c, float lr) {
+// Their sum and loss (if loss_dev is not null).
+wrach::UpdateArgs gradient_sum(const wrach_ctx *c, uint32_t bsz, float *loss_dev) {
+    wrach::UpdateArgs u{};
+    u.part = c->tpart;
+    u.cols = c->tcols;
+    u.chunks = (bsz + gemm_chunk(bsz) - 1) / gemm_chunk(bsz);
+    u.loss = loss_dev;
+    u.loss_scale = 0.5f * (1.0f / (float)bsz);
+    return u;
+}
+
+// The next Adam step with the gradient that u sums.
+int enqueue_adam(wrach_ctx *c, wrach::UpdateArgs u, float lr) {
     c->adam_t += 1;
-    wrach::AdamArgs a{};
-    a.params = c->lparams;
-    a.m = c->lm;
-    a.v = c->lv;
-    a.grad = c->lgrad;
-    a.lr = lr;
-    a.beta1 = kAdamBeta1;
-    a.beta2 = kAdamBeta2;
-    a.eps = kAdamEps;
-    a.c1 = (float)(1.0 / (1.0 - std::pow((double)kAdamBeta1, (double)c->adam_t)));
-    a.c2 = (float)(1.0 / (1.0 - std::pow((double)kAdamBeta2, (double)c->adam_t)));
-    WRACH_HIP(wrach::launch_learn_adam(a, c->stream));
-    WRACH_HIP(wrach::launch_learn_pack(c->lparams, c->lfrag, c->lw3, c->stream));
+    u.grad = nullptr;
+    u.params = c->lparams;
+    u.m = c->lm;
+    u.v = c->lv;
+    u.frag = c->lfrag;
+    u.w3 = c->lw3;
+    u.lr = lr;
+    u.beta1 = kAdamBeta1;
+    u.beta2 = kAdamBeta2;
+    u.eps = kAdamEps;
+    u.c1 = (float)(1.0 / (1.0 - std::pow((double)kAdamBeta1, (double)c->adam_t)));
+    u.c2 = (float)(1.0 / (1.0 - std::pow((double)kAdamBeta2, (double)c->adam_t)));
+    WRACH_HIP(wrach::launch_learn_update(u, c->stream));
     return WRACH_OK;
 }
 
@@ -1972,8 +1981,11 @@ int wrach_learn_gradient(wrach_ctx *c, const uint16_t *rows, const float *target
     WRACH_HIP(hipMemcpyAsync(t.p, targets, (size_t)n * 2 * sizeof(float), hipMemcpyHostToDevice, c->stream));
     WRACH_HIP(hipMemcpyAsync(sel.p, iota.data(), (size_t)n * sizeof(uint32_t), hipMemcpyHostToDevice, c->stream));
     {
-        const int rc = enqueue_gradient(c, f.p, t.p, sel.p, n, l.p);
+        const int rc = enqueue_gradient(c, f.p, t.p, sel.p, n);
         if (rc) return rc;
+        wrach::UpdateArgs u = gradient_sum(c, n, l.p);
+        u.grad = c->lgrad;
+        WRACH_HIP(wrach::launch_learn_update(u, c->stream));
     }
     WRACH_HIP(hipMemcpyAsync(grad, c->lgrad, wrach::kParams * sizeof(float), hipMemcpyDeviceToHost, c->stream));
     float hl = 0.0f;
@@ -1990,7 +2002,9 @@ int wrach_learn_adam(wrach_ctx *c, const float *grad, float lr) {
     WRACH_HIP(hipSetDevice(c->cfg.device));
     WRACH_HIP(hipMemcpyAsync(c->lgrad, grad, wrach::kParams * sizeof(float), hipMemcpyHostToDevice, c->stream));
     {
-        const int rc = enqueue_adam(c, lr);
+        wrach::UpdateArgs u{};
+        u.given = c->lgrad;
+        const int rc = enqueue_adam(c, u, lr);
         if (rc) return rc;
     }
     WRACH_SETTLE(c);
@@ -2103,8 +2117,8 @@ int wrach_learn_train(wrach_ctx *c, const uint32_t *order, size_t n_order, uint3
     }
     WRACH_HIP(hipMemcpyAsync(c->tsel, order, steps * batch * sizeof(uint32_t), hipMemcpyHostToDevice, c->stream));
     for (size_t s = 0; s < steps; ++s) {
-        int rc = enqueue_gradient(c, c->tfeat, c->ttarget, c->tsel + s * batch, batch, c->tloss + s);
-        if (!rc) rc = enqueue_adam(c, lr);
+        int rc = enqueue_gradient(c, c->tfeat, c->ttarget, c->tsel + s * batch, batch);
+        if (!rc) rc = enqueue_adam(c, gradient_sum(c, batch, c->tloss + s), lr);
         if (rc) return rc;
     }
     if (losses)

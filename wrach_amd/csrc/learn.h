@@ -78,38 +78,47 @@ hipError_t launch_learn_infer(const MlpWeights &w, const InferArgs &a, hipStream
 uint32_t resident_blocks_infer();
 
 // One training step's buffers (batch rows bsz, a multiple of 64).
+constexpr uint32_t kWeights = kFeat * kHid + kHid * kHid;  // dW1 and dW2 of a chunk
+constexpr uint32_t kCols = 4 * kHid + 3;                   // b1, b2, W3, b3, squared error
 struct TrainArgs {
     const uint16_t *feat;    // training rows
     const float2 *target;    // their targets
     const uint32_t *sel;     // batch row p is training row sel[p]
     uint32_t bsz;
     float inv_bsz;           // 1 / bsz
-    // Feature-major activations and gradients ([feature][bsz]):
-    uint16_t *xt;            // [64][bsz] the inputs
-    uint16_t *a1t, *dz1t;    // [128][bsz] SiLU(z1), dL/dz1 (bf16)
-    uint16_t *dz2t;          // [128][bsz] dL/dz2 (bf16)
-    float *a2t;              // [128][bsz] SiLU(z2)
+    // The weight gradients' k chunks: `chunks` of kc rows, a multiple of 32
+    // (the last one possibly shorter).
+    uint32_t kc, chunks;
+    // Activations and gradients, per 16 batch rows [feature][16]:
+    uint16_t *xt;            // 64 features: the inputs
+    uint16_t *a1t, *dz1t;    // 128: SiLU(z1), dL/dz1 (bf16)
+    uint16_t *dz2t;          // 128: dL/dz2 (bf16)
+    float *a2t;              // 128: SiLU(z2)
     float *dyt;              // [2][bsz] dL/dy
-    float *sqerr;            // [bsz / 16] squared error per 16-row tile
+    float *sqerr;            // [bsz / 16] squared error per 16 rows
+    float *part;             // [chunks][kWeights]
+    float *cols;             // [kCols] column sums
 };
-hipError_t launch_learn_rows(const MlpWeights &w, const TrainArgs &a, hipStream_t stream);
-// out[m][n] partial sums over k chunks: part[c][m][n] = sum over
-// k in [c * kc, (c + 1) * kc) of A[m][k] * B[n][k] (bf16, row length ldk).
-hipError_t launch_learn_gemm_nt(const uint16_t *A, const uint16_t *B, uint32_t M, uint32_t N,
-                                uint32_t ldk, uint32_t kc, uint32_t chunks, float *part,
-                                hipStream_t stream);
-// grad[kOff..] from the GEMM partials (dW1, dW2), the column sums (b1,
-// b2, W3, b3) and the loss (sum of sqerr / (2 bsz)) into loss_out.
-hipError_t launch_learn_reduce(const TrainArgs &a, const float *part1, const float *part2,
-                               uint32_t chunks, float *grad, float *loss_out, hipStream_t stream);
-// Adam on the master vector (f32, in place), then the packed weights.
-struct AdamArgs {
+// part and cols.
+hipError_t launch_learn_grad(const MlpWeights &w, const TrainArgs &a, hipStream_t stream);
+// The gradient from part and cols, or `given`; with `grad` it is written
+// there, otherwise Adam on the master vector (f32, in place) and the packed
+// weights.
+struct UpdateArgs {
+    const float *part;
+    const float *cols;
+    uint32_t chunks;
+    const float *given;
+    float *loss;        // loss_scale * the sum of squared errors (if not null)
+    float loss_scale;
+    float *grad;
     float *params, *m, *v;
-    const float *grad;
+    uint16_t *frag;
+    float *w3;
     float lr, beta1, beta2, eps;
     float c1, c2;  // 1 / (1 - beta1^t), 1 / (1 - beta2^t)
 };
-hipError_t launch_learn_adam(const AdamArgs &a, hipStream_t stream);
+hipError_t launch_learn_update(const UpdateArgs &u, hipStream_t stream);
 hipError_t launch_learn_pack(const float *params, uint16_t *frag, float *w3, hipStream_t stream);
 // target[row0 + i] = pk[i] - p0[i] for i < n.
 hipError_t launch_learn_target(const float2 *pk, const float2 *p0, float2 *target, uint32_t row0,

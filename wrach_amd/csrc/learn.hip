@@ -1,7 +1,7 @@
 // The learned warm start's network on gfx950: 64 -> 128 -> 128 -> 2 with
 // SiLU, bf16 weights and activations into v_mfma_f32_16x16x32_bf16 with f32
 // accumulation; inference, the training rows (forward + backward through the
-// layers), the weight-gradient GEMMs, the reductions and Adam.  No
+// layers), the weight gradients and Adam.  No
 // counterpart in the reference, whose separation is one Gauss-Seidel sweep
 // per cell (shaders/physics/src/particles.rs:62-93); the network predicts
 // the displacement that the plain separation passes produce, and those
@@ -73,85 +73,13 @@ __device__ __forceinline__ f32x4 mfma(bf16x8 a, bf16x8 b, f32x4 c) {
     return __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b, c, 0, 0, 0);
 }
 
-// Forward pass of NC column tiles (16 particles each) by one wavefront.
-// xb[c][s]: layer-1 B operands (feature rows).  frag: the packed
-// fragments (global or LDS).  Leaves z1, z2 (pre-activations) and y (the
-// output, summed over the lane groups: every lane holds its particle's y).
-template <int NC, typename FragPtr>
-__device__ __forceinline__ void mlp_forward(const bf16x8 (&xb)[NC][2], FragPtr frag,
-                                            const float *b1, const float *b2, const float *w3,
-                                            const float *b3, f32x4 (&z1)[8][NC], f32x4 (&z2)[8][NC],
-                                            float (&y)[NC][2]) {
-    const uint32_t l = lane_id(), g = l >> 4;
-#pragma unroll
-    for (int t = 0; t < 8; ++t) {
-        f32x4 bias;
-#pragma unroll
-        for (int r = 0; r < 4; ++r) bias[r] = b1[16 * t + 4 * g + r];
-#pragma unroll
-        for (int c = 0; c < NC; ++c) z1[t][c] = bias;
-#pragma unroll
-        for (int s = 0; s < 2; ++s) {
-            const bf16x8 a = frag[(kFragW1 + t * 2 + s) * 64 + l];
-#pragma unroll
-            for (int c = 0; c < NC; ++c) z1[t][c] = mfma(a, xb[c][s], z1[t][c]);
-        }
-    }
-    // Layer 2: B operands from layer 1's registers (permuted k).
-    bf16x8 h1[NC][4];
-#pragma unroll
-    for (int c = 0; c < NC; ++c)
-#pragma unroll
-        for (int s = 0; s < 4; ++s) {
-            float v[8];
-#pragma unroll
-            for (int r = 0; r < 4; ++r) {
-                v[r] = silu(z1[2 * s][c][r]);
-                v[4 + r] = silu(z1[2 * s + 1][c][r]);
-            }
-            h1[c][s] = pack8(v);
-        }
-#pragma unroll
-    for (int t = 0; t < 8; ++t) {
-        f32x4 bias;
-#pragma unroll
-        for (int r = 0; r < 4; ++r) bias[r] = b2[16 * t + 4 * g + r];
-#pragma unroll
-        for (int c = 0; c < NC; ++c) z2[t][c] = bias;
-#pragma unroll
-        for (int s = 0; s < 4; ++s) {
-            const bf16x8 a = frag[(kFragW2F + t * 4 + s) * 64 + l];
-#pragma unroll
-            for (int c = 0; c < NC; ++c) z2[t][c] = mfma(a, h1[c][s], z2[t][c]);
-        }
-    }
-    // Layer 3 (128 -> 2) on the vector ALUs: each lane group sums its 32
-    // outputs, then the four groups are added.
-#pragma unroll
-    for (int c = 0; c < NC; ++c) {
-        float y0 = 0.0f, y1 = 0.0f;
-#pragma unroll
-        for (int t = 0; t < 8; ++t)
-#pragma unroll
-            for (int r = 0; r < 4; ++r) {
-                const uint32_t o = 16 * t + 4 * g + r;
-                const float a2 = silu(z2[t][c][r]);
-                y0 = fmaf(a2, w3[2 * o], y0);
-                y1 = fmaf(a2, w3[2 * o + 1], y1);
-            }
-        y0 += __shfl_xor(y0, 16, 64);
-        y1 += __shfl_xor(y1, 16, 64);
-        y0 += __shfl_xor(y0, 32, 64);
-        y1 += __shfl_xor(y1, 32, 64);
-        y[c][0] = y0 + b3[0];
-        y[c][1] = y1 + b3[1];
-    }
-}
-
-// Inference of NC column tiles with few live registers: layer 1 a pair of
-// output tiles at a time (one k-step of layer 2's B operands), layer 2 one
-// output tile at a time, folded straight into layer 3.  Same arithmetic as
-// mlp_forward, in the same order.
+// Inference of NC column tiles (16 particles each) by one wavefront with few
+// live registers: layer 1 a pair of output tiles at a time (one k-step of
+// layer 2's B operands, its k order permuted), layer 2 one output tile at a
+// time, folded straight into layer 3 (128 -> 2, on the vector ALUs: each
+// lane group sums its 32 outputs, then the four groups are added).  xb[c][s]:
+// layer-1 B operands (feature rows); frag: the packed fragments (global or
+// LDS).  The same arithmetic in the same order as a training row's.
 template <int NC, typename FragPtr>
 __device__ __forceinline__ void mlp_infer(const bf16x8 (&xb)[NC][2], FragPtr frag, const float *b1,
                                           const float *b2, const float *w3, const float *b3,
@@ -306,201 +234,358 @@ __global__ __launch_bounds__(kInferBlock) __attribute__((amdgpu_waves_per_eu(4))
 }
 
 // ---------------------------------------------------------------------------
-// Training rows: one wavefront per 16 batch rows.  Forward (kept in
-// registers), the output error, the backward pass through the layers (dW2's
-// transpose product on MFMA with the backward-packed W2), and the
-// feature-major activations and gradients the weight GEMMs read.
+// A training step is three launches, none of them near a rate of the chip at
+// 8,192 rows (1.1 GFLOP, 12 MB): each is a chain of latencies, so each
+// spreads its chain over as many wavefronts as it can.
+//
+// learn_rows_kernel     16 batch rows a block of 4 wavefronts, wavefront w
+//                       the output tiles 2w and 2w + 1 of every layer:
+//                       forward, output error and backward.  All weights a
+//                       wavefront needs (20 fragments) are on their way to
+//                       registers before the first product; the layers'
+//                       operands pass through LDS, a wavefront's two tiles
+//                       being exactly one k-step of the next layer.
+// learn_sums_kernel     the weight gradients, MFMA products over chunks of
+//                       the batch, one 16 x 16 tile a wavefront, and beside
+//                       them the column sums for b1, b2, W3, b3 and the loss.
+// learn_update_kernel   sums the chunks in order and applies Adam and the
+//                       packing of the new weights to each entry.
+//
+// Every sum keeps a fixed order (deterministic, and the same however the
+// work is spread).  With one wavefront a row tile, two product launches, a
+// reduction, Adam and the packing apart, a step of 8,192 rows took 26 + 2 * 6
+// + 20 + 5 + 4 us and 75 us with the gaps; now 12.8 + 9.1 + 4.7 and 41 us.
+// (One kernel for the rows and their products, partial gradients per block:
+// 22 us, and sums in another order.)
 
-__global__ __launch_bounds__(256) void learn_rows_kernel(MlpWeights w, TrainArgs a) {
+// The activations and gradients the weight gradients read: for every 16
+// batch rows a block of [feature][16 rows], so that a block of the rows
+// kernel writes whole lines and an operand's 8 rows of a feature are 16
+// bytes.
+__device__ __forceinline__ size_t tiled(uint32_t features, uint32_t f, uint32_t row) {
+    return ((size_t)(row >> 4) * features + f) * 16 + (row & 15);
+}
+
+__global__ __launch_bounds__(256, 2) void learn_rows_kernel(MlpWeights w, TrainArgs a) {
+    __shared__ bf16x8 s_h1[4][64], s_d2[4][64];
+    __shared__ f32x4 s_a2[8][64];
     const uint32_t l = lane_id(), g = l >> 4, col = l & 15;
-    const uint32_t tile = blockIdx.x * 4 + (threadIdx.x >> 6);
-    const uint32_t row0 = tile * 16;
-    if (row0 >= a.bsz) return;  // whole wavefronts (bsz is a multiple of 64)
-    const bf16x8 *frag = reinterpret_cast<const bf16x8 *>(w.frag);
-    bf16x8 xb[1][2];
-    load_rows<1>(a.feat, a.sel, row0, a.bsz, xb);
-    f32x4 z1[8][1], z2[8][1];
-    float y[1][2];
-    mlp_forward<1>(xb, frag, w.params + kOffB1, w.params + kOffB2, w.w3, w.params + kOffB3, z1, z2, y);
-    const uint32_t p = row0 + col;
-    const float2 tg = a.target[a.sel[p]];
-    const float e0 = y[0][0] - tg.x, e1 = y[0][1] - tg.y;
-    const float dy0 = e0 * a.inv_bsz, dy1 = e1 * a.inv_bsz;
-    // Squared error of the tile (lane group 0 holds each row once).
-    float se = g == 0 ? e0 * e0 + e1 * e1 : 0.0f;
+    const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const uint32_t p = blockIdx.x * 16 + col;
+    const uint32_t row = a.sel[p];
+    const bf16x8 *frag = reinterpret_cast<const bf16x8 *>(w.frag) + l;
+    // Loads, all in flight together: this wavefront's weights, the rows.
+    bf16x8 w1[2][2], w2f[2][4], w2b[2][4], xb[2];
+    f32x4 bias1[2], bias2[2], w3a[8], w3b[8];
 #pragma unroll
-    for (int o = 32; o > 0; o >>= 1) se += __shfl_xor(se, o, 64);
-    if (l == 0) a.sqerr[tile] = se;
-    if (g == 0) {
-        a.dyt[p] = dy0;
-        a.dyt[a.bsz + p] = dy1;
+    for (int h = 0; h < 2; ++h) {
+        const uint32_t t = 2 * wave + h;
+#pragma unroll
+        for (int s = 0; s < 2; ++s) w1[h][s] = frag[(kFragW1 + t * 2 + s) * 64];
+#pragma unroll
+        for (int s = 0; s < 4; ++s) w2f[h][s] = frag[(kFragW2F + t * 4 + s) * 64];
+#pragma unroll
+        for (int s = 0; s < 4; ++s) w2b[h][s] = frag[(kFragW2B + t * 4 + s) * 64];
+        bias1[h] = *reinterpret_cast<const f32x4 *>(w.params + kOffB1 + 16 * t + 4 * g);
+        bias2[h] = *reinterpret_cast<const f32x4 *>(w.params + kOffB2 + 16 * t + 4 * g);
     }
-    // dL/dz2 = (W3 . dy) * SiLU'(z2); the B operands of the transpose
-    // product, and the feature-major copies.
-    bf16x8 d2[4];
 #pragma unroll
-    for (int s = 0; s < 4; ++s) {
-        float v[8];
-#pragma unroll
-        for (int h = 0; h < 2; ++h)
-#pragma unroll
-            for (int r = 0; r < 4; ++r) {
-                const int t = 2 * s + h;
-                const uint32_t o = 16 * t + 4 * g + r;
-                const float z = z2[t][0][r];
-                float da = w.w3[2 * o] * dy0;
-                da = da + w.w3[2 * o + 1] * dy1;
-                const float dz = da * silu_grad(z);
-                v[4 * h + r] = dz;
-                a.a2t[(size_t)o * a.bsz + p] = silu(z);
-                a.dz2t[(size_t)o * a.bsz + p] = bf16_bits(dz);
-            }
-        d2[s] = pack8(v);
+    for (int t = 0; t < 8; ++t) {  // W3's rows of this lane group: outputs 16t + 4g ..
+        w3a[t] = *reinterpret_cast<const f32x4 *>(w.w3 + 2 * (16 * t + 4 * g));
+        w3b[t] = *reinterpret_cast<const f32x4 *>(w.w3 + 2 * (16 * t + 4 * g) + 4);
     }
-    // dL/da1 = W2 . dz2 (rows = layer-2 inputs), then dL/dz1.
+    const float b30 = w.params[kOffB3], b31 = w.params[kOffB3 + 1];
+#pragma unroll
+    for (int s = 0; s < 2; ++s)
+        xb[s] = *reinterpret_cast<const bf16x8 *>(a.feat + (size_t)row * kFeat + 32 * s + 8 * g);
+    const float2 tg = a.target[row];
+
+    f32x4 z1[2], z2[2];
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+        z1[h] = bias1[h];
+#pragma unroll
+        for (int s = 0; s < 2; ++s) z1[h] = mfma(w1[h][s], xb[s], z1[h]);
+    }
+    float v[8];
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+        v[r] = silu(z1[0][r]);
+        v[4 + r] = silu(z1[1][r]);
+    }
+    const bf16x8 h1 = pack8(v);
+    s_h1[wave][l] = h1;
+    __syncthreads();
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+        z2[h] = bias2[h];
+#pragma unroll
+        for (int s = 0; s < 4; ++s) z2[h] = mfma(w2f[h][s], s_h1[s][l], z2[h]);
+    }
+    f32x4 a2[2];
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+#pragma unroll
+        for (int r = 0; r < 4; ++r) a2[h][r] = silu(z2[h][r]);
+        s_a2[2 * wave + h][l] = a2[h];
+    }
+    __syncthreads();
+    // Layer 3, in every wavefront: each lane group sums its 32 outputs, then
+    // the four groups are added.
+    float y0 = 0.0f, y1 = 0.0f;
 #pragma unroll
     for (int t = 0; t < 8; ++t) {
-        f32x4 acc = {0.0f, 0.0f, 0.0f, 0.0f};
-#pragma unroll
-        for (int s = 0; s < 4; ++s) acc = mfma(frag[(kFragW2B + t * 4 + s) * 64 + l], d2[s], acc);
+        const f32x4 h = s_a2[t][l];
 #pragma unroll
         for (int r = 0; r < 4; ++r) {
-            const uint32_t o = 16 * t + 4 * g + r;
-            const float z = z1[t][0][r];
-            a.a1t[(size_t)o * a.bsz + p] = bf16_bits(silu(z));
-            a.dz1t[(size_t)o * a.bsz + p] = bf16_bits(acc[r] * silu_grad(z));
+            y0 = fmaf(h[r], r < 2 ? w3a[t][2 * (r & 1)] : w3b[t][2 * (r & 1)], y0);
+            y1 = fmaf(h[r], r < 2 ? w3a[t][2 * (r & 1) + 1] : w3b[t][2 * (r & 1) + 1], y1);
         }
     }
-    // The inputs, feature-major, from the raw bits of the B operands (a
-    // whole-vector cast: subscripting the bf16 vector type here read
-    // element 0 for every element).
+    y0 += __shfl_xor(y0, 16, 64);
+    y1 += __shfl_xor(y1, 16, 64);
+    y0 += __shfl_xor(y0, 32, 64);
+    y1 += __shfl_xor(y1, 32, 64);
+    const float e0 = (y0 + b30) - tg.x, e1 = (y1 + b31) - tg.y;
+    const float dy0 = e0 * a.inv_bsz, dy1 = e1 * a.inv_bsz;
+    // dL/dz2 = (W3 . dy) * SiLU'(z2) of this wavefront's tiles.
+    f32x4 wa[2] = {w3a[0], w3a[1]}, wb[2] = {w3b[0], w3b[1]};
 #pragma unroll
-    for (int s = 0; s < 2; ++s) {
-        typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
-        const u32x4 w4 = __builtin_bit_cast(u32x4, xb[0][s]);
+    for (int t = 2; t < 8; ++t) {
+        const bool own = (uint32_t)(t >> 1) == wave;
+        wa[t & 1] = own ? w3a[t] : wa[t & 1];
+        wb[t & 1] = own ? w3b[t] : wb[t & 1];
+    }
 #pragma unroll
-        for (int e = 0; e < 8; ++e)
-            a.xt[(size_t)(32 * s + 8 * g + e) * a.bsz + p] = (uint16_t)(w4[e >> 1] >> (16 * (e & 1)));
+    for (int h = 0; h < 2; ++h)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+            const float u0 = r < 2 ? wa[h][2 * (r & 1)] : wb[h][2 * (r & 1)];
+            const float u1 = r < 2 ? wa[h][2 * (r & 1) + 1] : wb[h][2 * (r & 1) + 1];
+            float da = u0 * dy0;
+            da = da + u1 * dy1;
+            v[4 * h + r] = da * silu_grad(z2[h][r]);
+        }
+    typedef uint16_t u16x8 __attribute__((ext_vector_type(8)));
+    const bf16x8 d2 = pack8(v);
+    s_d2[wave][l] = d2;
+    __syncthreads();
+    // dL/da1 = W2 . dz2 (rows = layer-2 inputs), then dL/dz1.
+    f32x4 acc[2];
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+        acc[h] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+        for (int s = 0; s < 4; ++s) acc[h] = mfma(w2b[h][s], s_d2[s][l], acc[h]);
+    }
+    // What the weight gradients read.  (Turned in LDS to store 16 bytes a
+    // lane instead of 2: no faster, 12.8 us either way.)
+    const u16x8 h1b = __builtin_bit_cast(u16x8, h1), d2b = __builtin_bit_cast(u16x8, d2);
+#pragma unroll
+    for (int h = 0; h < 2; ++h)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+            const size_t at = tiled(kHid, 16 * (2 * wave + h) + 4 * g + r, p);
+            a.a2t[at] = a2[h][r];
+            a.dz2t[at] = d2b[4 * h + r];
+            a.a1t[at] = h1b[4 * h + r];
+            a.dz1t[at] = bf16_bits(acc[h][r] * silu_grad(z1[h][r]));
+        }
+    const u16x8 xw = __builtin_bit_cast(u16x8, wave < 2 ? xb[0] : xb[1]);
+#pragma unroll
+    for (int e = 0; e < 4; ++e)
+        a.xt[tiled(kFeat, 32 * (wave >> 1) + 8 * g + 4 * (wave & 1) + e, p)] = wave & 1 ? xw[4 + e] : xw[e];
+    if (wave == 0) {
+        // Squared error of the tile (lane group 0 holds each row once).
+        float se = g == 0 ? e0 * e0 + e1 * e1 : 0.0f;
+#pragma unroll
+        for (int o = 32; o > 0; o >>= 1) se += __shfl_xor(se, o, 64);
+        if (l == 0) a.sqerr[blockIdx.x] = se;
+        if (g == 0) {
+            a.dyt[p] = dy0;
+            a.dyt[a.bsz + p] = dy1;
+        }
     }
 }
 
-// part[c][m][n] = sum over k in chunk c (k < ldk) of A[m][k] B[n][k]: a
-// 32 x 32 output tile per block, one 16 x 16 MFMA tile per wavefront.
-__global__ __launch_bounds__(256) void learn_gemm_nt_kernel(const uint16_t *A, const uint16_t *B,
-                                                            uint32_t M, uint32_t N, uint32_t ldk,
-                                                            uint32_t kc, float *part) {
+// chunk c of in^T . dz: sum over its rows k of A[m][k] B[n][k], a 32 x 32
+// output tile per block, one 16 x 16 MFMA tile per wavefront.
+__device__ __forceinline__ void weight_tile(const uint16_t *A, uint32_t fa, const uint16_t *B, uint32_t m32,
+                                            uint32_t n32, uint32_t first, uint32_t rows, float *out) {
     const uint32_t l = lane_id(), g = l >> 4, wave = threadIdx.x >> 6;
-    const uint32_t m0 = blockIdx.x * 32 + (wave & 1) * 16, n0 = blockIdx.y * 32 + (wave >> 1) * 16;
-    const uint32_t chunk = blockIdx.z;
+    const uint32_t m0 = m32 * 32 + (wave & 1) * 16, n0 = n32 * 32 + (wave >> 1) * 16;
     f32x4 acc = {0.0f, 0.0f, 0.0f, 0.0f};
-    const uint16_t *ar = A + (size_t)(m0 + (l & 15)) * ldk + (size_t)chunk * kc + 8 * g;
-    const uint16_t *br = B + (size_t)(n0 + (l & 15)) * ldk + (size_t)chunk * kc + 8 * g;
-    const uint32_t kend = min(kc, ldk - chunk * kc);  // the last chunk may be shorter
-    for (uint32_t k = 0; k < kend; k += 32)
-        acc = mfma(*reinterpret_cast<const bf16x8 *>(ar + k), *reinterpret_cast<const bf16x8 *>(br + k), acc);
-    float *out = part + (size_t)chunk * M * N;
+    const uint16_t *ar = A + tiled(fa, m0 + (l & 15), first + 8 * g);
+    const uint16_t *br = B + tiled(kHid, n0 + (l & 15), first + 8 * g);
+    uint32_t k = 0;
+    for (; k + 128 <= rows; k += 128) {  // four steps' operands in flight together
+        bf16x8 x[4], y[4];
 #pragma unroll
-    for (int r = 0; r < 4; ++r) out[(size_t)(m0 + 4 * g + r) * N + n0 + (l & 15)] = acc[r];
-}
-
-// Sum of 256 per-thread partials in a fixed order (deterministic).
-__device__ __forceinline__ float block_sum(float v, float *s) {
-    s[threadIdx.x] = v;
-    __syncthreads();
-    for (uint32_t h = 128; h > 0; h >>= 1) {
-        if (threadIdx.x < h) s[threadIdx.x] += s[threadIdx.x + h];
-        __syncthreads();
-    }
-    const float r = s[0];
-    __syncthreads();
-    return r;
-}
-
-// Blocks 0..kFeat*kHid/256 - 1 and the next kHid*kHid/256: dW1 and dW2
-// from the GEMM partials (summed in chunk order), one element per thread.
-// Then one block per bias entry / W3 row (column sums over the batch in a
-// fixed order), and a last block for b3 and the loss.
-constexpr uint32_t kGradBlocksW = (kFeat * kHid + kHid * kHid) / 256;
-
-__global__ __launch_bounds__(256) void learn_reduce_kernel(TrainArgs a, const float *part1,
-                                                           const float *part2, uint32_t chunks,
-                                                           float *grad, float *loss_out) {
-    __shared__ float s[256];
-    const uint32_t blk = blockIdx.x;
-    if (blk < kGradBlocksW) {
-        const uint32_t e = blk * 256 + threadIdx.x;
-        if (e < (uint32_t)(kFeat * kHid)) {
-            float v = 0.0f;
-            for (uint32_t c = 0; c < chunks; ++c) v += part1[(size_t)c * kFeat * kHid + e];
-            grad[kOffW1 + e] = v;
-        } else {
-            const uint32_t f = e - kFeat * kHid;
-            float v = 0.0f;
-            for (uint32_t c = 0; c < chunks; ++c) v += part2[(size_t)c * kHid * kHid + f];
-            grad[kOffW2 + f] = v;
+        for (int s = 0; s < 4; ++s) {
+            x[s] = *reinterpret_cast<const bf16x8 *>(ar + (size_t)(k + 32 * s) * fa);
+            y[s] = *reinterpret_cast<const bf16x8 *>(br + (size_t)(k + 32 * s) * kHid);
         }
+#pragma unroll
+        for (int s = 0; s < 4; ++s) acc = mfma(x[s], y[s], acc);
+    }
+    for (; k < rows; k += 32)
+        acc = mfma(*reinterpret_cast<const bf16x8 *>(ar + (size_t)k * fa),
+                   *reinterpret_cast<const bf16x8 *>(br + (size_t)k * kHid), acc);
+#pragma unroll
+    for (int r = 0; r < 4; ++r) out[(size_t)(m0 + 4 * g + r) * kHid + n0 + (l & 15)] = acc[r];
+}
+
+// Sums of 256 per-thread partials, N of them at once, in a fixed order
+// (halves added to halves); thread 0 has them.
+template <int N>
+__device__ __forceinline__ void block_sums(float (&v)[N], float (*s)[256]) {
+    const uint32_t t = threadIdx.x;
+#pragma unroll
+    for (int q = 0; q < N; ++q) s[q][t] = v[q];
+    __syncthreads();
+    if (t < 128)
+#pragma unroll
+        for (int q = 0; q < N; ++q) v[q] = s[q][t] + s[q][t + 128];
+    __syncthreads();
+    if (t < 128)
+#pragma unroll
+        for (int q = 0; q < N; ++q) s[q][t] = v[q];
+    __syncthreads();
+    if (t < 64) {
+#pragma unroll
+        for (int q = 0; q < N; ++q) {
+            v[q] += s[q][t + 64];
+#pragma unroll
+            for (int h = 32; h > 0; h >>= 1) v[q] += __shfl_down(v[q], h, 64);
+        }
+    }
+}
+
+// Blocks: first the column sums, the longest, four columns a block (whole
+// lines of the tiled arrays): b1, b2, W3's rows, then b3 and the loss; after
+// them the chunks' tiles of dW1 (2 x 4) and dW2 (4 x 4).
+constexpr uint32_t kColBlocks = 3 * kHid / 4 + 1;
+
+__global__ __launch_bounds__(256) void learn_sums_kernel(TrainArgs a) {
+    __shared__ float s[8][256];
+    uint32_t blk = blockIdx.x;
+    if (blk >= kColBlocks) {
+        blk -= kColBlocks;
+        // Blocks go to the 8 XCDs in turn: a chunk's 24 tiles on one of them,
+        // whose L2 then fetches its rows once.
+        const uint32_t c = blk % 8 + blk / 192 * 8, q = blk / 8 % 24, first = c * a.kc;
+        if (c >= a.chunks) return;
+        const uint32_t rows = min(a.kc, a.bsz - first);  // the last chunk may be shorter
+        float *part = a.part + (size_t)c * kWeights;
+        if (q < 8) weight_tile(a.xt, kFeat, a.dz1t, q / 4, q % 4, first, rows, part);
+        else weight_tile(a.a1t, kHid, a.dz2t, (q - 8) / 4, q % 4, first, rows, part + kFeat * kHid);
         return;
     }
-    const uint32_t j = blk - kGradBlocksW;
-    if (j < (uint32_t)kHid) {  // b1
-        float v = 0.0f;
-        for (uint32_t p = threadIdx.x; p < a.bsz; p += 256) v += bf16_float(a.dz1t[(size_t)j * a.bsz + p]);
-        v = block_sum(v, s);
-        if (threadIdx.x == 0) grad[kOffB1 + j] = v;
-    } else if (j < 2u * kHid) {  // b2
-        const uint32_t o = j - kHid;
-        float v = 0.0f;
-        for (uint32_t p = threadIdx.x; p < a.bsz; p += 256) v += bf16_float(a.dz2t[(size_t)o * a.bsz + p]);
-        v = block_sum(v, s);
-        if (threadIdx.x == 0) grad[kOffB2 + o] = v;
-    } else if (j < 3u * kHid) {  // W3 row o
-        const uint32_t o = j - 2 * kHid;
-        float v0 = 0.0f, v1 = 0.0f;
+    float *cols = a.cols;
+    if (blk < 2u * kHid / 4) {  // b1, b2
+        const uint32_t o = blk % (kHid / 4) * 4;
+        const uint16_t *d = blk < (uint32_t)kHid / 4 ? a.dz1t : a.dz2t;
+        float v[4] = {0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll 8
         for (uint32_t p = threadIdx.x; p < a.bsz; p += 256) {
-            const float h = a.a2t[(size_t)o * a.bsz + p];
-            v0 = fmaf(h, a.dyt[p], v0);
-            v1 = fmaf(h, a.dyt[a.bsz + p], v1);
+            const uint16_t *e = d + tiled(kHid, o, p);
+#pragma unroll
+            for (int q = 0; q < 4; ++q) v[q] += bf16_float(e[16 * q]);
         }
-        v0 = block_sum(v0, s);
-        v1 = block_sum(v1, s);
-        if (threadIdx.x == 0) {
-            grad[kOffW3 + 2 * o] = v0;
-            grad[kOffW3 + 2 * o + 1] = v1;
-        }
-    } else {  // b3 and the loss
-        float v0 = 0.0f, v1 = 0.0f, se = 0.0f;
+        block_sums<4>(v, s);
+        if (threadIdx.x == 0)
+#pragma unroll
+            for (int q = 0; q < 4; ++q) cols[(blk < (uint32_t)kHid / 4 ? 0 : kHid) + o + q] = v[q];
+    } else if (blk < 3u * kHid / 4) {  // W3 rows o .. o + 3
+        const uint32_t o = (blk - 2 * kHid / 4) * 4;
+        float v[8] = {0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll 8
         for (uint32_t p = threadIdx.x; p < a.bsz; p += 256) {
-            v0 += a.dyt[p];
-            v1 += a.dyt[a.bsz + p];
+            const float *e = a.a2t + tiled(kHid, o, p);
+            const float d0 = a.dyt[p], d1 = a.dyt[a.bsz + p];
+#pragma unroll
+            for (int q = 0; q < 4; ++q) {
+                const float h = e[16 * q];
+                v[2 * q] = fmaf(h, d0, v[2 * q]);
+                v[2 * q + 1] = fmaf(h, d1, v[2 * q + 1]);
+            }
         }
-        for (uint32_t t = threadIdx.x; t < a.bsz / 16; t += 256) se += a.sqerr[t];
-        v0 = block_sum(v0, s);
-        v1 = block_sum(v1, s);
-        se = block_sum(se, s);
-        if (threadIdx.x == 0) {
-            grad[kOffB3] = v0;
-            grad[kOffB3 + 1] = v1;
-            if (loss_out) *loss_out = se * (0.5f * a.inv_bsz);
+        block_sums<8>(v, s);
+        if (threadIdx.x == 0)
+#pragma unroll
+            for (int q = 0; q < 8; ++q) cols[2 * kHid + 2 * o + q] = v[q];
+    } else {  // b3 and the squared error
+        float v[3] = {0.0f, 0.0f, 0.0f};
+        for (uint32_t p = threadIdx.x; p < a.bsz; p += 256) {
+            v[0] += a.dyt[p];
+            v[1] += a.dyt[a.bsz + p];
         }
+        for (uint32_t t = threadIdx.x; t < a.bsz / 16; t += 256) v[2] += a.sqerr[t];
+        block_sums<3>(v, s);
+        if (threadIdx.x == 0)
+#pragma unroll
+            for (int q = 0; q < 3; ++q) cols[4 * kHid + q] = v[q];
     }
 }
 
-// Adam (Kingma & Ba, 2015) on the master vector, each step a rounded f32
-// operation in this order (no contraction).
-__global__ __launch_bounds__(256) void learn_adam_kernel(AdamArgs a) {
-    const uint32_t i = blockIdx.x * 256 + threadIdx.x;
-    if (i >= kParams) return;
-    const float gr = a.grad[i];
-    float m = a.beta1 * a.m[i];
-    m = m + (1.0f - a.beta1) * gr;
-    float v = a.beta2 * a.v[i];
-    v = v + (1.0f - a.beta2) * (gr * gr);
-    a.m[i] = m;
-    a.v[i] = v;
-    const float mh = m * a.c1;
-    const float vh = v * a.c2;
-    const float step = a.lr * mh / (sqrtf(vh) + a.eps);
-    a.params[i] = a.params[i] - step;
+// Where entry (k, o) of a weight matrix lies in its fragments: rows of the A
+// operand are `row`, its k-step entries `k`; natural or permuted k order
+// (the inverse of kmap).
+__device__ __forceinline__ uint32_t frag_index(uint32_t first, uint32_t steps, uint32_t row, uint32_t k,
+                                               bool permuted) {
+    const uint32_t s = k / 32, q = k % 32;
+    const uint32_t g = permuted ? (q % 16) / 4 : q / 8, e = permuted ? q % 4 + (q < 16 ? 0u : 4u) : q % 8;
+    return (first + row / 16 * steps + s) * kFragElems + (16 * g + row % 16) * 8 + e;
+}
+
+// One entry a thread (64-thread blocks, so that the 25,090 reach every CU):
+// its gradient -- the chunks' sums in order, or the column sum -- and then
+// that gradient out (u.grad), or Adam (Kingma & Ba, 2015) on the master
+// vector, each step a rounded f32 operation in this order (no contraction),
+// and the packing of the new value.
+__global__ __launch_bounds__(64) void learn_update_kernel(UpdateArgs u) {
+    const uint32_t i = blockIdx.x * 64 + threadIdx.x;
+    if (i >= kParams) {
+        if (i == kParams && u.loss) *u.loss = u.cols[4 * kHid + 2] * u.loss_scale;
+        return;
+    }
+    float gr;
+    if (u.given) {
+        gr = u.given[i];
+    } else if (i < kOffB1 || (i >= kOffW2 && i < kOffB2)) {
+        const float *q = u.part + (i < kOffB1 ? i : i - kOffW2 + kFeat * kHid);
+        gr = 0.0f;
+#pragma unroll 32
+        for (uint32_t c = 0; c < u.chunks; ++c) gr += q[(size_t)c * kWeights];
+    } else {
+        gr = u.cols[i < kOffW2 ? i - kOffB1 : i < kOffW3 ? i - kOffB2 + kHid : i - kOffW3 + 2 * kHid];
+    }
+    if (u.grad) {
+        u.grad[i] = gr;
+        return;
+    }
+    float m = u.beta1 * u.m[i];
+    m = m + (1.0f - u.beta1) * gr;
+    float q = u.beta2 * u.v[i];
+    q = q + (1.0f - u.beta2) * (gr * gr);
+    u.m[i] = m;
+    u.v[i] = q;
+    const float mh = m * u.c1;
+    const float vh = q * u.c2;
+    const float step = u.lr * mh / (sqrtf(vh) + u.eps);
+    const float x = u.params[i] - step;
+    u.params[i] = x;
+    const uint16_t h = bf16_bits(x);
+    if (i < kOffB1) {
+        const uint32_t k = i / kHid, o = i % kHid;
+        u.frag[frag_index(kFragW1, 2, o, k, false)] = h;
+    } else if (i >= kOffW2 && i < kOffB2) {
+        const uint32_t k = (i - kOffW2) / kHid, o = (i - kOffW2) % kHid;
+        u.frag[frag_index(kFragW2F, 4, o, k, true)] = h;
+        u.frag[frag_index(kFragW2B, 4, k, o, true)] = h;
+    } else if (i >= kOffW3 && i < kOffB3) {
+        u.w3[i - kOffW3] = bf16_float(h);
+    }
 }
 
 // Fragments and the rounded W3 from the master vector: one thread per
@@ -554,32 +639,20 @@ hipError_t launch_learn_infer(const MlpWeights &w, const InferArgs &a, hipStream
     return hipGetLastError();
 }
 
-hipError_t launch_learn_rows(const MlpWeights &w, const TrainArgs &a, hipStream_t stream) {
-    if (a.bsz == 0 || a.bsz % 64) return hipErrorInvalidValue;
-    hipLaunchKernelGGL(learn_rows_kernel, dim3(a.bsz / 64), dim3(256), 0, stream, w, a);
-    return hipGetLastError();
-}
-
-hipError_t launch_learn_gemm_nt(const uint16_t *A, const uint16_t *B, uint32_t M, uint32_t N,
-                                uint32_t ldk, uint32_t kc, uint32_t chunks, float *part,
-                                hipStream_t stream) {
-    if (M % 32 || N % 32 || kc % 32 || ldk % 32 || chunks == 0 || (size_t)kc * (chunks - 1) >= ldk ||
-        (size_t)kc * chunks < ldk)
+hipError_t launch_learn_grad(const MlpWeights &w, const TrainArgs &a, hipStream_t stream) {
+    if (a.bsz == 0 || a.bsz % 64 || a.kc == 0 || a.kc % 32 || a.chunks == 0 ||
+        (size_t)a.kc * (a.chunks - 1) >= a.bsz || (size_t)a.kc * a.chunks < a.bsz)
         return hipErrorInvalidValue;
-    hipLaunchKernelGGL(learn_gemm_nt_kernel, dim3(M / 32, N / 32, chunks), dim3(256), 0, stream, A, B, M,
-                       N, ldk, kc, part);
+    hipLaunchKernelGGL(learn_rows_kernel, dim3(a.bsz / 16), dim3(256), 0, stream, w, a);
+    const hipError_t e = hipGetLastError();
+    if (e != hipSuccess) return e;
+    hipLaunchKernelGGL(learn_sums_kernel, dim3((a.chunks + 7) / 8 * 8 * 24 + kColBlocks), dim3(256), 0, stream, a);
     return hipGetLastError();
 }
 
-hipError_t launch_learn_reduce(const TrainArgs &a, const float *part1, const float *part2,
-                               uint32_t chunks, float *grad, float *loss_out, hipStream_t stream) {
-    hipLaunchKernelGGL(learn_reduce_kernel, dim3(kGradBlocksW + 3 * kHid + 1), dim3(256), 0, stream, a,
-                       part1, part2, chunks, grad, loss_out);
-    return hipGetLastError();
-}
-
-hipError_t launch_learn_adam(const AdamArgs &a, hipStream_t stream) {
-    hipLaunchKernelGGL(learn_adam_kernel, dim3((kParams + 255) / 256), dim3(256), 0, stream, a);
+hipError_t launch_learn_update(const UpdateArgs &u, hipStream_t stream) {
+    if (!u.given && (!u.part || !u.cols || u.chunks == 0)) return hipErrorInvalidValue;
+    hipLaunchKernelGGL(learn_update_kernel, dim3((kParams + 64) / 64), dim3(64), 0, stream, u);
     return hipGetLastError();
 }
 
