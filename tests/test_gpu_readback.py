@@ -1,0 +1,67 @@
+"""The readback's canonical order and the upload's counts at the sizes where
+their kernels change path, against the oracle's packer, bit for bit (needs a
+GPU)."""
+import numpy as np
+import pytest
+
+from tests.test_gpu_parity import f32, say
+from wrach_amd import World, WrachConfig, WrachError, _lib
+
+pytestmark = pytest.mark.gpu
+
+
+def packed_by_the_oracle(oracle, cfg, pos, vel):
+    W, H = cfg.dimensions
+    return oracle.pack(pos, vel, (0, 0, W, H), cfg.cell_size)
+
+
+def assert_packed(got, want, what):
+    for a, b, name in zip(got, want, ("indices", "positions", "velocities")):
+        assert a.shape == b.shape, f"{what}: {name} shape"
+        assert np.array_equal(a.view(np.uint32), b.view(np.uint32)), f"{what}: {name} differ"
+
+
+@pytest.mark.parametrize("m", [1, 2, 3, 16, 63, 64, 65, 128, 257, 703, 704, 705, 2048, 2049])
+@pytest.mark.parametrize("shift", [0, 1, 37, 63])
+def test_canonical_order_of_a_cell(oracle, m, shift):
+    """A cell of m particles that starts at packed index `shift`, one of the
+    same size right behind it, then a few lone ones, right after an upload:
+    every particle is a run of its own there, in arbitrary order.  Cells
+    inside a wavefront, past its end, over several, and those that a block
+    sorts (over 704, in LDS and past it)."""
+    rng = np.random.default_rng(100 * m + shift)
+    n = shift + 2 * m + 5
+    cell = np.concatenate([np.arange(shift) % 7, np.full(m, 8), np.full(m, 9), 12 + np.arange(5)])
+    pos = f32(np.stack([cell + rng.uniform(0.01, 0.99, n), rng.uniform(0.01, 0.99, n)], 1))
+    vel = f32(rng.uniform(-1, 1, (n, 2)))
+    order = rng.permutation(n)
+    pos, vel = pos[order], vel[order]
+    cfg = WrachConfig(dimensions=(96, 64), cell_size=1)
+    with World(cfg) as w:
+        w.add_particles(pos, vel)
+        assert_packed(w.read(), packed_by_the_oracle(oracle, cfg, pos, vel), f"m={m} shift={shift}")
+
+
+@pytest.mark.parametrize("n", [1, 64, 65, 255, 257, 4000])
+def test_upload_counts_with_particles_outside(oracle, n):
+    """The inside count of the device binning from its striped count of the
+    particles outside: none, some, all of them, and a refused upload's."""
+    rng = np.random.default_rng(n)
+    cfg = WrachConfig(dimensions=(60, 60), cell_size=3)
+    for share in (0.0, 0.3, 1.0):
+        pos = f32(rng.uniform(0, 60, (n, 2)))
+        out = rng.uniform(0, 1, n) < share
+        pos[out] = f32(rng.uniform(70, 90, (int(out.sum()), 2))) * np.where(rng.uniform(0, 1, (int(out.sum()), 1)) < 0.5,
+                                                                         np.float32(-1), np.float32(1))
+        vel = f32(rng.uniform(-1, 1, (n, 2)))
+        say(f"[readback] upload of {n}, {int(out.sum())} outside")
+        with World(cfg) as w:
+            w.add_particles(pos, vel)
+            want = packed_by_the_oracle(oracle, cfg, pos, vel)
+            assert w.n_particles == len(want[1])
+            assert_packed(w.read(), want, f"n={n} share={share}")
+            many = np.tile(np.float32([[30, 30]]), (w.capacity + 1, 1))
+            with pytest.raises(WrachError) as e:
+                w.add_particles(many, np.zeros_like(many))
+            assert e.value.code == _lib.WRACH_E_CAPACITY
+            assert_packed(w.read(), want, f"n={n} share={share}, after a refused upload")

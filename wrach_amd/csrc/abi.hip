@@ -94,7 +94,7 @@ struct wrach_ctx {
     std::vector<float> store_pos, store_vel;
     float2 *dstore_pos = nullptr, *dstore_vel = nullptr;
     uint2 *dks = nullptr;
-    uint32_t *dvalid = nullptr;
+    uint32_t *doutside = nullptr;
     size_t dstore_n = 0, dstore_cap = 0;
     uint32_t *dstore_world = nullptr;  // world of each store particle (a batch)
     uint32_t worlds = 1;               // worlds of a batch (one grid each, keys one after another)
@@ -382,7 +382,6 @@ void release(wrach_ctx *c) {
     (void)hipFree(c->buf.chunk_prefix);
     (void)hipFree(c->buf.epoch);
     (void)hipFree(c->buf.error);
-    (void)hipFree(c->buf.canon_ctr);
     if (c->err_host) (void)hipHostFree(c->err_host);
     (void)hipFree(c->dstore_pos);
     (void)hipFree(c->dstore_vel);
@@ -390,7 +389,7 @@ void release(wrach_ctx *c) {
     (void)hipFree(c->dstore_world);
     (void)hipFree(c->dgrids);
     (void)hipFree(c->dchunk_world);
-    (void)hipFree(c->dvalid);
+    (void)hipFree(c->doutside);
     (void)hipFree(c->buf.cells);
     (void)hipFree(c->buf.class_ctr);
     (void)hipFree(c->scell);
@@ -572,7 +571,7 @@ wrach::UploadParams store_params(const wrach_ctx *c, size_t n) {
     u.pos = c->dstore_pos;
     u.vel = c->dstore_vel;
     u.ks = c->dks;
-    u.valid = c->dvalid;
+    u.outside = c->doutside;
     u.n = (uint32_t)n;
     u.cs = (float)c->cfg.cell_size;
     u.gx = c->settings.grid_dimensions[0];
@@ -609,11 +608,13 @@ int add_device_packed(wrach_ctx *c, const float *pos_xy, const float *vel_xy, ui
                                         (int)world, n, c->stream));
     }
     const wrach::UploadParams u = store_params(c, total);
-    WRACH_HIP(hipMemsetAsync(c->dvalid, 0, sizeof(uint32_t), c->stream));
+    uint32_t outside[wrach::kOutsideStripes * wrach::kCtrStride];
+    WRACH_HIP(hipMemsetAsync(c->doutside, 0, sizeof outside, c->stream));
     WRACH_HIP(wrach::launch_upload_bin(u, c->buf, c->stream));
-    uint32_t packed = 0;
-    WRACH_HIP(hipMemcpyAsync(&packed, c->dvalid, sizeof packed, hipMemcpyDeviceToHost, c->stream));
+    WRACH_HIP(hipMemcpyAsync(outside, c->doutside, sizeof outside, hipMemcpyDeviceToHost, c->stream));
     WRACH_SETTLE(c);
+    uint32_t packed = (uint32_t)total;
+    for (uint32_t t = 0; t < wrach::kOutsideStripes; ++t) packed -= outside[t * wrach::kCtrStride];
     if (packed > c->capacity) {
         // the counts are the only state touched: clear them for the next frame
         WRACH_HIP(hipMemsetAsync(c->buf.cnt, 0, (c->ncell + 16) * sizeof(uint32_t), c->stream));
@@ -805,12 +806,11 @@ int create_ctx(const wrach_config *cfg, uint32_t n_worlds, const wrach_config *w
     WRACH_HIP_C(dmalloc(&b.chunk_prefix, c->chunks));
     WRACH_HIP_C(dmalloc(&b.epoch, 1));
     WRACH_HIP_C(dmalloc(&b.error, 1));
-    WRACH_HIP_C(dmalloc(&b.canon_ctr, 1));
     WRACH_HIP_C(hipHostMalloc((void **)&c->err_host, sizeof(uint32_t), hipHostMallocDefault));
     *c->err_host = 0;
     WRACH_HIP_C(dmalloc(&b.cells, ncells_total));
     WRACH_HIP_C(dmalloc(&b.class_ctr, wrach::kCtrWords));
-    WRACH_HIP_C(dmalloc(&c->dvalid, 1));
+    WRACH_HIP_C(dmalloc(&c->doutside, (size_t)wrach::kOutsideStripes * wrach::kCtrStride));
     WRACH_HIP_C(hipMemsetAsync(c->idx_alloc, 0, (nidx + 64) * sizeof(uint32_t), c->stream));
     WRACH_HIP_C(hipMemsetAsync(b.pos, 0, cap * sizeof(float2), c->stream));
     WRACH_HIP_C(hipMemsetAsync(b.vel, 0, cap * sizeof(float2), c->stream));
@@ -828,7 +828,6 @@ int create_ctx(const wrach_config *cfg, uint32_t n_worlds, const wrach_config *w
     }
     WRACH_HIP_C(hipMemsetAsync(b.class_ctr, 0, wrach::kCtrWords * sizeof(uint32_t), c->stream));
     WRACH_HIP_C(hipMemsetAsync(b.error, 0, sizeof(uint32_t), c->stream));
-    WRACH_HIP_C(hipMemsetAsync(b.canon_ctr, 0, sizeof(uint32_t), c->stream));
     if (world_cfgs) {
         std::vector<uint32_t> chunk_world(c->chunks);
         for (uint32_t w = 0; w < n_worlds; ++w) {
@@ -1221,9 +1220,7 @@ int wrach_canonical_device(wrach_ctx *c, wrach_device_view *out) {
     if (!c || !out) return fail(WRACH_E_INVALID, "null argument");
     WRACH_HIP(hipSetDevice(c->cfg.device));
     if (!c->canonical_valid) {
-        // the offsets of chunks the last scan found empty, then the order
-        WRACH_HIP(wrach::launch_materialize(c->fp, c->buf, c->stream));
-        if (c->fp.n > 0) WRACH_HIP(wrach::launch_canonical(c->fp, c->buf, c->stream));
+        WRACH_HIP(wrach::launch_canonical(c->fp, c->buf, nullptr, c->stream));
         c->canonical_valid = true;
     }
     out->indices = c->buf.idx;
@@ -2261,7 +2258,6 @@ size_t carve_noalloc(unsigned char *base, uint32_t n, uint64_t ncell, wrach::Fra
     b.chunk_prefix = reinterpret_cast<uint32_t *>(take(chunks * sizeof(uint32_t)));
     b.epoch = reinterpret_cast<uint32_t *>(take(sizeof(uint32_t)));
     b.error = reinterpret_cast<uint32_t *>(take(sizeof(uint32_t)));
-    b.canon_ctr = reinterpret_cast<uint32_t *>(take(sizeof(uint32_t)));
     b.class_ctr = reinterpret_cast<uint32_t *>(take(wrach::kCtrWords * sizeof(uint32_t)));
     ncells_total = 0;
     for (int k = 0; k < wrach::kClasses; ++k) {
@@ -2344,7 +2340,6 @@ int wrach_frame_noalloc(const wrach_world_settings *ws, const float gravity[2], 
     WRACH_HIP(wrach::launch_fill32(reinterpret_cast<uint32_t *>(b.chunk_live), 0x01010101u, (chunks + 3) / 4, st));
     WRACH_HIP(wrach::launch_fill32(b.epoch, 1u, 1, st));  // status words start at 0, never valid
     WRACH_HIP(wrach::launch_fill32(b.error, 0u, 1, st));
-    WRACH_HIP(wrach::launch_fill32(b.canon_ctr, 0u, 1, st));
     WRACH_HIP(wrach::launch_fill32(b.class_ctr, 0u, wrach::kCtrWords, st));
     // The caller's packed triple becomes the state (each cell one run).
     WRACH_HIP(wrach::launch_copy32(b.idx, indices, ncell + 2, st));
@@ -2359,8 +2354,7 @@ int wrach_frame_noalloc(const wrach_world_settings *ws, const float gravity[2], 
         WRACH_HIP(wrach::launch_cells(fp, b, st));
         WRACH_HIP(wrach::launch_scan(fp, b, st));
         WRACH_HIP(wrach::launch_scatter(fp, b, st));
-        WRACH_HIP(wrach::launch_materialize(fp, b, st));
-        WRACH_HIP(wrach::launch_canonical(fp, b, st));
+        WRACH_HIP(wrach::launch_canonical(fp, b, nullptr, st));
         WRACH_HIP(wrach::launch_copy32(reinterpret_cast<uint32_t *>(pos_xy), reinterpret_cast<const uint32_t *>(b.pos_out),
                                        2 * (size_t)n, st));
         WRACH_HIP(wrach::launch_copy32(reinterpret_cast<uint32_t *>(vel_xy), reinterpret_cast<const uint32_t *>(b.vel_out),

@@ -82,7 +82,6 @@ struct FrameBuffers {
     uint32_t *chunk_prefix;
     uint32_t *epoch;      // frame counter tagging the scan's status words; the scatter advances it
     uint32_t *error;      // kErr* bits raised by a kernel that gave up a wait; zero otherwise
-    uint32_t *canon_ctr;  // the readback's queue of large cells (zero outside launch_canonical)
     uint4 *cells;         // queued cells (s, n, cell, 0), one region per size class
     uint32_t *class_ctr;  // fill of every slice and overflow list (ctr_index); reset by the scan
     uint32_t class_off[8];  // first entry of each class's region in `cells`
@@ -136,7 +135,6 @@ constexpr int kScatterBlock = 256;
 constexpr int kScatterPerLane[] = {2, 1, 4};
 constexpr int kNumScatterShapes = 3;
 constexpr int kMaxInCell = 9;            // cell.rs:29-30
-constexpr int kRegCell = 16;             // cells up to this size sort in registers
 constexpr int kLdsSort = 2048;           // keys per LDS bitonic sort (block path)
 constexpr int kWavesPerBlock = kCollideBlock / 64;
 
@@ -184,7 +182,10 @@ hipError_t launch_scan(const FrameParams &p, const FrameBuffers &b, hipStream_t 
                        hipEvent_t start = nullptr, hipEvent_t stop = nullptr);
 hipError_t launch_scatter(const FrameParams &p, const FrameBuffers &b, hipStream_t stream,
                           hipEvent_t start = nullptr, hipEvent_t stop = nullptr);
-hipError_t launch_canonical(const FrameParams &p, const FrameBuffers &b, hipStream_t stream);
+// The canonical order of the state into pos_out/vel_out, and every offset:
+// idx made whole as launch_materialize does, or, with idx_out (ncell + 2
+// words), written there.
+hipError_t launch_canonical(const FrameParams &p, const FrameBuffers &b, uint32_t *idx_out, hipStream_t stream);
 // Fills the idx entries of chunks the last scan found empty (before a readback).
 hipError_t launch_materialize(const FrameParams &p, const FrameBuffers &b, hipStream_t stream);
 hipError_t launch_iota(uint32_t *dst, uint32_t n, hipStream_t stream);
@@ -197,13 +198,14 @@ hipError_t launch_keys_from_offsets(const uint32_t *idx, uint32_t ncell, uint32_
 hipError_t launch_fill32(uint32_t *dst, uint32_t v, size_t n, hipStream_t stream);
 hipError_t launch_copy32(uint32_t *dst, const uint32_t *src, size_t n, hipStream_t stream);
 
+constexpr uint32_t kOutsideStripes = 16;
 // Upload binning on the device: the store (every particle added, in
 // insertion order) and where its particles go.
 struct UploadParams {
     const float2 *pos;  // store positions
     const float2 *vel;  // store velocities
     uint2 *ks;          // per store particle: (cell key or ~0, slot in the cell)
-    uint32_t *valid;    // particles inside the grid (one counter)
+    uint32_t *outside;  // particles outside the grid: kOutsideStripes counters kCtrStride words apart
     uint32_t n;         // store size, < 2^31
     float cs;           // cell side
     uint32_t gx, gy;    // grid dimensions
@@ -213,8 +215,8 @@ struct UploadParams {
     const WorldGrid *grids;  // worlds of different sizes: each world's grid (else null)
     int32_t blx, bly;       // the grid's bottom-left cell: the view anchor / cell size
 };
-// Cell and slot of every store particle, counts into b.cnt, inside-grid
-// total into u.valid (zeroed by the caller).
+// Cell and slot of every store particle, counts into b.cnt, those outside
+// the grid into u.outside (zeroed by the caller).
 hipError_t launch_upload_bin(const UploadParams &u, const FrameBuffers &b, hipStream_t stream);
 // The store's particles outside the grid in store order, copied to
 // dpos/dvel from index base on: counts[b] receives block b's number (blocks
