@@ -1,10 +1,13 @@
 """The readback's canonical order and the upload's counts at the sizes where
 their kernels change path, against the oracle's packer, bit for bit (needs a
 GPU)."""
+import ctypes
+
 import numpy as np
 import pytest
 
 from tests.test_gpu_parity import f32, say
+from tests.test_zz_no_alloc import Hip
 from wrach_amd import World, WrachConfig, WrachError, _lib
 
 pytestmark = pytest.mark.gpu
@@ -65,3 +68,44 @@ def test_upload_counts_with_particles_outside(oracle, n):
                 w.add_particles(many, np.zeros_like(many))
             assert e.value.code == _lib.WRACH_E_CAPACITY
             assert_packed(w.read(), want, f"n={n} share={share}, after a refused upload")
+
+
+@pytest.mark.parametrize("m", [1, 8, 9, 64, 65, 300, 1200])
+@pytest.mark.parametrize("offset", [0, 4])
+def test_noalloc_frame_of_a_crowded_cell(oracle, m, offset):
+    """The allocation-free frame's start: cells of up to 8 particles by their
+    own thread, larger ones by their wavefront, more cells than particles and
+    the reverse; pairs on the caller's side aligned as float2 and only as
+    float; twice in a row, the second from what the first left."""
+    hip = Hip()
+    rng = np.random.default_rng(m + offset)
+    n = m + 40
+    pos = f32(np.concatenate([rng.uniform((3, 3), (3.99, 3.99), (m, 2)), rng.uniform(0, 30, (40, 2))]))
+    vel = f32(rng.uniform(-1, 1, (n, 2)))
+    cfg = WrachConfig(dimensions=(30, 30), cell_size=1, gravity=(0.0, -0.1))
+    idx, pos, vel = packed_by_the_oracle(oracle, cfg, pos, vel)
+    P = oracle.params(30, 30, 1, n, gravity=cfg.gravity)
+    ws = _lib.WorldSettingsC()
+    ws.view_dimensions[:] = [30.0, 30.0]
+    ws.view_anchor[:] = [0.0, 0.0]
+    ws.grid_dimensions[:] = [31, 31]
+    ws.cell_size = 1
+    ws.particles_in_frame_count = n
+    g = (ctypes.c_float * 2)(*cfg.gravity)
+    skip = offset // 4
+    arrays = [idx, np.concatenate([np.zeros(skip, np.float32), pos.ravel()]),
+              np.concatenate([np.zeros(skip, np.float32), vel.ravel()])]
+    di, dp, dv = (hip.upload(a) for a in arrays)
+    ref = (idx, pos, vel)
+    try:
+        for call in range(2):
+            say(f"[readback] noalloc m={m} offset={offset} call {call}")
+            assert _lib.load().wrach_frame_noalloc(ctypes.byref(ws), g, 1.0, di, dp.value + offset, dv.value + offset,
+                                                   n, None) == 0
+            assert hip.h.hipDeviceSynchronize() == 0
+            ref = oracle.step(P, *ref)
+            got = (hip.download(di, idx), hip.download(dp, arrays[1])[skip:].reshape(-1, 2),
+                   hip.download(dv, arrays[2])[skip:].reshape(-1, 2))
+            assert_packed(got, ref, f"m={m} offset={offset} call {call}")
+    finally:
+        hip.free(di, dp, dv)

@@ -2331,35 +2331,34 @@ int wrach_frame_noalloc(const wrach_world_settings *ws, const float gravity[2], 
     fp.wait_limit = wrach::kDefaultWaitLimit;
     fp.epoch_skew = 0;
     hipStream_t st = static_cast<hipStream_t>(stream);
-    const size_t chunks = (ncell + wrach::kChunkCells - 1) / wrach::kChunkCells;
-    const size_t tiles = (ncell + wrach::kMinScanTile - 1) / wrach::kMinScanTile;
-    // The array keeps the last call's contents: clear what starts at zero.
-    WRACH_HIP(wrach::launch_fill32(b.cnt, 0u, ncell + 16, st));
-    WRACH_HIP(wrach::launch_fill32(reinterpret_cast<uint32_t *>(b.tile_state), 0u, 2 * tiles, st));
-    WRACH_HIP(wrach::launch_fill32(reinterpret_cast<uint32_t *>(b.chunk_next), 0u, (chunks + 3) / 4, st));
-    WRACH_HIP(wrach::launch_fill32(reinterpret_cast<uint32_t *>(b.chunk_live), 0x01010101u, (chunks + 3) / 4, st));
-    WRACH_HIP(wrach::launch_fill32(b.epoch, 1u, 1, st));  // status words start at 0, never valid
-    WRACH_HIP(wrach::launch_fill32(b.error, 0u, 1, st));
-    WRACH_HIP(wrach::launch_fill32(b.class_ctr, 0u, wrach::kCtrWords, st));
-    // The caller's packed triple becomes the state (each cell one run).
-    WRACH_HIP(wrach::launch_copy32(b.idx, indices, ncell + 2, st));
-    if (n) {
-        WRACH_HIP(wrach::launch_copy32(reinterpret_cast<uint32_t *>(b.pos), reinterpret_cast<const uint32_t *>(pos_xy),
-                                       2 * (size_t)n, st));
-        WRACH_HIP(wrach::launch_copy32(reinterpret_cast<uint32_t *>(b.vel), reinterpret_cast<const uint32_t *>(vel_xy),
-                                       2 * (size_t)n, st));
-        WRACH_HIP(wrach::launch_iota(b.src, n, st));
-        WRACH_HIP(wrach::launch_keys_from_offsets(b.idx, (uint32_t)ncell, n, b.key, st));
-        WRACH_HIP(wrach::launch_collide(fp, b, st));
-        WRACH_HIP(wrach::launch_cells(fp, b, st));
-        WRACH_HIP(wrach::launch_scan(fp, b, st));
-        WRACH_HIP(wrach::launch_scatter(fp, b, st));
-        WRACH_HIP(wrach::launch_canonical(fp, b, nullptr, st));
-        WRACH_HIP(wrach::launch_copy32(reinterpret_cast<uint32_t *>(pos_xy), reinterpret_cast<const uint32_t *>(b.pos_out),
-                                       2 * (size_t)n, st));
-        WRACH_HIP(wrach::launch_copy32(reinterpret_cast<uint32_t *>(vel_xy), reinterpret_cast<const uint32_t *>(b.vel_out),
-                                       2 * (size_t)n, st));
-        WRACH_HIP(wrach::launch_copy32(indices, b.idx, ncell + 2, st));
+    if (n == 0) return WRACH_OK;  // an empty world does not change
+    // The collision reads the caller's triple (each cell one run), the re-bin
+    // writes the scratch arrays, and the canonical pass writes the caller's:
+    // nothing is copied but where the caller's pairs are not aligned as such.
+    const bool aligned = ((reinterpret_cast<uintptr_t>(pos_xy) | reinterpret_cast<uintptr_t>(vel_xy)) &
+                          (alignof(float2) - 1)) == 0;
+    wrach::FrameBuffers in = b, out = b;
+    in.idx = indices;
+    if (aligned) {
+        in.pos = out.pos_out = reinterpret_cast<float2 *>(pos_xy);
+        in.vel = out.vel_out = reinterpret_cast<float2 *>(vel_xy);
+    }
+    auto copy = [&](void *dst, const void *src) {
+        return wrach::launch_copy32(static_cast<uint32_t *>(dst), static_cast<const uint32_t *>(src), 2 * (size_t)n, st);
+    };
+    WRACH_HIP(wrach::launch_noalloc_init(fp, b, indices, st));
+    if (!aligned) {
+        WRACH_HIP(copy(b.pos, pos_xy));
+        WRACH_HIP(copy(b.vel, vel_xy));
+    }
+    WRACH_HIP(wrach::launch_collide(fp, in, st));
+    WRACH_HIP(wrach::launch_cells(fp, in, st));
+    WRACH_HIP(wrach::launch_scan(fp, b, st));
+    WRACH_HIP(wrach::launch_scatter(fp, b, st));
+    WRACH_HIP(wrach::launch_canonical(fp, out, indices, st));
+    if (!aligned) {
+        WRACH_HIP(copy(pos_xy, b.pos_out));
+        WRACH_HIP(copy(vel_xy, b.vel_out));
     }
     return WRACH_OK;
 }

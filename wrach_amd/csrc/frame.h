@@ -188,14 +188,17 @@ hipError_t launch_scatter(const FrameParams &p, const FrameBuffers &b, hipStream
 hipError_t launch_canonical(const FrameParams &p, const FrameBuffers &b, uint32_t *idx_out, hipStream_t stream);
 // Fills the idx entries of chunks the last scan found empty (before a readback).
 hipError_t launch_materialize(const FrameParams &p, const FrameBuffers &b, hipStream_t stream);
+// Before a frame on a caller's packed triple in buffers that hold anything:
+// what must be clean cleared, src and key from the caller's offsets.
+hipError_t launch_noalloc_init(const FrameParams &p, const FrameBuffers &b, const uint32_t *indices,
+                               hipStream_t stream);
 hipError_t launch_iota(uint32_t *dst, uint32_t n, hipStream_t stream);
 // key[i] = the cell whose range [idx[c + 1], idx[c + 2]) holds packed
 // particle i, for offsets given whole (an upload from the host, a
 // checkpoint): a binary search per particle.
 hipError_t launch_keys_from_offsets(const uint32_t *idx, uint32_t ncell, uint32_t n, uint32_t *key,
                                     hipStream_t stream);
-// n words of v / of src (kernels, so that a captured stream records no memset).
-hipError_t launch_fill32(uint32_t *dst, uint32_t v, size_t n, hipStream_t stream);
+// n words of src (a kernel, for a captured stream).
 hipError_t launch_copy32(uint32_t *dst, const uint32_t *src, size_t n, hipStream_t stream);
 
 constexpr uint32_t kOutsideStripes = 16;
