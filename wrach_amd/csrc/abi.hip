@@ -120,8 +120,6 @@ struct wrach_ctx {
     uint4 *srows = nullptr;   // each lane's rows and particle (capacity entries)
     uint2 *srows2 = nullptr;
     uint32_t *sperm = nullptr;   // the separation kernels' lane order (capacity entries)
-    uint32_t *scrowd = nullptr;  // the frame's crowded cells (crowd_cap entries)
-    uint32_t crowd_cap = 0;
     uint32_t *err_host = nullptr;  // pinned copy of buf.error, read at each synchronisation
     // The learned warm start (wrach_learn_*, WRACH_SOLVER_L): the network's
     // master parameters, gradient and Adam moments (f32, wrach::kParams
@@ -179,8 +177,7 @@ int settle(wrach_ctx *c) {
         if (rc_ != WRACH_OK) return rc_; \
     } while (0)
 
-// The separation kernels' buffers; the lane order when both of its
-// buffers are there.
+// The separation kernels' buffers.
 wrach::StencilArgs stencil_args(const wrach_ctx *c) {
     wrach::StencilArgs a{};
     a.cell = c->scell;
@@ -188,11 +185,7 @@ wrach::StencilArgs stencil_args(const wrach_ctx *c) {
     a.sums = c->ssums;
     a.rows = c->srows;
     a.rows2 = c->srows2;
-    if (c->sperm && c->scrowd) {
-        a.perm = c->sperm;
-        a.crowd = c->scrowd;
-        a.crowd_cap = c->crowd_cap;
-    }
+    a.perm = c->sperm;
     return a;
 }
 
@@ -206,7 +199,7 @@ int enqueue_stencil(wrach_ctx *c) {
     if (c->solver != WRACH_SOLVER_S || c->passes == 0 || c->fp.n == 0) return WRACH_OK;
     wrach::StencilArgs a = stencil_args(c);
     a.tol = c->overlap_tol;
-    WRACH_HIP(wrach::launch_stencil_clear(c->fp, c->buf, a, c->buf.pos, c->stream));
+    WRACH_HIP(wrach::launch_stencil_begin(c->fp, c->buf, a, c->buf.pos, c->stream));
     const uint32_t passes = c->passes;
     // With a tolerance, the start of every pass is measured before it (the
     // pass runs only above the tolerance).  With tolerance 0 a pass over no
@@ -270,7 +263,7 @@ int enqueue_learned(wrach_ctx *c) {
     const uint32_t k = c->passes;
     float2 *X = c->buf.pos, *Y = c->buf.pos_out, *Z = c->lbuf;
     wrach::StencilArgs a = stencil_args(c);
-    WRACH_HIP(wrach::launch_stencil_clear(c->fp, c->buf, a, X, c->stream));
+    WRACH_HIP(wrach::launch_stencil_begin(c->fp, c->buf, a, X, c->stream));
     wrach::FeatureArgs f{};
     f.pos = X;
     f.vel = c->buf.vel;
@@ -398,7 +391,6 @@ void release(wrach_ctx *c) {
     (void)hipFree(c->srows);
     (void)hipFree(c->srows2);
     (void)hipFree(c->sperm);
-    (void)hipFree(c->scrowd);
     for (void *q : {(void *)c->lparams, (void *)c->lgrad, (void *)c->lm, (void *)c->lv, (void *)c->lw3,
                     (void *)c->lfrag, (void *)c->lfeat, (void *)c->lbuf, (void *)c->tfeat,
                     (void *)c->ttarget, (void *)c->tsel, (void *)c->txt, (void *)c->ta1t,
@@ -1074,14 +1066,6 @@ int ensure_stencil(wrach_ctx *c) {
         uint32_t *perm = nullptr;
         WRACH_HIP(dmalloc(&perm, c->capacity ? c->capacity : 1));
         c->sperm = perm;
-    }
-    if (!c->scrowd) {
-        // A crowded cell holds at least kCrowdMin particles.
-        const uint32_t cap = c->capacity / wrach::kCrowdMin + 1;
-        uint32_t *crowd = nullptr;
-        WRACH_HIP(dmalloc(&crowd, cap));
-        c->scrowd = crowd;
-        c->crowd_cap = cap;
     }
     return WRACH_OK;
 }
@@ -2054,7 +2038,7 @@ int wrach_learn_sample(wrach_ctx *c, uint32_t target_passes, uint64_t *rows_tota
         // The plain passes from the state, which stays as it is: pos ->
         // pos_out -> lbuf -> pos_out ...
         wrach::StencilArgs a = stencil_args(c);
-        WRACH_HIP(wrach::launch_stencil_clear(c->fp, c->buf, a, c->buf.pos, c->stream));
+        WRACH_HIP(wrach::launch_stencil_begin(c->fp, c->buf, a, c->buf.pos, c->stream));
         a.rows_from = wrach::kRowsOfCell;
         a.record = c->srows && target_passes > 1 ? 1 : 0;
         const float2 *in = c->buf.pos;

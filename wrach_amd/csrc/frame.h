@@ -237,7 +237,7 @@ hipError_t launch_upload_scatter(const UploadParams &u, const FrameBuffers &b, h
 // largest overlap (float bits) after 0..max_passes passes for the last
 // frame; the passes that ran are those whose start exceeded the tolerance.
 constexpr uint32_t kMaxStencilPasses = 64;
-constexpr uint32_t kStencilWords = kMaxStencilPasses + 4;
+constexpr uint32_t kStencilWords = kMaxStencilPasses + 3;
 // The words lie in kWordStripes copies on cache lines of their own: block b
 // raises the overlap words of stripe b % kWordStripes (the largest over the
 // stripes counts), the words that are no overlaps are stripe 0's.
@@ -260,13 +260,11 @@ constexpr uint32_t kStencilSumEntries = kStencilSumSets * kStencilSumSlots * kSt
 // frame-start positions (the warm start left more mean overlap than it
 // found), else 0.
 constexpr uint32_t kFallbackWord = kMaxStencilPasses + 1;
-// words[kCrowdCountWord]: the crowded cells listed for the frame.
-constexpr uint32_t kCrowdCountWord = kMaxStencilPasses + 2;
 // words[kOverBudgetWord]: nonzero once a stencil kernel of the frame has met
 // a particle whose 3x3 cells hold more than kStencilBudget particles (the
 // cells are the frame start's, so the frame's first pass or measure finds
 // every such particle).
-constexpr uint32_t kOverBudgetWord = kMaxStencilPasses + 3;
+constexpr uint32_t kOverBudgetWord = kMaxStencilPasses + 2;
 constexpr float kOverlapScale = 16777216.0f;  // 2^24
 // Crowded cells (kCrowdMin..kCrowdMax particles): the separation kernels'
 // lanes take their particles in order of x (the lane order; the results
@@ -300,12 +298,8 @@ struct StencilArgs {
     // block 0 records the choice in words[kFallbackWord].
     const float2 *pin_alt;
     // The lane order (null: lane t takes particle t): lane t takes particle
-    // perm[t], a permutation that orders each crowded cell by x; the
-    // crowded cells of the frame (words[kCrowdCountWord] of them, at most
-    // crowd_cap).
+    // perm[t], a permutation that orders each crowded cell by x.
     uint32_t *perm;
-    uint32_t *crowd;
-    uint32_t crowd_cap;
     // A measure after a pass or measure of the frame: each pair from one
     // side only (the particle's own cell past it, the cell to its right and
     // the three cells above), the pair count and overlap sum doubled, unless
@@ -319,7 +313,7 @@ hipError_t launch_stencil_move(const FrameParams &p, const FrameBuffers &b, cons
                                hipStream_t stream);
 // The frame's first stencil launch: clears the overlap words and sums and,
 // with a.perm, orders the lanes of the crowded cells by the x of `pos`.
-hipError_t launch_stencil_clear(const FrameParams &p, const FrameBuffers &b, const StencilArgs &a,
+hipError_t launch_stencil_begin(const FrameParams &p, const FrameBuffers &b, const StencilArgs &a,
                                 const float2 *pos, hipStream_t stream);
 hipError_t launch_copy_pos(float2 *dst, const float2 *src, uint32_t n, hipStream_t stream);
 // Adds to out[0..3] (zeroed by the caller) the mismatches of the pair
