@@ -393,3 +393,29 @@ def test_stencil_rows_at_the_edges_of_the_short_path(oracle, row, n):
     cfg = WrachConfig(dimensions=(64, 32), cell_size=1)
     run_stencil(oracle, cfg, pos, vel, 3, 3, every=1, label=f"rows of {row}")
     run_stencil(oracle, cfg, pos, vel, 2, 3, tol=0.3, every=1, label=f"rows of {row}, tolerance", graph=False)
+
+
+@pytest.mark.parametrize("passes", [1, 2, 3, 4, 5, 8, 9])
+@pytest.mark.parametrize("quiet", [False, True])
+def test_stencil_tolerance_at_every_pass(oracle, passes, quiet):
+    """A tolerance between the overlaps at the starts of two passes, for each
+    pass it can end at (none of them, the first, .., all run): the passes that
+    run, the positions from either buffer, and the report."""
+    pos, vel = uniform(3000, 96, 128, 77)
+    cfg = WrachConfig(dimensions=(96, 128), cell_size=1, gravity=(0.0, -0.1))
+    P, ref = oracle_world(oracle, cfg, pos, vel)
+    starts = [oracle.step_s(P, *ref, max_passes=k, overlap_tol=0.0, nsteps=1)[3][1] for k in range(passes + 1)]
+    starts[0] = oracle.step_s(P, *ref, max_passes=1, overlap_tol=0.0, nsteps=1)[3][0]
+    tols = {0.999 * s for s in starts if s > 0} | {1.001 * s for s in starts if s > 0}
+    for tol in sorted(np.float32(t) for t in tols):
+        want = oracle.step_s(P, *ref, max_passes=passes, overlap_tol=float(tol), nsteps=1)
+        with World(cfg) as w:
+            w.add_particles(pos, vel)
+            w.set_solver("S", passes, float(tol), quiet=quiet)
+            w.step(1)
+            assert_same_state(w.read(), tuple(want[:3]), f"passes={passes} tol={tol}")
+            got = w.solver_stats()
+            st = want[3]
+            assert got[0] == st[0] and got[2] == st[2] and got[3][:2] == st[3][:2], f"{got} against {st}"
+            if not quiet:
+                assert got == st, f"{got} against {st}"

@@ -194,50 +194,42 @@ uint32_t later_rows(const wrach_ctx *c) { return c->srows ? wrach::kRowsRecorded
 
 // Mode S's passes: P0 = pos; pass k reads pos or pos_out (k even or odd)
 // and writes the other (pos_out is free until the collide kernel writes
-// it); an odd count leaves the result in pos_out and a copy brings it back.
+// it).  The closing measure, or a copy in its place, brings the result back
+// to pos.
 int enqueue_stencil(wrach_ctx *c) {
     if (c->solver != WRACH_SOLVER_S || c->passes == 0 || c->fp.n == 0) return WRACH_OK;
     wrach::StencilArgs a = stencil_args(c);
     a.tol = c->overlap_tol;
     WRACH_HIP(wrach::launch_stencil_begin(c->fp, c->buf, a, c->buf.pos, c->stream));
     const uint32_t passes = c->passes;
-    // With a tolerance, the start of every pass is measured before it (the
-    // pass runs only above the tolerance).  With tolerance 0 a pass over no
-    // overlap moves nothing, so each pass measures its own start and only
-    // the end has a measure of its own.
+    // With a tolerance a pass may be one too many; the passes after it stay
+    // away and the end takes the positions from where they ended.
     const bool check = c->overlap_tol > 0.0f;
     a.rows_from = wrach::kRowsOfPosition;  // the frame's first kernel derives the rows
-    a.record = c->srows && (check || passes > 1 || !c->quiet) ? 1 : 0;
-    if (check) {
-        a.pin = c->buf.pos;
-        a.in_slot = 0;
-        a.stat = 1;  // the overlap sums before the passes
-        WRACH_HIP(wrach::launch_stencil_measure(c->fp, c->buf, a, c->stream));
-        a.rows_from = later_rows(c);
-        a.record = 0;
-    }
+    a.record = c->srows && (passes > 1 || !c->quiet) ? 1 : 0;
     for (uint32_t k = 0; k < passes; ++k) {
-        float2 *in = k % 2 == 0 ? c->buf.pos : c->buf.pos_out;
-        float2 *out = k % 2 == 0 ? c->buf.pos_out : c->buf.pos;
-        a.pin = in;
-        a.pout = out;
+        a.pin = k % 2 == 0 ? c->buf.pos : c->buf.pos_out;
+        a.pout = k % 2 == 0 ? c->buf.pos_out : c->buf.pos;
         a.in_slot = k;
-        a.check = check ? 1 : 0;
-        a.stat = !check && k == 0 ? 1 : 0;
+        a.check = check && k > 0 ? 1 : 0;
+        a.stat = k == 0 ? 1 : 0;  // the overlap sums before the passes
         WRACH_HIP(wrach::launch_stencil_move(c->fp, c->buf, a, c->stream));
         a.rows_from = later_rows(c);
         a.record = 0;
-        if (check ? (k + 1 < passes || !c->quiet) : (k + 1 == passes && !c->quiet)) {
-            a.pin = out;
-            a.in_slot = k + 1;
-            a.check = 0;
-            a.stat = k + 1 == passes ? 2 : 0;  // the last measure: the sums after the passes
-            a.half = 1;  // the frame's first kernel has run: each pair from one side
-            WRACH_HIP(wrach::launch_stencil_measure(c->fp, c->buf, a, c->stream));
-            a.half = 0;
-        }
     }
-    if (passes % 2) WRACH_HIP(wrach::launch_copy_pos(c->buf.pos, c->buf.pos_out, c->fp.n, c->stream));
+    a.pin = !check && passes % 2 ? c->buf.pos_out : c->buf.pos;
+    a.pin_odd = check ? c->buf.pos_out : nullptr;
+    a.select = check ? passes : 0;
+    a.pout = c->buf.pos;
+    if (c->quiet) {
+        WRACH_HIP(wrach::launch_stencil_end(c->fp, a, c->stream));
+        return WRACH_OK;
+    }
+    a.in_slot = passes;
+    a.check = 0;
+    a.stat = 2;  // the sums after the passes
+    a.half = 1;  // the frame's first kernel has run: each pair from one side
+    WRACH_HIP(wrach::launch_stencil_measure(c->fp, c->buf, a, c->stream));
     return WRACH_OK;
 }
 
@@ -313,10 +305,11 @@ int enqueue_learned(wrach_ctx *c) {
         a.rows_from = later_rows(c);
         a.record = 0;
     }
-    if (cur != X) WRACH_HIP(wrach::launch_copy_pos(X, cur, c->fp.n, c->stream));
-    if (!c->quiet) {
-        a.pin = X;
-        a.pout = nullptr;
+    a.pin = cur;
+    a.pout = X;
+    if (c->quiet) {
+        WRACH_HIP(wrach::launch_stencil_end(c->fp, a, c->stream));
+    } else {
         a.in_slot = k;
         a.stat = 2;  // set 1: after the passes
         a.pin_alt = nullptr;

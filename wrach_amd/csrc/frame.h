@@ -275,12 +275,12 @@ constexpr uint32_t kCrowdMax = 1024;
 constexpr uint32_t kRowsRecorded = 0, kRowsOfPosition = 1, kRowsOfCell = 2;
 struct StencilArgs {
     const float2 *pin;  // positions entering the kernel
-    float2 *pout;       // a move's output
+    float2 *pout;       // a move's output (a measure's: see pin_odd)
     uint32_t *cell;     // each particle's cell at the frame's start (kRowsOfCell)
     uint32_t *words;    // kWordEntries words
     unsigned long long *sums;  // kStencilSumEntries entries
     uint32_t stat;      // a measure: 0, or 1 / 2 to add its overlaps to the first / last sums
-    uint32_t in_slot;   // a measure: the word it raises; a move: the word of its start
+    uint32_t in_slot;   // the word a measure or move raises to the overlap of its input
     // A lane's particle and the rows of its 3x3 cells: kRowsOfPosition, the
     // frame's first kernel derives them from its input; kRowsOfCell, from
     // `cell`; kRowsRecorded, a kernel of the frame has recorded them (24
@@ -290,8 +290,13 @@ struct StencilArgs {
     uint32_t record;
     uint4 *rows;
     uint2 *rows2;
-    uint32_t check;     // a move: skip (copy) when the measured start is within tol
-    float tol;          // a move runs while the overlap at its start exceeds this
+    uint32_t check;     // a move: stay away once the passes have ended (words[in_slot - 1] within tol)
+    float tol;          // the passes run while the overlap at their start exceeds this
+    // A measure, or the frame's end: the positions are pin, or with pin_odd
+    // where `select` passes between pin and pin_odd ended; pout (if not
+    // null): they are brought there.
+    const float2 *pin_odd;
+    uint32_t select;
     // A move after a learned warm start (else null): it reads pin_alt (the
     // frame-start positions) instead of pin when the mean overlap of the
     // warm start (sums set 2) exceeds that of the frame start (set 0), and
@@ -315,7 +320,9 @@ hipError_t launch_stencil_move(const FrameParams &p, const FrameBuffers &b, cons
 // with a.perm, orders the lanes of the crowded cells by the x of `pos`.
 hipError_t launch_stencil_begin(const FrameParams &p, const FrameBuffers &b, const StencilArgs &a,
                                 const float2 *pos, hipStream_t stream);
-hipError_t launch_copy_pos(float2 *dst, const float2 *src, uint32_t n, hipStream_t stream);
+// The frame's last stencil launch where nothing is measured: brings the
+// positions to a.pout.
+hipError_t launch_stencil_end(const FrameParams &p, const StencilArgs &a, hipStream_t stream);
 // Adds to out[0..3] (zeroed by the caller) the mismatches of the pair
 // arithmetic's short root and force sequences against the correctly
 // rounded ones over their whole input ranges, and the inputs tried.

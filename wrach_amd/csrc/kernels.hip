@@ -2389,14 +2389,43 @@ __device__ __forceinline__ bool warm_rejected(const StencilArgs &a) {
     return s_rej != 0;
 }
 
+// Whether the largest overlap recorded in word `slot` exceeds tol (overlaps
+// lie in [0, 1]: the stripes' bits order as the floats).
+__device__ __forceinline__ bool overlap_above(const uint32_t *words, uint32_t slot, float tol) {
+    const uint32_t v = words[(lane_id() % kWordStripes) * kWordStride + slot];
+    return __ballot(__uint_as_float(v) > tol) != 0;
+}
+
+// Where the positions are after passes that stop at the tolerance: pass k
+// went from a.pin to a.pin_odd for even k and back for odd k, and the first
+// whose start did not exceed the tolerance, if any, ended them (its output
+// does not count).  The whole grid decides alike from the words.
+__device__ __forceinline__ bool passes_end_odd(const StencilArgs &a) {
+    static_assert(kWordStripes == 16, "four words' stripes a wavefront");
+    uint32_t k = 0;
+    for (bool on = true; on && k < a.select;) {
+        const uint32_t v = a.words[(lane_id() & 15) * kWordStride + k + (lane_id() >> 4)];
+        unsigned long long above = __ballot(__uint_as_float(v) > a.tol);
+        for (int u = 0; u < 4 && on && k < a.select; ++u, above >>= 16) {
+            on = (above & 0xffffull) != 0;
+            k += on ? 1u : 0u;
+        }
+    }
+    return (k & 1u) != 0;
+}
+
 // The largest overlap at positions a.pin, raised into a.words[a.in_slot]
-// (non-negative floats order as their bits).
+// (non-negative floats order as their bits).  With a.pin_odd the positions
+// are where the frame's a.select passes ended; with a.pout they are brought
+// there.
 __global__ __launch_bounds__(256, 8) void stencil_measure_kernel(FrameParams p, FrameBuffers b,
                                                               StencilArgs a) {
     __shared__ float2 s_list[kHitList * 256];
+    if (a.pin_odd && passes_end_odd(a)) a.pin = a.pin_odd;
     uint32_t i;
     float2 q;
     const StencilRows r = stencil_lane(p, b, a, i, q);
+    if (a.pout && a.pout != a.pin && i < p.n) a.pout[i] = q;
     const bool half = a.half && a.words[kOverBudgetWord] == 0;  // the whole grid alike
     float2 *list = s_list + threadIdx.x;
     const PairSums s = half ? (a.stat ? stencil_particle<false, true, true>(a.pin, i, q.x, q.y, r, list)
@@ -2406,27 +2435,26 @@ __global__ __launch_bounds__(256, 8) void stencil_measure_kernel(FrameParams p, 
     block_report(a.words, a.in_slot, s, stencil_sums(a), half ? 2ull : 1ull);
 }
 
-// Whether the largest overlap recorded in word `slot` exceeds tol (overlaps
-// lie in [0, 1]: the stripes' bits order as the floats).
-__device__ __forceinline__ bool overlap_above(const uint32_t *words, uint32_t slot, float tol) {
-    const uint32_t v = words[(lane_id() % kWordStripes) * kWordStride + slot];
-    return __ballot(__uint_as_float(v) > tol) != 0;
+// The same without the measure.
+__global__ __launch_bounds__(256) void stencil_end_kernel(FrameParams p, StencilArgs a) {
+    if (a.pin_odd && passes_end_odd(a)) a.pin = a.pin_odd;
+    if (a.pout == a.pin) return;
+    const uint32_t i = blockIdx.x * 256 + threadIdx.x;
+    if (i < p.n) a.pout[i] = a.pin[i];
 }
 
-// One pass: a.pin -> a.pout.  With a.check it runs only while the
-// overlap at its start (a.words[a.in_slot], measured before, the same for
-// the whole grid) exceeds the tolerance, and is a copy otherwise.  Either
-// way it raises a.words[a.in_slot] to the largest overlap of its input, so
-// that a frame without a check (tolerance 0, where a pass over no overlap
-// moves nothing) needs no measure between passes.
+// One pass: a.pin -> a.pout, raising a.words[a.in_slot] to the largest
+// overlap of its input.  A pass over no overlap moves nothing, so passes
+// without a tolerance need no test.  With a.check the pass runs only while
+// the overlap at the start of the pass before it exceeded the tolerance:
+// that pass need not have run where its start did not, so the passes end at
+// its start, which this one leaves alone (it would overwrite it), raising no
+// overlap, so that every later pass stays away as well.  One pass too many
+// costs less than a measure before each.
 __global__ __launch_bounds__(256, 7) void stencil_move_kernel(FrameParams p, FrameBuffers b,
                                                            StencilArgs a) {
     __shared__ float2 s_list[kHitList * 256];
-    if (a.check && !overlap_above(a.words, a.in_slot, a.tol)) {
-        const uint32_t t = blockIdx.x * 256 + threadIdx.x;
-        if (t < p.n) a.pout[t] = a.pin[t];
-        return;  // the whole grid: no barrier follows
-    }
+    if (a.check && !overlap_above(a.words, a.in_slot - 1, a.tol)) return;  // the whole grid
     if (a.pin_alt) {
         const bool rej = warm_rejected(a);
         if (blockIdx.x == 0 && threadIdx.x == 0) a.words[kFallbackWord] = rej ? 1u : 0u;
@@ -2449,11 +2477,6 @@ __global__ __launch_bounds__(256, 7) void stencil_move_kernel(FrameParams p, Fra
         dy = dy / (float)s.pairs;
     }
     a.pout[i] = make_float2(q.x + dx, q.y + dy);
-}
-
-__global__ __launch_bounds__(256) void copy_pos_kernel(float2 *dst, const float2 *src, uint32_t n) {
-    const uint32_t i = blockIdx.x * 256 + threadIdx.x;
-    if (i < n) dst[i] = src[i];
 }
 
 // The frame's first stencil launch: clears the overlap words and sums, and
@@ -2958,6 +2981,12 @@ hipError_t launch_stencil_measure(const FrameParams &p, const FrameBuffers &b, c
     return hipGetLastError();
 }
 
+hipError_t launch_stencil_end(const FrameParams &p, const StencilArgs &a, hipStream_t stream) {
+    if (p.n == 0 || (!a.pin_odd && a.pin == a.pout)) return hipSuccess;
+    hipLaunchKernelGGL(stencil_end_kernel, dim3((p.n + 255) / 256), dim3(256), 0, stream, p, a);
+    return hipGetLastError();
+}
+
 hipError_t launch_stencil_move(const FrameParams &p, const FrameBuffers &b, const StencilArgs &a,
                                hipStream_t stream) {
     if (p.n == 0) return hipSuccess;
@@ -2981,12 +3010,6 @@ hipError_t launch_stencil_begin(const FrameParams &p, const FrameBuffers &b, con
 
 hipError_t launch_check_pair_arithmetic(unsigned long long *out, hipStream_t stream) {
     hipLaunchKernelGGL(check_pair_arithmetic_kernel, dim3(4096), dim3(256), 0, stream, out);
-    return hipGetLastError();
-}
-
-hipError_t launch_copy_pos(float2 *dst, const float2 *src, uint32_t n, hipStream_t stream) {
-    if (n == 0) return hipSuccess;
-    hipLaunchKernelGGL(copy_pos_kernel, dim3((n + 255) / 256), dim3(256), 0, stream, dst, src, n);
     return hipGetLastError();
 }
 
