@@ -312,3 +312,32 @@ def test_training_beats_the_untrained_network(oracle):
         say(f"[learn] passes to reach 8 plain passes' mean overlap {target:.4f}: {need}")
         assert need["trained"] is not None
         assert need["untrained"] is None or need["trained"] < need["untrained"]
+
+
+@pytest.mark.parametrize("crowd", [1, 9, 31, 33, 60, 127, 129, 300])
+@pytest.mark.parametrize("n", [63, 257])
+def test_features_of_crowds(oracle, crowd, n):
+    """Feature rows where the gather changes its path: fewer and more than 32
+    and 128 candidates in the 5x5 cells, exact ties of distance among them (a
+    mirrored crowd, coincident copies), particles in the world's corners, and
+    a last block and wavefront of few lanes; cell sizes 1 and 3."""
+    rng = np.random.default_rng(1000 * n + crowd)
+    for cs in (1, 3):
+        side = 40 * cs
+        centre = np.array([20.5, 20.5]) * cs
+        half = rng.uniform(0, cs, (crowd // 2, 2))
+        group = np.concatenate([centre + half, centre - half, centre[None] + 0.25 * cs, centre[None] + 0.25 * cs])
+        rest = rng.uniform(0, side, (n, 2))
+        corners = np.array([[0, 0], [side, 0], [0, side], [side, side], [0.5, side - 0.5]])
+        pos = np.round(np.concatenate([group, rest, corners]) * 64) / 64  # a grid of positions: more ties
+        pos = pos.astype(np.float32)
+        vel = rng.uniform(-1, 1, pos.shape).astype(np.float32)
+        cfg = WrachConfig(dimensions=(side, side), cell_size=cs)
+        with World(cfg) as w:
+            w.add_particles(pos, vel)
+            rows, sums = w.learn_features()
+            idx, p, v = w.read()
+        ref_rows, ref_sums = ol.features(oracle.params(side, side, cs, len(p)), idx, p, v)
+        bad = np.flatnonzero((rows != ref_rows).any(axis=1))
+        assert bad.size == 0, f"crowd={crowd} n={n} cs={cs}: {bad.size} rows differ, first {bad[:5]}"
+        assert sums == ref_sums, f"crowd={crowd} n={n} cs={cs}"

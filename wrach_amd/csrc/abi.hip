@@ -130,6 +130,7 @@ struct wrach_ctx {
     uint32_t adam_t = 0;
     uint16_t *lfeat = nullptr;
     float2 *lbuf = nullptr;
+    float4 *lstate = nullptr;  // the features' (position, velocity) pairs
     // Training set (rows of features and target displacements) and the
     // workspace of one batch.
     uint16_t *tfeat = nullptr;
@@ -241,9 +242,18 @@ wrach::MlpWeights mlp_weights(const wrach_ctx *c) {
     return w;
 }
 
+// The features leave what the passes after them need.
+void learned_rows(const wrach_ctx *c, wrach::FeatureArgs &f) {
+    f.perm = c->sperm;
+    f.rows = c->srows;
+    f.rows2 = c->srows2;
+    f.cell = c->scell;
+    f.words = c->swords;
+}
+
 // The learned frame (WRACH_SOLVER_L), before the reference step.  With X =
 // pos (the frame start), Y = pos_out and Z = lbuf:
-//   features of X (and each particle's cell, and X's overlap sums, set 0);
+//   features of X (and each lane's rows, and X's overlap sums, set 0);
 //   the network's warm start X -> Y;
 //   pass 1 Y -> Z (its input's sums: set 2);
 //   pass 2 Z -> Y, reading X instead of Z when the warm start left more mean
@@ -260,8 +270,9 @@ int enqueue_learned(wrach_ctx *c) {
     f.pos = X;
     f.vel = c->buf.vel;
     f.feat = c->lfeat;
+    f.state = c->lstate;
     f.row0 = 0;
-    f.cell = c->scell;
+    learned_rows(c, f);
     f.sums = c->ssums;  // set 0: the frame start
     WRACH_HIP(wrach::launch_learn_features(c->fp, c->buf, f, c->stream));
     wrach::InferArgs in{};
@@ -292,8 +303,7 @@ int enqueue_learned(wrach_ctx *c) {
         }
     }
     a.tol = 0.0f;
-    a.rows_from = wrach::kRowsOfCell;  // the cells came from the features
-    a.record = c->srows ? 1 : 0;
+    a.rows_from = later_rows(c);  // the rows came with the features
     for (uint32_t j = 0; j < plan.size(); ++j) {
         a.pin = plan[j].first;
         a.pout = plan[j].second;
@@ -302,8 +312,6 @@ int enqueue_learned(wrach_ctx *c) {
         a.stat = j == 0 ? 3 : 0;  // set 2: the warm start
         a.pin_alt = j == 1 ? X : nullptr;
         WRACH_HIP(wrach::launch_stencil_move(c->fp, c->buf, a, c->stream));
-        a.rows_from = later_rows(c);
-        a.record = 0;
     }
     a.pin = cur;
     a.pout = X;
@@ -385,7 +393,7 @@ void release(wrach_ctx *c) {
     (void)hipFree(c->srows2);
     (void)hipFree(c->sperm);
     for (void *q : {(void *)c->lparams, (void *)c->lgrad, (void *)c->lm, (void *)c->lv, (void *)c->lw3,
-                    (void *)c->lfrag, (void *)c->lfeat, (void *)c->lbuf, (void *)c->tfeat,
+                    (void *)c->lfrag, (void *)c->lfeat, (void *)c->lbuf, (void *)c->lstate, (void *)c->tfeat,
                     (void *)c->ttarget, (void *)c->tsel, (void *)c->txt, (void *)c->ta1t,
                     (void *)c->tdz1t, (void *)c->tdz2t, (void *)c->ta2t, (void *)c->tdyt, (void *)c->tsq,
                     (void *)c->tpart, (void *)c->tcols, (void *)c->tloss})
@@ -1075,6 +1083,14 @@ int ensure_learned_frame(wrach_ctx *c) {
         float2 *b = nullptr;
         WRACH_HIP(dmalloc(&b, rows));
         c->lbuf = b;
+    }
+    if (!c->lstate) {
+        float4 *b = nullptr;
+        if (dmalloc(&b, rows) != hipSuccess) {  // no room: the gathers take two loads
+            (void)hipGetLastError();
+            b = nullptr;
+        }
+        c->lstate = b;
     }
     return WRACH_OK;
 }
@@ -1890,6 +1906,7 @@ int wrach_learn_features(wrach_ctx *c, uint16_t *rows, size_t rows_cap, uint64_t
     f.pos = reinterpret_cast<const float2 *>(v.positions);
     f.vel = reinterpret_cast<const float2 *>(v.velocities);
     f.feat = c->lfeat;
+    f.state = c->lstate;
     f.sums = sums.p;
     WRACH_HIP(wrach::launch_learn_features(c->fp, c->buf, f, c->stream));
     if (rows && n)
@@ -2025,15 +2042,15 @@ int wrach_learn_sample(wrach_ctx *c, uint32_t target_passes, uint64_t *rows_tota
         f.pos = c->buf.pos;
         f.vel = c->buf.vel;
         f.feat = c->tfeat;
+        f.state = c->lstate;
         f.row0 = (uint32_t)c->trows;
-        f.cell = c->scell;
+        learned_rows(c, f);
+        wrach::StencilArgs a = stencil_args(c);
+        WRACH_HIP(wrach::launch_stencil_begin(c->fp, c->buf, a, c->buf.pos, c->stream));
         WRACH_HIP(wrach::launch_learn_features(c->fp, c->buf, f, c->stream));
         // The plain passes from the state, which stays as it is: pos ->
         // pos_out -> lbuf -> pos_out ...
-        wrach::StencilArgs a = stencil_args(c);
-        WRACH_HIP(wrach::launch_stencil_begin(c->fp, c->buf, a, c->buf.pos, c->stream));
-        a.rows_from = wrach::kRowsOfCell;
-        a.record = c->srows && target_passes > 1 ? 1 : 0;
+        a.rows_from = later_rows(c);
         const float2 *in = c->buf.pos;
         for (uint32_t k = 0; k < target_passes; ++k) {
             float2 *out = k % 2 == 0 ? c->buf.pos_out : c->lbuf;
@@ -2041,8 +2058,6 @@ int wrach_learn_sample(wrach_ctx *c, uint32_t target_passes, uint64_t *rows_tota
             a.pout = out;
             a.in_slot = k;
             WRACH_HIP(wrach::launch_stencil_move(c->fp, c->buf, a, c->stream));
-            a.rows_from = later_rows(c);
-            a.record = 0;
             in = out;
         }
         WRACH_HIP(wrach::launch_learn_target(in, c->buf.pos, c->ttarget, (uint32_t)c->trows, n, c->stream));
@@ -2119,6 +2134,7 @@ int wrach_learn_profile(wrach_ctx *c, uint32_t reps, double *ms) {
     f.pos = c->buf.pos;
     f.vel = c->buf.vel;
     f.feat = c->lfeat;
+    f.state = c->lstate;
     wrach::InferArgs in{};
     in.feat = c->lfeat;
     in.n = c->fp.n;

@@ -2192,6 +2192,7 @@ __device__ __forceinline__ void stencil_long(const float2 *pin, uint32_t i, floa
                                              const uint32_t (&rs)[3], const uint32_t (&re)[3],
                                              double &ax, double &ay, double &osum, uint32_t &worst,
                                              uint32_t &pairs) {
+#pragma unroll
     for (int t = HALF ? 1 : 0; t < 3; ++t) {
         uint32_t j = rs[t];
         const uint32_t e = re[t];
@@ -2303,7 +2304,7 @@ __device__ __forceinline__ void block_report(uint32_t *words, uint32_t slot, con
     __syncthreads();
     if (threadIdx.x == 0) {
         const uint32_t m = max(max(s_max[0], s_max[1]), max(s_max[2], s_max[3]));
-        if (m) atomicMax(&words[(blockIdx.x % kWordStripes) * kWordStride + slot], m);
+        if (words && m) atomicMax(&words[(blockIdx.x % kWordStripes) * kWordStride + slot], m);
         const unsigned long long n = (unsigned long long)s_cnt[0] + s_cnt[1] + s_cnt[2] + s_cnt[3];
         if (sums && n) {
             unsigned long long *to = sums + (blockIdx.x % kStencilSumSlots) * kStencilSumStride;
@@ -2505,6 +2506,15 @@ __device__ __forceinline__ float wave_min(float v) {
     return v;
 }
 
+// Positions and velocities side by side, for the features' gathers.
+__global__ __launch_bounds__(256) void learn_state_kernel(const float2 *pos, const float2 *vel, float4 *state,
+                                                          uint32_t n) {
+    const uint32_t i = blockIdx.x * 256 + threadIdx.x;
+    if (i >= n) return;
+    const float2 q = pos[i], v = vel[i];
+    state[i] = make_float4(q.x, q.y, v.x, v.y);
+}
+
 __global__ __launch_bounds__(256) void stencil_begin_kernel(FrameParams p, FrameBuffers b, StencilArgs a,
                                                             const float2 *pos) {
     __shared__ uint32_t slice_count[4][kOrderSlices];
@@ -2607,8 +2617,12 @@ __device__ __forceinline__ bool cand_less(const float2 *pos, const float2 *vel, 
     return false;
 }
 
-constexpr int kSortLog2 = 5;
-constexpr int kSortCands = 1 << kSortLog2;  // candidates sorted by the network
+constexpr int kSortCands = 32;  // candidates ordered by the network
+// A candidate's 32-bit key: its squared distance in fixed point above its
+// number, for the first kKeyCands candidates.
+constexpr int kNumberBits = 7;
+constexpr uint32_t kKeyCands = 1u << kNumberBits;
+constexpr uint32_t kDistMax = (1u << (32 - kNumberBits)) - 2;  // a key of all ones is no candidate
 
 // Inserts candidate c into the ascending list k[0..15] (dropping the last).
 // Squared distances are finite, so a real key's high word never equals the
@@ -2626,191 +2640,275 @@ __device__ __forceinline__ void insert16(const float2 *pos, const float2 *vel, u
     }
 }
 
-__global__ __launch_bounds__(256) void learn_features_kernel(FrameParams p, FrameBuffers b,
+// Two f32 as bf16 bits, rounded to nearest even (v_cvt_pk_bf16_f32; a NaN as
+// bf16_bits keeps it).
+__device__ __forceinline__ uint32_t bf16_pair(float x, float y) {
+    if ((x != x) | (y != y)) return (uint32_t)bf16_bits(x) | ((uint32_t)bf16_bits(y) << 16);
+    typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
+    bf16x2 v;
+    v[0] = (__bf16)x;
+    v[1] = (__bf16)y;
+    return __builtin_bit_cast(uint32_t, v);
+}
+
+__device__ __forceinline__ float squared_distance(float2 o, float2 q) {
+    const float dx = o.x - q.x;
+    const float dy = o.y - q.y;
+    float sq = dx * dx;
+    sq = sq + dy * dy;
+    return sq;
+}
+
+// A particle's position and velocity.
+__device__ __forceinline__ float4 particle_state(const FeatureArgs &a, uint32_t j) {
+    if (a.state) return a.state[j];
+    const float2 q = a.pos[j], v = a.vel[j];
+    return make_float4(q.x, q.y, v.x, v.y);
+}
+
+// Candidate u of the list over the five rows: rows 1..4 begin at c1..c4, and
+// a row's candidates lie at u + o.  (By value: a selection among array
+// elements, or a closure's, became a load from scratch memory.)
+__device__ __forceinline__ uint32_t candidate(uint32_t u, uint32_t c1, uint32_t c2, uint32_t c3, uint32_t c4,
+                                              uint32_t o0, uint32_t o1, uint32_t o2, uint32_t o3, uint32_t o4) {
+    uint32_t o = u >= c1 ? o1 : o0;
+    o = u >= c2 ? o2 : o;
+    o = u >= c3 ? o3 : o;
+    o = u >= c4 ? o4 : o;
+    return u + o;
+}
+
+// The first kSortCands candidates are ordered in registers by Batcher's
+// odd-even merge network for 32 keys, pruned to the 174 comparators that
+// decide the first 17 places (select_nets.h), on 32-bit keys: the squared
+// distance in 25 bits of fixed point over the largest the 5x5 cells allow,
+// and the candidate's number; the next 96 are inserted into the best 17.  A
+// comparator is a minimum and a maximum (on the 64-bit key of distance bits
+// and packed index it was five instructions, and a wavefront inserts a few
+// past the first 32 nearly always).  The order is the exact one unless two of
+// the first 17 share the 25 bits: a wavefront where any lane finds that
+// (hundreds do not) orders its candidates again by insertion with the exact
+// comparator, as it inserts those past the first 128.
+//
+// 1M particles: 181 us and 4,222 vector instructions a wavefront before, now
+// 122 (and 6.5 for learn_state_kernel) and 2,750.  What bounds it is the L1:
+// 2,700 accesses a wavefront, most of them the 16 neighbours' gathers, one of
+// 16 bytes each since positions and velocities lie side by side (two of 8
+// before), and the candidates'; rows stored from each lane were 450 more.
+__global__ __launch_bounds__(256, 4) void learn_features_kernel(FrameParams p, FrameBuffers b,
                                                              FeatureArgs a) {
-    const uint32_t i = blockIdx.x * 256 + threadIdx.x;
-    unsigned long long osum = 0, ocnt = 0;
-    if (i < p.n) {
-        const float2 q = a.pos[i];
-        const float2 w = a.vel[i];
+    __shared__ union {
+        uint4 rows[4][64 * 4];
+        float2 list[kHitList * 256];
+    } sh;
+    const uint32_t lane = lane_id();
+    const uint32_t lane_t = blockIdx.x * 256 + threadIdx.x;
+    const bool on = lane_t < p.n;
+    uint32_t i = on ? lane_t : 0u;  // a lane past the particles reads particle 0 and writes nothing
+    if (on && a.perm) i = a.perm[lane_t];
+    const float2 q = a.pos[i], w = a.vel[i];
+    uint32_t rs[5], cum[5], m5 = 0;  // a row's first particle; candidates before its row
+    StencilRows r3;
+#pragma unroll
+    for (int t = 0; t < 3; ++t) r3.rs[t] = r3.len[t] = 0;
+    r3.half = 0;
+#pragma unroll
+    for (int t = 0; t < 5; ++t) rs[t] = cum[t] = 0;
+    if (on) {
         const Grid g = particle_grid(p, b, i);
-        const uint32_t base = g.base;
-        const uint32_t k = cell_key(p, g, q.x, q.y);
-        if (a.cell) a.cell[i] = k;
         uint32_t ucx, ucy;
+        const uint32_t k = cell_key(p, g, q.x, q.y);
         cell_coords(g, k, ucx, ucy);
         const int cx = (int)ucx, cy = (int)ucy;
         const int gx = (int)g.gx, gy = (int)g.gy;
-        const int x0 = cx > 1 ? cx - 2 : 0, x1 = cx + 2 < gx ? cx + 2 : gx - 1;
-        const int i0 = cx > 0 ? cx - 1 : 0, i1 = cx + 1 < gx ? cx + 1 : gx - 1;
-        uint32_t rs[5], re[5], is[5], ie[5];
+        // Per row of the 5x5 cells, its first cell and the one past its last;
+        // of the 3x3 cells the same, and the own cell.  Every load is issued
+        // before the first is used.
+        uint32_t c[17], at[17], live[17], pre[17];
+#pragma unroll
+        for (int t = 0; t < 5; ++t) {
+            int y = cy + t - 2;
+            y = y < 0 ? 0 : y < gy ? y : gy - 1;  // a row outside the world: loaded, not used
+            const uint32_t row = g.base + (uint32_t)(y * gx);
+            c[2 * t] = row + (uint32_t)(cx > 1 ? cx - 2 : 0);
+            c[2 * t + 1] = row + (uint32_t)(cx + 2 < gx ? cx + 3 : gx);
+            if (t >= 1 && t <= 3) {
+                c[8 + 2 * t] = row + (uint32_t)(cx > 0 ? cx - 1 : 0);
+                c[9 + 2 * t] = row + (uint32_t)(cx + 1 < gx ? cx + 2 : gx);
+            }
+        }
+        c[16] = k;
+#pragma unroll
+        for (int u = 0; u < 17; ++u) {
+            const uint32_t v = c[u] < p.ncell ? c[u] : p.ncell - 1;
+            live[u] = b.chunk_live[v >> kChunkShift];
+            pre[u] = b.chunk_prefix[v >> kChunkShift];
+            at[u] = b.idx[v + 1];
+        }
+#pragma unroll
+        for (int u = 0; u < 17; ++u) {
+            at[u] = live[u] ? at[u] : pre[u];
+            at[u] = c[u] < p.ncell && at[u] < p.n ? at[u] : p.n;
+        }
         uint64_t tot5 = 0, tot3 = 0;
+        uint32_t re1 = 0;
 #pragma unroll
         for (int t = 0; t < 5; ++t) {
             const int y = cy + t - 2;
-            rs[t] = re[t] = is[t] = ie[t] = 0;
-            if (y < 0 || y >= gy) continue;
-            const uint32_t row = base + (uint32_t)(y * gx);
-            rs[t] = cell_start(p, b, row + (uint32_t)x0);
-            re[t] = cell_start(p, b, row + (uint32_t)x1 + 1);
-            if (re[t] < rs[t]) re[t] = rs[t];
-            tot5 += re[t] - rs[t];
+            const bool in = y >= 0 && y < gy;  // the world's own rows only
+            rs[t] = in ? at[2 * t] : 0u;
+            const uint32_t re = in && at[2 * t + 1] > at[2 * t] ? at[2 * t + 1] : rs[t];
+            cum[t] = (uint32_t)tot5;
+            tot5 += re - rs[t];
             if (t >= 1 && t <= 3) {
-                is[t] = cell_start(p, b, row + (uint32_t)i0);
-                ie[t] = cell_start(p, b, row + (uint32_t)i1 + 1);
-                if (ie[t] < is[t]) ie[t] = is[t];
-                tot3 += ie[t] - is[t];
+                r3.rs[t - 1] = in ? at[8 + 2 * t] : 0u;
+                const uint32_t e3 = in && at[9 + 2 * t] > at[8 + 2 * t] ? at[9 + 2 * t] : r3.rs[t - 1];
+                r3.len[t - 1] = e3 - r3.rs[t - 1];
+                tot3 += r3.len[t - 1];
+                if (t == 2) re1 = e3;
             }
         }
-        const bool feats = tot5 <= kFeatBudget;
-        const bool sums = a.sums != nullptr && tot3 <= kStencilBudget;
-        // The overlap sums: the 3x3 cells, as a separation pass visits them.
-        if (sums) {
-#pragma unroll
-            for (int t = 1; t <= 3; ++t) {
-                for (uint32_t j = is[t]; j < ie[t]; ++j) {
-                    if (j == i) continue;
-                    const float2 o = a.pos[j];
-                    float ov, f;
-                    if (stencil_reach(q.x - o.x, q.y - o.y, true, ov, f)) {
-                        osum += (uint32_t)rintf(ov * kOverlapScale);
-                        ocnt += 1;
-                    }
-                }
-            }
+        m5 = tot5 <= kFeatBudget ? (uint32_t)tot5 : 0u;
+        const bool over = tot3 > kStencilBudget;
+        r3.half = over ? 0u : min(max(r3.rs[1], at[16]), re1) - r3.rs[1];
+        if (over) r3.len[0] = r3.len[1] = r3.len[2] = 0;
+        // What the passes that follow need (stencil_lane).
+        if (a.words && over) atomicOr(&a.words[kOverBudgetWord], 1u);
+        if (a.rows) {
+            a.rows[lane_t] = make_uint4(r3.rs[0], r3.rs[1], r3.rs[2], r3.len[0] | (r3.half << 16));
+            a.rows2[lane_t] = make_uint2(r3.len[1] | (r3.len[2] << 16), i);
+        } else if (a.cell) {
+            a.cell[i] = k;
         }
-        // The 16 nearest.  The first kSortCands candidates are ordered in
-        // registers by Batcher's odd-even merge network for 32 keys, pruned
-        // to the 174 comparators that decide the first 17 places
-        // (select_nets.h), comparing the 64-bit key (squared distance bits,
-        // packed index) as one integer.  That is the exact order unless two
-        // of the first 17 share a distance: a wavefront where any lane finds
-        // such a tie orders its keys again with the exact comparator (a
-        // bitonic network of 240 compare-exchanges over cand_less).  Any
-        // further candidates are inserted into the best 16.  (Networks for
-        // 24 and 28 keys beside it, chosen per wavefront, took 137-165
-        // VGPRs: one wavefront less per SIMD.)
-        unsigned long long key[kNbrs];
+    }
+    const uint32_t c1 = cum[1], c2 = cum[2], c3 = cum[3], c4 = cum[4];
+    const uint32_t o0 = rs[0], o1 = rs[1] - c1, o2 = rs[2] - c2, o3 = rs[3] - c3, o4 = rs[4] - c4;
+#define WRACH_CAND(u) candidate(u, c1, c2, c3, c4, o0, o1, o2, o3, o4)
+    // The 5x5 cells keep both differences below three cell sides.
+    const float to_fixed = (float)(kDistMax + 2) / (18.01f * p.cs * p.cs);
+    uint32_t ck[kSortCands];
 #pragma unroll
-        for (int r = 0; r < kNbrs; ++r) key[r] = ~0ull;
-        uint32_t cum[5], m5 = 0;
+    for (int u0 = 0; u0 < kSortCands; u0 += 8) {
+        float sq[8];
+        bool real[8];
 #pragma unroll
-        for (int t = 0; t < 5; ++t) {
-            cum[t] = m5;
-            m5 += re[t] - rs[t];
+        for (int v = 0; v < 8; ++v) {
+            const uint32_t u = (uint32_t)(u0 + v);
+            uint32_t j = WRACH_CAND(u);
+            j = u < m5 ? j : i;
+            real[v] = j != i;
+            sq[v] = squared_distance(a.pos[j], q);
         }
-        unsigned long long ck[kSortCands];
-        bool tie = false;
-        if (feats) {
 #pragma unroll
-            for (int u = 0; u < kSortCands; ++u) {
-                ck[u] = ~0ull;
-                if ((uint32_t)u < m5) {
-                    uint32_t j = 0;
-#pragma unroll
-                    for (int t = 0; t < 5; ++t)
-                        if ((uint32_t)u >= cum[t] && (uint32_t)u < cum[t] + (re[t] - rs[t]))
-                            j = rs[t] + ((uint32_t)u - cum[t]);
-                    if (j != i) {
-                        const float2 o = a.pos[j];
-                        const float dx = o.x - q.x;
-                        const float dy = o.y - q.y;
-                        float sq = dx * dx;
-                        sq = sq + dy * dy;
-                        ck[u] = ((unsigned long long)__float_as_uint(sq) << 32) | j;
-                    }
-                }
-            }
+        for (int v = 0; v < 8; ++v) {
+            // Not finite or past the largest (no layout of the frames): the
+            // largest, which two of them share.
+            const uint32_t d = (uint32_t)fminf(sq[v] * to_fixed, (float)kDistMax);
+            ck[u0 + v] = real[v] ? min(d, kDistMax) << kNumberBits | (uint32_t)(u0 + v) : 0xffffffffu;
+        }
+    }
 #define WRACH_SEL_CE(x, y)                                 \
     {                                                      \
-        const unsigned long long lo_ = ck[x], hi_ = ck[y]; \
-        const bool sw_ = hi_ < lo_;                        \
-        ck[x] = sw_ ? hi_ : lo_;                           \
-        ck[y] = sw_ ? lo_ : hi_;                           \
+        const uint32_t lo_ = min(ck[x], ck[y]);            \
+        ck[y] = max(ck[x], ck[y]);                         \
+        ck[x] = lo_;                                       \
     }
-            SEL_NET_32(WRACH_SEL_CE)
+    SEL_NET_32(WRACH_SEL_CE)
 #undef WRACH_SEL_CE
-            // Real keys never have the empty key's high word (distances are
-            // finite), so only real neighbours can tie.
+    // Two at a time, loads together, each pushed through the best 17.
+    for (uint32_t u = kSortCands; u < kKeyCands && __ballot(u < m5) != 0; u += 2) {
+        uint32_t x[2];
+        float sq[2];
 #pragma unroll
-            for (int r = 0; r < kNbrs; ++r)
-                tie = tie || (ck[r + 1] != ~0ull && (uint32_t)(ck[r] >> 32) == (uint32_t)(ck[r + 1] >> 32));
+        for (int v = 0; v < 2; ++v) {
+            const uint32_t j = u + v < m5 ? WRACH_CAND(u + v) : i;
+            sq[v] = squared_distance(a.pos[j], q);
+            x[v] = j != i ? u + v : 0xffffffffu;
         }
-        const bool exact = __ballot(tie) != 0;  // every lane votes
-        if (feats) {
-            if (exact) {
 #pragma unroll
-                for (int kb = 1; kb <= kSortLog2; ++kb) {
+        for (int v = 0; v < 2; ++v) {
+            const uint32_t d = (uint32_t)fminf(sq[v] * to_fixed, (float)kDistMax);
+            uint32_t c = x[v] != 0xffffffffu ? min(d, kDistMax) << kNumberBits | x[v] : 0xffffffffu;
 #pragma unroll
-                    for (int jb = kb - 1; jb >= 0; --jb) {
-                        const int kk = 1 << kb, jj = 1 << jb;
-#pragma unroll
-                        for (int u = 0; u < kSortCands; ++u) {
-                            const int l = u ^ jj;
-                            if (l > u) {
-                                const bool up = (u & kk) == 0;
-                                const unsigned long long x = ck[u], y = ck[l];
-                                const bool sw = up ? cand_less(a.pos, a.vel, y, x) : cand_less(a.pos, a.vel, x, y);
-                                ck[u] = sw ? y : x;
-                                ck[l] = sw ? x : y;
-                            }
-                        }
-                    }
-                }
-            }
-#pragma unroll
-            for (int r = 0; r < kNbrs; ++r) key[r] = ck[r];
-            for (uint32_t u = kSortCands; u < m5; ++u) {
-                uint32_t j = 0;
-#pragma unroll
-                for (int t = 0; t < 5; ++t)
-                    if (u >= cum[t] && u < cum[t] + (re[t] - rs[t])) j = rs[t] + (u - cum[t]);
-                if (j == i) continue;
-                const float2 o = a.pos[j];
-                const float dx = o.x - q.x;
-                const float dy = o.y - q.y;
-                float sq = dx * dx;
-                sq = sq + dy * dy;
-                insert16(a.pos, a.vel, key, ((unsigned long long)__float_as_uint(sq) << 32) | j);
+            for (int r = 0; r <= kNbrs; ++r) {
+                const uint32_t lo = min(ck[r], c);
+                c = max(ck[r], c);
+                ck[r] = lo;
             }
         }
-        uint4 *row = reinterpret_cast<uint4 *>(a.feat + (size_t)(a.row0 + i) * kFeat);
+    }
+    bool tie = false;
 #pragma unroll
-        for (int r = 0; r < kNbrs; r += 2) {
+    for (int r = 0; r < kNbrs; ++r) tie = tie || (ck[r + 1] != 0xffffffffu && (ck[r] ^ ck[r + 1]) < kKeyCands);
+    uint32_t near[kNbrs];  // the neighbours; ~0: none
+#pragma unroll
+    for (int r = 0; r < kNbrs; ++r) near[r] = ck[r] != 0xffffffffu ? WRACH_CAND(ck[r] & (kKeyCands - 1)) : 0xffffffffu;
+    const bool more = m5 > kKeyCands;
+    if (__ballot(tie || more) != 0) {  // every lane votes
+        // Lanes with a tie from their first candidate on, lanes with more
+        // than kKeyCands from there on; a candidate past the 16th in fixed
+        // point is past it exactly.
+        const uint32_t last = ck[kNbrs - 1] >> kNumberBits;
+        unsigned long long key[kNbrs];
+#pragma unroll
+        for (int r = 0; r < kNbrs; ++r)
+            key[r] = tie || near[r] == 0xffffffffu
+                         ? ~0ull
+                         : ((unsigned long long)__float_as_uint(squared_distance(a.pos[near[r]], q)) << 32) | near[r];
+        const uint32_t begin = tie ? 0u : kKeyCands, end = tie || more ? m5 : 0u;
+        for (uint32_t u = __ballot(tie) != 0 ? 0u : kKeyCands; __ballot(u < end) != 0; ++u) {
+            if (u < begin || u >= end) continue;
+            const uint32_t j = WRACH_CAND(u);
+            if (j == i) continue;
+            const float sq = squared_distance(a.pos[j], q);
+            if ((uint32_t)fminf(sq * to_fixed, (float)kDistMax) > last) continue;
+            insert16(a.pos, a.vel, key, ((unsigned long long)__float_as_uint(sq) << 32) | j);
+        }
+#pragma unroll
+        for (int r = 0; r < kNbrs; ++r)
+            if (tie || more) near[r] = key[r] != ~0ull ? (uint32_t)key[r] : 0xffffffffu;
+    }
+#undef WRACH_CAND
+    // The rows through LDS, half a row at a time, so that a wavefront stores
+    // 64 bytes of 16 rows at once (a lane's 16 bytes at a time, its stores hit
+    // 64 rows each): chunk c of lane l at place c ^ (l / 2 % 4), which spreads
+    // both sides over the banks.
+    uint4 *out = sh.rows[threadIdx.x >> 6];
+    const unsigned long long rows_on = __ballot(on);
+#pragma unroll
+    for (uint32_t h0 = 0; h0 < 8; h0 += 4) {
+#pragma unroll
+        for (uint32_t c = 0; c < 4; ++c) {
             uint32_t h[4] = {0u, 0u, 0u, 0u};
-#pragma unroll
-            for (int u = 0; u < 2; ++u) {
-                if (key[r + u] != ~0ull) {
-                    const uint32_t j = (uint32_t)key[r + u];
-                    const float2 o = a.pos[j];
-                    const float2 ov = a.vel[j];
-                    h[2 * u] = (uint32_t)bf16_bits(o.x - q.x) | ((uint32_t)bf16_bits(o.y - q.y) << 16);
-                    h[2 * u + 1] = (uint32_t)bf16_bits(ov.x - w.x) | ((uint32_t)bf16_bits(ov.y - w.y) << 16);
-                }
+            const uint32_t n0 = near[2 * (h0 + c)], n1 = near[2 * (h0 + c) + 1];
+            const float4 s0 = particle_state(a, n0 != 0xffffffffu ? n0 : i);
+            const float4 s1 = particle_state(a, n1 != 0xffffffffu ? n1 : i);
+            if (n0 != 0xffffffffu) {
+                h[0] = bf16_pair(s0.x - q.x, s0.y - q.y);
+                h[1] = bf16_pair(s0.z - w.x, s0.w - w.y);
             }
-            row[r / 2] = make_uint4(h[0], h[1], h[2], h[3]);
+            if (n1 != 0xffffffffu) {
+                h[2] = bf16_pair(s1.x - q.x, s1.y - q.y);
+                h[3] = bf16_pair(s1.z - w.x, s1.w - w.y);
+            }
+            out[lane * 4 + (c ^ (lane >> 1 & 3))] = make_uint4(h[0], h[1], h[2], h[3]);
         }
+        wave_sync();
+#pragma unroll
+        for (uint32_t v = 0; v < 4; ++v) {
+            const uint32_t row = v * 16 + (lane >> 2), c = lane & 3;
+            const uint32_t to = (uint32_t)__shfl((int)i, (int)row, 64);
+            if ((rows_on >> row) & 1ull)
+                reinterpret_cast<uint4 *>(a.feat + (size_t)(a.row0 + to) * kFeat)[h0 + c] =
+                    out[row * 4 + (c ^ (row >> 1 & 3))];
+        }
+        wave_sync();
     }
     if (a.sums) {
-        __shared__ unsigned long long s_sum[4], s_cnt[4];
-#pragma unroll
-        for (int o = 32; o > 0; o >>= 1) {
-            osum += __shfl_xor(osum, o, 64);
-            ocnt += __shfl_xor(ocnt, o, 64);
-        }
-        if (lane_id() == 0) {
-            s_sum[threadIdx.x >> 6] = osum;
-            s_cnt[threadIdx.x >> 6] = ocnt;
-        }
+        // The overlap sums: the 3x3 cells, as a separation pass visits them.
         __syncthreads();
-        if (threadIdx.x == 0) {
-            const unsigned long long cnt = s_cnt[0] + s_cnt[1] + s_cnt[2] + s_cnt[3];
-            if (cnt) {
-                unsigned long long *slot = a.sums + (blockIdx.x % kStencilSumSlots) * kStencilSumStride;
-                atomicAdd(slot, s_sum[0] + s_sum[1] + s_sum[2] + s_sum[3]);
-                atomicAdd(slot + 1, cnt);
-            }
-        }
+        const PairSums s = stencil_particle<false, true, false>(a.pos, i, q.x, q.y, r3, sh.list + threadIdx.x);
+        block_report(nullptr, 0, s, a.sums, 1ull);
     }
 }
 
@@ -2997,6 +3095,12 @@ hipError_t launch_stencil_move(const FrameParams &p, const FrameBuffers &b, cons
 hipError_t launch_learn_features(const FrameParams &p, const FrameBuffers &b, const FeatureArgs &a,
                                  hipStream_t stream) {
     if (p.n == 0) return hipSuccess;
+    if (a.state) {
+        hipLaunchKernelGGL(learn_state_kernel, dim3((p.n + 255) / 256), dim3(256), 0, stream, a.pos, a.vel, a.state,
+                           p.n);
+        const hipError_t e = hipGetLastError();
+        if (e != hipSuccess) return e;
+    }
     hipLaunchKernelGGL(learn_features_kernel, dim3((p.n + 255) / 256), dim3(256), 0, stream, p, b, a);
     return hipGetLastError();
 }

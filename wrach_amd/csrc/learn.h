@@ -49,15 +49,23 @@ struct MlpWeights {
 
 // Neighbour features of the packed state (pos, vel) for particles
 // [0, p.n): row row0 + i of `feat` (64 bf16) for particle i.  Optional:
-// each particle's cell (`cell`), and the overlap sums of these positions
-// over the 3x3 cells as a separation pass measures them, added to `sums`
-// (the layout of the stencil sums: slot block % kStencilSumSlots).
+// what the separation passes that follow need, in their lane order (`perm`,
+// null: the particles' own) -- the rows of each lane's 3x3 cells (`rows`,
+// `rows2`), or without them each particle's cell (`cell`), and the budget's
+// word (`words`) -- and the overlap sums of these positions over the 3x3
+// cells as a separation pass measures them, added to `sums` (the layout of
+// the stencil sums: slot block % kStencilSumSlots).
 struct FeatureArgs {
     const float2 *pos;
     const float2 *vel;
+    float4 *state;  // workspace: (pos, vel) of each particle (null: gathered apart)
     uint16_t *feat;
     uint32_t row0;
+    const uint32_t *perm;
+    uint4 *rows;
+    uint2 *rows2;
     uint32_t *cell;
+    uint32_t *words;
     unsigned long long *sums;
 };
 hipError_t launch_learn_features(const FrameParams &p, const FrameBuffers &b, const FeatureArgs &a,

@@ -208,13 +208,14 @@ __global__ __launch_bounds__(kInferBlock) __attribute__((amdgpu_waves_per_eu(4))
         bf16x8 xb[kInferCols][2];
         load_rows<kInferCols>(a.feat, nullptr, row0, a.n, xb);
         float y[kInferCols][2];
-        // The weights stay in LDS: an address the optimiser cannot see
+        // The weights stay in LDS: an offset the optimiser cannot see
         // through keeps it from hoisting all 48 fragments into registers for
-        // the whole loop (192 VGPRs, one wavefront per SIMD).
-        const bf16x8 *fr = s_frag;
-        const float *b1 = s_b1, *b2 = s_b2, *w3 = s_w3;
-        asm volatile("" : "+v"(fr), "+v"(b1), "+v"(b2), "+v"(w3));
-        mlp_infer<kInferCols>(xb, fr, b1, b2, w3, s_b3, y);
+        // the whole loop (192 VGPRs, one wavefront per SIMD).  An offset, not
+        // the addresses: those would lose their address space and turn every
+        // LDS read into a flat load (111 us for 1M rows).
+        uint32_t z = 0;
+        asm volatile("" : "+v"(z));
+        mlp_infer<kInferCols>(xb, s_frag + z, s_b1 + z, s_b2 + z, s_w3 + z, s_b3, y);
         if (l < 16) {
 #pragma unroll
             for (int c = 0; c < kInferCols; ++c) {
