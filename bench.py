@@ -283,19 +283,21 @@ def traffic_summary(args) -> int:
     fetch_scale = probe_kib / copy_value(copy_fetch_csv, "FETCH_SIZE")   # copy reads probe bytes
     write_scale = probe_kib / copy_value(copy_write_csv, "WRITE_SIZE")   # and writes them
     fetch, write = per_kernel(fetch_csv, "FETCH_SIZE"), per_kernel(write_csv, "WRITE_SIZE")
-    names = {"collide": "collide_kernel", "cells": "cells_kernel", "scan": "scan_kernel",
-             "scatter": "scatter_kernel"}
+    # a large grid's scan is two kernels
+    names = {"collide": ["collide_kernel"], "cells": ["cells_kernel"],
+             "scan": ["cell_scan_kernel", "chunk_scan_kernel"] if any("cell_scan_kernel" in k for k in fetch)
+             else ["scan_kernel"], "scatter": ["scatter_kernel"]}
     kernels = {}
     def find(table, needle):
         # "::scatter_kernel<" or "::scatter_kernel(", not upload_scatter_kernel
         return next(k for k in table if f"::{needle}<" in k or f"::{needle}(" in k)
 
-    for short, needle in names.items():
-        fk, wk = find(fetch, needle), find(write, needle)
-        f = float(np.median(fetch[fk][-args.profile_steps:])) * 1024 * fetch_scale
-        w = float(np.median(write[wk][-args.profile_steps:])) * 1024 * write_scale
+    for short, needles in names.items():
+        fks, wks = [find(fetch, k) for k in needles], [find(write, k) for k in needles]
+        f = sum(float(np.median(fetch[k][-args.profile_steps:])) for k in fks) * 1024 * fetch_scale
+        w = sum(float(np.median(write[k][-args.profile_steps:])) for k in wks) * 1024 * write_scale
         kernels[short] = {"hbm_bytes_per_launch": int(f + w), "fetch_bytes": int(f), "write_bytes": int(w),
-                          "dispatches": len(fetch[fk])}
+                          "dispatches": len(fetch[fks[0]])}
     out = {"_about": "HBM bytes per launch from rocprofv3 FETCH_SIZE and WRITE_SIZE (KiB per dispatch), "
                      f"scaled by a {args.copy_probe_bytes} B device copy (FETCH x{fetch_scale:.3f}, WRITE "
                      f"x{write_scale:.3f}); median over each frame kernel's last {args.profile_steps} "

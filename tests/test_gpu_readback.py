@@ -6,7 +6,7 @@ import ctypes
 import numpy as np
 import pytest
 
-from tests.test_gpu_parity import f32, say
+from tests.test_gpu_parity import f32, oracle_world, say
 from tests.test_zz_no_alloc import Hip
 from wrach_amd import World, WrachConfig, WrachError, _lib
 
@@ -109,3 +109,89 @@ def test_noalloc_frame_of_a_crowded_cell(oracle, m, offset):
             assert_packed(got, ref, f"m={m} offset={offset} call {call}")
     finally:
         hip.free(di, dp, dv)
+
+
+@pytest.mark.parametrize("cells", [(2897, 2897), (4096, 2049), (11000, 800)])
+def test_grids_just_above_the_large_scan(oracle, cells):
+    """Grids of 2^23 cells and a little more (a last chunk that is not whole,
+    one that ends with the grid, a row of a fraction of the chunks): offsets
+    counted from their chunk's first cell until a readback.  Particles in the
+    first and last cells, a crowded one, one chunk alone; read, stepped, read
+    again, a world's count, an append, and Mode S passes from such offsets."""
+    gx, gy = cells
+    rng = np.random.default_rng(gx)
+    W, H = gx - 1, gy - 1
+    n = 3000
+    pos = np.concatenate([rng.uniform((1, 1), (W - 1, 40), (n, 2)),             # the first chunks
+                          rng.uniform((W - 60, H - 30), (W - 0.5, H - 0.5), (n, 2)),  # the last
+                          rng.uniform((700, 500), (703, 503), (300, 2)),        # crowded, alone
+                          [[0.0, 0.0], [W, H], [W, 0.0], [0.0, H]]])
+    pos, vel = f32(pos), f32(rng.uniform(-0.4, 0.4, (len(pos), 2)))
+    cfg = WrachConfig(dimensions=(W, H), cell_size=1, gravity=(0.0, -0.03))
+    P, ref = oracle_world(oracle, cfg, pos, vel)
+    say(f"[readback] grid {gx} x {gy}")
+    with World(cfg) as w:
+        w.add_particles(pos, vel)
+        assert_packed(w.read(), ref, "upload")
+        for frames in (1, 5):
+            w.step(frames)
+            assert w.world_settings(0).particles_in_frame_count == len(ref[1])
+            ref = oracle.step(P, *ref, nsteps=frames)
+            assert_packed(w.read(), ref, f"{frames} frames")
+        w.step(1)
+        ref = oracle.step(P, *ref, nsteps=1)
+        w.autotune(2)  # its snapshot holds offsets as the frame left them
+        w.step(1)
+        ref = oracle.step(P, *ref, nsteps=1)
+        assert_packed(w.read(), ref, "after autotune")
+        w.step(1)
+        ref = oracle.step(P, *ref, nsteps=1)
+        w.set_solver("S", 2)  # the offsets of a frame without passes
+        w.step(2)
+        *ref, st = oracle.step_s(P, *ref, max_passes=2, nsteps=2)
+        assert_packed(w.read(), ref, "Mode S")
+        assert w.solver_stats() == st
+        w.set_solver("R")
+        w.step(1)
+        more = f32(rng.uniform(0, 30, (50, 2)))
+        ref = oracle.step(P, *ref, nsteps=1)
+        w.store_write_back()  # the append re-packs where the particles are now
+        w.add_particles(more, more * 0)
+        got = w.read()
+        assert got[0][-1] == len(ref[1]) + 50 and np.all(np.diff(got[0].astype(np.int64)) >= 0)
+        cell = np.floor(got[1][:, 1]).astype(np.int64) * gx + np.floor(got[1][:, 0]).astype(np.int64)
+        assert np.array_equal(np.bincount(cell, minlength=gx * gy), np.diff(got[0][1:].astype(np.int64)))
+
+
+@pytest.mark.parametrize("m", [65534, 65535, 70000])
+def test_large_grid_with_a_chunk_past_16_bits(oracle, m):
+    """A chunk of as many particles as 16-bit offsets hold, and more, beside
+    ordinary ones: frames, Mode S passes and the readback."""
+    rng = np.random.default_rng(m)
+    gx, gy = 4099, 2053
+    W, H = gx - 1, gy - 1
+    cell = 1024 * 8 + np.arange(m) % 1000
+    pos = np.concatenate([np.stack([cell % gx, cell // gx], 1) + rng.uniform(0.01, 0.99, (m, 2)),
+                          rng.uniform((1, 20), (W - 1, 90), (2000, 2))])
+    pos, vel = f32(pos), f32(rng.uniform(-0.2, 0.2, (m + 2000, 2)))
+    cfg = WrachConfig(dimensions=(W, H), cell_size=1, gravity=(0.0, -0.01))
+    P, ref = oracle_world(oracle, cfg, pos, vel)
+    assert np.diff(ref[0][1:].astype(np.int64))[1024 * 8:1024 * 9].sum() == m
+    say(f"[readback] chunk of {m}")
+    with World(cfg) as w:
+        w.add_particles(pos, vel)
+        assert_packed(w.read(), ref, "upload")
+        w.set_solver("S", 1)
+        for frames in (1, 2):
+            w.step(frames)
+            *ref, st = oracle.step_s(P, *ref, max_passes=1, nsteps=frames)
+            assert w.world_settings(0).particles_in_frame_count == len(ref[1])
+            assert_packed(w.read(), ref, f"{frames} frames")
+        w.set_solver("R")
+        w.step(2)
+        ref = oracle.step(P, *ref, nsteps=2)
+        w.set_solver("S", 1)  # the offsets of a frame without passes
+        w.step(1)
+        *ref, st = oracle.step_s(P, *ref, max_passes=1, nsteps=1)
+        assert_packed(w.read(), ref, "passes after plain frames")
+        assert w.solver_stats() == st

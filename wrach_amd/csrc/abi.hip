@@ -374,6 +374,8 @@ void release(wrach_ctx *c) {
     (void)hipFree(c->buf.chunk_next);
     (void)hipFree(c->buf.chunk_live);
     (void)hipFree(c->buf.chunk_prefix);
+    (void)hipFree(c->buf.chunk_sum);
+    (void)hipFree(c->buf.rel);
     (void)hipFree(c->buf.epoch);
     (void)hipFree(c->buf.error);
     if (c->err_host) (void)hipHostFree(c->err_host);
@@ -472,7 +474,7 @@ int add_host_packed(wrach_ctx *c, const float *pos_xy, const float *vel_xy, uint
     WRACH_HIP(wrach::launch_iota(c->buf.src, packed, c->stream));
     WRACH_HIP(wrach::launch_keys_from_offsets(c->buf.idx, (uint32_t)c->ncell, packed, c->buf.key, c->stream));
     // every offset came from the host: no chunk's offsets are stale
-    WRACH_HIP(hipMemsetAsync(c->buf.chunk_live, 1, c->chunks, c->stream));
+    WRACH_HIP(hipMemsetAsync(c->buf.chunk_live, wrach::kChunkWhole, c->chunks, c->stream));
     WRACH_SETTLE(c);
     if (c->fp.n != packed) free_graphs(c);
     c->fp.n = packed;
@@ -797,6 +799,17 @@ int create_ctx(const wrach_config *cfg, uint32_t n_worlds, const wrach_config *w
     WRACH_HIP_C(dmalloc(&b.chunk_next, c->chunks));
     WRACH_HIP_C(dmalloc(&b.chunk_live, c->chunks));
     WRACH_HIP_C(dmalloc(&b.chunk_prefix, c->chunks));
+    b.off = b.idx + 1;
+    b.off_shift = 0;
+    b.off_mask = ~0u;
+    if (wrach::relative_offsets(ncell)) {
+        WRACH_HIP_C(dmalloc(&b.chunk_sum, c->chunks));
+        WRACH_HIP_C(dmalloc(&b.rel, c->chunks * wrach::kChunkCells));
+        b.off = reinterpret_cast<const uint32_t *>(b.rel);
+        b.off_shift = 1;
+        b.off_mask = 0xffff;
+        WRACH_HIP_C(hipMemsetAsync(b.rel, 0, c->chunks * wrach::kChunkCells * sizeof(uint16_t), c->stream));
+    }
     WRACH_HIP_C(dmalloc(&b.epoch, 1));
     WRACH_HIP_C(dmalloc(&b.error, 1));
     WRACH_HIP_C(hipHostMalloc((void **)&c->err_host, sizeof(uint32_t), hipHostMallocDefault));
@@ -1072,7 +1085,17 @@ int ensure_stencil(wrach_ctx *c) {
 }
 
 // The learned frame's buffers: feature rows and a third position buffer.
+// The passes and features read idx; a large grid's frames leave offsets there
+// only with a solver that has them (FrameParams::idx_read).
+int offsets_for_passes(wrach_ctx *c) {
+    if (wrach::relative_offsets(c->ncell) && !c->fp.idx_read)
+        WRACH_HIP(wrach::launch_materialize(c->fp, c->buf, c->stream));
+    return WRACH_OK;
+}
+
 int ensure_learned_frame(wrach_ctx *c) {
+    const int offsets = offsets_for_passes(c);
+    if (offsets) return offsets;
     const size_t rows = c->capacity ? c->capacity : 1;
     if (!c->lfeat) {
         uint16_t *f = nullptr;
@@ -1118,7 +1141,8 @@ int wrach_set_solver(wrach_ctx *c, uint32_t mode, uint32_t max_passes, float ove
     WRACH_HIP(hipSetDevice(c->cfg.device));
     WRACH_SETTLE(c);
     if (mode != WRACH_SOLVER_R) {
-        const int rc = ensure_stencil(c);
+        int rc = ensure_stencil(c);
+        if (!rc) rc = offsets_for_passes(c);
         if (rc) return rc;
     }
     if (mode == WRACH_SOLVER_L) {
@@ -1129,6 +1153,7 @@ int wrach_set_solver(wrach_ctx *c, uint32_t mode, uint32_t max_passes, float ove
     if (c->ssums) WRACH_HIP(hipMemset(c->ssums, 0, wrach::kStencilSumEntries * sizeof(unsigned long long)));
     free_graphs(c);  // captured with the previous solver
     c->solver = mode;
+    c->fp.idx_read = mode != WRACH_SOLVER_R ? 1 : 0;
     c->quiet = quiet;
     c->passes = mode != WRACH_SOLVER_R ? max_passes : 0;
     c->overlap_tol = mode == WRACH_SOLVER_S ? overlap_tol : 0.0f;
@@ -1402,7 +1427,7 @@ int wrach_load_packed(wrach_ctx *c, const uint32_t *indices, size_t n_indices, c
     }
     WRACH_HIP(wrach::launch_iota(c->buf.src, n, c->stream));
     WRACH_HIP(wrach::launch_keys_from_offsets(c->buf.idx, (uint32_t)c->ncell, n, c->buf.key, c->stream));
-    WRACH_HIP(hipMemsetAsync(c->buf.chunk_live, 1, c->chunks, c->stream));  // offsets from the host
+    WRACH_HIP(hipMemsetAsync(c->buf.chunk_live, wrach::kChunkWhole, c->chunks, c->stream));  // offsets from the host
     if (c->host_pack) {
         c->store_pos.assign(pos_xy, pos_xy + 2 * (size_t)n);
         c->store_vel.assign(vel_xy, vel_xy + 2 * (size_t)n);
@@ -1496,7 +1521,7 @@ int wrach_autotune(wrach_ctx *c, uint32_t frames, wrach_tuning *out) {
     // clean between frames).
     const size_t nidx = c->ncell + 2;
     void *s_idx = nullptr, *s_pos = nullptr, *s_vel = nullptr, *s_src = nullptr, *s_key = nullptr,
-         *s_live = nullptr, *s_pre = nullptr;
+         *s_live = nullptr, *s_pre = nullptr, *s_rel = nullptr;
     hipEvent_t e0 = nullptr, e1 = nullptr;
     auto cleanup = [&]() {
         (void)hipFree(s_idx);
@@ -1506,13 +1531,16 @@ int wrach_autotune(wrach_ctx *c, uint32_t frames, wrach_tuning *out) {
         (void)hipFree(s_key);
         (void)hipFree(s_live);
         (void)hipFree(s_pre);
+        (void)hipFree(s_rel);
         if (e0) (void)hipEventDestroy(e0);
         if (e1) (void)hipEventDestroy(e1);
     };
     auto copy = [&](void *dst, const void *src, size_t bytes) {
         return hipMemcpyAsync(dst, src, bytes, hipMemcpyDeviceToDevice, c->stream);
     };
+    const size_t rel_bytes = c->buf.rel ? c->chunks * wrach::kChunkCells * sizeof(uint16_t) : 0;
     hipError_t e = hipMalloc(&s_idx, nidx * sizeof(uint32_t));
+    if (e == hipSuccess && rel_bytes) e = hipMalloc(&s_rel, rel_bytes);
     if (e == hipSuccess) e = hipMalloc(&s_pos, (size_t)n * sizeof(float2));
     if (e == hipSuccess) e = hipMalloc(&s_vel, (size_t)n * sizeof(float2));
     if (e == hipSuccess) e = hipMalloc(&s_src, (size_t)n * sizeof(uint32_t));
@@ -1528,6 +1556,7 @@ int wrach_autotune(wrach_ctx *c, uint32_t frames, wrach_tuning *out) {
     if (e == hipSuccess) e = copy(s_key, c->buf.key, (size_t)n * sizeof(uint32_t));
     if (e == hipSuccess) e = copy(s_live, c->buf.chunk_live, c->chunks);
     if (e == hipSuccess) e = copy(s_pre, c->buf.chunk_prefix, c->chunks * sizeof(uint32_t));
+    if (e == hipSuccess && rel_bytes) e = copy(s_rel, c->buf.rel, rel_bytes);
     if (e != hipSuccess) {
         cleanup();
         return fail(WRACH_E_DEVICE, std::string("autotune snapshot: ") + hipGetErrorString(e));
@@ -1540,6 +1569,7 @@ int wrach_autotune(wrach_ctx *c, uint32_t frames, wrach_tuning *out) {
         if (r == hipSuccess) r = copy(c->buf.key, s_key, (size_t)n * sizeof(uint32_t));
         if (r == hipSuccess) r = copy(c->buf.chunk_live, s_live, c->chunks);
         if (r == hipSuccess) r = copy(c->buf.chunk_prefix, s_pre, c->chunks * sizeof(uint32_t));
+        if (r == hipSuccess && rel_bytes) r = copy(c->buf.rel, s_rel, rel_bytes);
         if (r == hipSuccess) r = hipStreamSynchronize(c->stream);
         return r;
     };
@@ -2234,6 +2264,9 @@ size_t carve_noalloc(unsigned char *base, uint32_t n, uint64_t ncell, wrach::Fra
     const size_t np = n ? n : 1;
     b.idx = reinterpret_cast<uint32_t *>(take((ncell + 2 + 64) * sizeof(uint32_t)));
     if (b.idx) b.idx += 3;  // &idx[1] on a 16-byte boundary
+    b.off = b.idx ? b.idx + 1 : nullptr;
+    b.off_shift = 0;
+    b.off_mask = ~0u;
     b.pos = reinterpret_cast<float2 *>(take(np * sizeof(float2)));
     b.vel = reinterpret_cast<float2 *>(take(np * sizeof(float2)));
     b.src = reinterpret_cast<uint32_t *>(take(np * sizeof(uint32_t)));
@@ -2332,6 +2365,7 @@ int wrach_frame_noalloc(const wrach_world_settings *ws, const float gravity[2], 
                           (alignof(float2) - 1)) == 0;
     wrach::FrameBuffers in = b, out = b;
     in.idx = indices;
+    in.off = indices + 1;
     if (aligned) {
         in.pos = out.pos_out = reinterpret_cast<float2 *>(pos_xy);
         in.vel = out.vel_out = reinterpret_cast<float2 *>(vel_xy);

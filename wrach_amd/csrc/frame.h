@@ -46,6 +46,12 @@ struct FrameParams {
     // epoch_skew is 0 except in a test that forces that path from the host:
     // the look-back then expects an epoch no status word carries.
     uint32_t wait_limit;
+    // Large grids: the scan leaves its offsets in idx too, besides rel (where
+    // they are counted from the chunk's first cell alike): frames whose
+    // separation passes read up to 17 of them a particle, for which the
+    // look-up in 16 bits costs registers.  Elsewhere launch_materialize makes
+    // idx good for those kernels.
+    uint32_t idx_read;
     uint32_t epoch_skew;
 };
 
@@ -75,11 +81,18 @@ struct FrameBuffers {
     unsigned long long *tile_state;  // scan look-back words
     // Per chunk of kChunkCells cells: chunk_next is set by the first slot
     // claimed in the chunk during a frame (the scan visits only those and
-    // clears it); chunk_live is what the last scan found; chunk_prefix the
-    // offset at the chunk's first cell.  idx entries of a chunk that is not
-    // live are left as they were until a readback fills them in.
+    // clears it); chunk_live is what the last scan found and made of the
+    // chunk's idx entries (kChunk*); chunk_prefix the offset at the chunk's
+    // first cell; chunk_sum (large grids) its particles.  A readback makes
+    // every entry of idx a whole offset.
     uint8_t *chunk_next, *chunk_live;
-    uint32_t *chunk_prefix;
+    uint32_t *chunk_prefix, *chunk_sum;
+    // Where the readers look up an offset: idx + 1, or on large grids
+    // (relative_offsets) `rel`, per cell its offset from the chunk's first
+    // cell in 16 bits, two cells a word (off_shift 1, off_mask 0xffff).
+    const uint32_t *off;
+    uint16_t *rel;
+    uint32_t off_shift, off_mask;
     uint32_t *epoch;      // frame counter tagging the scan's status words; the scatter advances it
     uint32_t *error;      // kErr* bits raised by a kernel that gave up a wait; zero otherwise
     uint4 *cells;         // queued cells (s, n, cell, 0), one region per size class
@@ -96,6 +109,12 @@ struct FrameBuffers {
 constexpr int kCollideBlock = 256;
 constexpr uint32_t kChunkShift = 10;  // a chunk: the cells of one collide block
 constexpr uint32_t kChunkCells = 1u << kChunkShift;
+// States of a chunk: no particles, its entries left as they were; whole
+// offsets in idx; offsets from the chunk's first cell (chunk_prefix to be
+// added) in rel, or, for a chunk of too many particles, all kWideOffset there
+// and in idx.
+constexpr uint8_t kChunkEmpty = 0, kChunkWhole = 1, kChunkRelative = 2;
+constexpr uint32_t kWideOffset = 0xffff;
 // Launch shapes the autotuner (wrach_autotune) chooses among; entry 0 of
 // each table is the default (the scan's: see default_scan_shape).  Scan
 // tiles: threads x counts per thread (1024 x 8 is the fastest in the
@@ -118,7 +137,8 @@ constexpr int kNumScanShapes = 9;
 // 1024 x 8, 18.3 at 1024 x 32, 31.7 at 1024 x 64 and 17.4 at 256 x 128;
 // the 4M blobs' 16.8M cells in 67.5, 57.8, 50.3 and 53.4 us; the
 // 512-world batch's 227M cells at 1024 x 32, 1024 x 64, 512 x 64 and
-// 256 x 128 in 401, 344, 338 and 322 us.
+// 256 x 128 in 401, 344, 338 and 322 us.  (Above kLargeScanGrid the shape is
+// reported and not used, below.)
 constexpr uint64_t kLargeScanGrid = 1ull << 23;
 constexpr uint64_t kHugeScanGrid = 1ull << 26;
 constexpr uint32_t kLargeScanShape = 6;
@@ -127,6 +147,11 @@ static_assert(kScanShapes[kLargeScanShape].threads == 1024 && kScanShapes[kLarge
               "the large-grid scan shape");
 static_assert(kScanShapes[kHugeScanShape].threads == 256 && kScanShapes[kHugeScanShape].items == 128,
               "the huge-grid scan shape");
+// Grids above kLargeScanGrid cells scan each chunk by itself and then the
+// chunks' totals, in two launches (cell_scan_kernel: 29 us for the 16.8M cells
+// and 113 for the 227M above); the shapes apply up to there.
+constexpr bool relative_offsets(uint64_t ncell) { return ncell > kLargeScanGrid; }
+constexpr uint32_t kChunkTile = 4096;  // chunks per block of the totals' scan
 constexpr uint32_t default_scan_shape(uint64_t ncell) {
     return ncell > kHugeScanGrid ? kHugeScanShape : ncell > kLargeScanGrid ? kLargeScanShape : 0u;
 }
@@ -186,7 +211,7 @@ hipError_t launch_scatter(const FrameParams &p, const FrameBuffers &b, hipStream
 // idx made whole as launch_materialize does, or, with idx_out (ncell + 2
 // words), written there.
 hipError_t launch_canonical(const FrameParams &p, const FrameBuffers &b, uint32_t *idx_out, hipStream_t stream);
-// Fills the idx entries of chunks the last scan found empty (before a readback).
+// Makes every idx entry a whole offset (before a readback).
 hipError_t launch_materialize(const FrameParams &p, const FrameBuffers &b, hipStream_t stream);
 // Before a frame on a caller's packed triple in buffers that hold anything:
 // what must be clean cleared, src and key from the caller's offsets.

@@ -49,6 +49,7 @@
 // the reference's shader crate.
 #include <hip/hip_ext.h>
 
+#include <algorithm>
 #include <atomic>
 
 #include "frame.h"
@@ -165,14 +166,38 @@ __device__ __forceinline__ uint32_t claim(const FrameBuffers &b, uint32_t k, uin
     return old;
 }
 
-// First particle of cell k (k == ncell: the end).  Cells of a chunk the last
-// scan found empty all start at the chunk's prefix (their idx entries are
-// stale); a live chunk's are in idx.
+// The offset of a cell, in steps, so that a caller can have the loads of
+// several cells in flight: the word that holds it (of idx, or of a large
+// grid's 16-bit offsets: two cells a word), the entry in that word, on large
+// grids the entry in idx where the 16 bits hold none, and the offset from
+// that and the chunk's state and prefix (frame.h): an empty chunk's entries
+// are stale, its cells all start at the prefix; a live chunk's are offsets,
+// whole or counted from the prefix.
+__device__ __forceinline__ uint32_t offset_word(const FrameBuffers &b, uint32_t k) {
+    return b.off[k >> b.off_shift];
+}
+
+__device__ __forceinline__ uint32_t offset_entry(const FrameBuffers &b, uint32_t k, uint32_t word) {
+    return (word >> ((k & b.off_shift) << 4)) & b.off_mask;
+}
+
+__device__ __forceinline__ uint32_t wide_entry(const FrameBuffers &b, uint32_t k, uint32_t at, uint32_t state) {
+    return state == kChunkWhole || at == kWideOffset ? b.idx[k + 1] : at;
+}
+
+__device__ __forceinline__ uint32_t offset_of(uint32_t at, uint32_t state, uint32_t prefix) {
+    return state == kChunkWhole ? at : state == kChunkRelative ? prefix + at : prefix;
+}
+
+// First particle of cell k (k == ncell: the end).
 __device__ __forceinline__ uint32_t cell_start(const FrameParams &p, const FrameBuffers &b,
                                                uint32_t k) {
     if (k >= p.ncell) return p.n;
     const uint32_t ch = k >> kChunkShift;
-    const uint32_t s = b.chunk_live[ch] ? b.idx[k + 1] : b.chunk_prefix[ch];
+    const uint32_t state = b.chunk_live[ch];
+    uint32_t at = offset_entry(b, k, offset_word(b, k));
+    if (b.off_shift) at = wide_entry(b, k, at, state);
+    const uint32_t s = offset_of(at, state, b.chunk_prefix[ch]);
     return s < p.n ? s : p.n;
 }
 
@@ -211,6 +236,21 @@ __device__ __forceinline__ uint32_t wave_inclusive_sum(uint32_t v) {
         const uint32_t u = __shfl_up(v, off, 64);
         if (lane >= off) v += u;
     }
+    return v;
+}
+
+// Inclusive sum over the wavefront by DPP moves (lanes without a source add
+// 0), one instruction a step.
+__device__ __forceinline__ uint32_t wave_inclusive_dpp(uint32_t v) {
+#define WRACH_DPP_ADD(ctrl, rows) \
+    v += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, ctrl, rows, 0xf, false)
+    WRACH_DPP_ADD(0x111, 0xf);  // row_shr:1, :2, :4, :8
+    WRACH_DPP_ADD(0x112, 0xf);
+    WRACH_DPP_ADD(0x114, 0xf);
+    WRACH_DPP_ADD(0x118, 0xf);
+    WRACH_DPP_ADD(0x142, 0xa);  // row_bcast:15 into rows 1 and 3
+    WRACH_DPP_ADD(0x143, 0xc);  // row_bcast:31 into rows 2 and 3
+#undef WRACH_DPP_ADD
     return v;
 }
 
@@ -533,16 +573,17 @@ __device__ __forceinline__ uint32_t wave_max_u32(uint32_t v) {
 __device__ __forceinline__ void cell_range(const FrameParams &p, const FrameBuffers &b, uint32_t k,
                                            uint32_t &st, uint32_t &en) {
     const uint32_t c0 = k >> kChunkShift;
-    const uint32_t live0 = b.chunk_live[c0], at0 = b.idx[k + 1], pre0 = b.chunk_prefix[c0];
-    uint32_t live1 = 1, at1 = p.n, pre1 = p.n;
-    if (k + 1 < p.ncell) {
-        const uint32_t c1 = (k + 1) >> kChunkShift;
-        live1 = b.chunk_live[c1];
-        at1 = b.idx[k + 2];
-        pre1 = b.chunk_prefix[c1];
+    const uint32_t live0 = b.chunk_live[c0], w0 = offset_word(b, k), pre0 = b.chunk_prefix[c0];
+    const bool last = k + 1 >= p.ncell;
+    const uint32_t k1 = last ? k : k + 1, c1 = k1 >> kChunkShift;
+    const uint32_t live1 = b.chunk_live[c1], w1 = offset_word(b, k1), pre1 = b.chunk_prefix[c1];
+    uint32_t at0 = offset_entry(b, k, w0), at1 = offset_entry(b, k1, w1);
+    if (b.off_shift) {
+        at0 = wide_entry(b, k, at0, live0);
+        at1 = wide_entry(b, k1, at1, live1);
     }
-    st = live0 ? at0 : pre0;
-    en = live1 ? at1 : pre1;
+    st = offset_of(at0, live0, pre0);
+    en = last ? p.n : offset_of(at1, live1, pre1);
     st = st < p.n ? st : p.n;
     en = en < p.n ? en : p.n;
 }
@@ -1312,7 +1353,8 @@ __global__ __launch_bounds__(kCollideBlock) void cells_kernel(FrameParams p, Fra
 // block sorting each of them from the queue.
 //
 // The blocks after the particles' fill the offsets: to b.idx those of the
-// chunks the last scan found empty, or to `idx_out` all of them.
+// chunks the last scan found empty, or to `idx_out` all of them (no chunk is
+// relative then: launch_canonical).
 __global__ __launch_bounds__(kCollideBlock) void canonical_kernel(FrameParams p, FrameBuffers b,
                                                                   uint32_t *idx_out) {
     __shared__ unsigned long long sk[kLdsSort];
@@ -1476,6 +1518,28 @@ __device__ uint32_t look_back(const FrameParams &p, const FrameBuffers &b, uint3
     }
 }
 
+// By the first wavefront of a tile with total `agg`: publishes it, finds the
+// tile's exclusive prefix and publishes that.
+__device__ __forceinline__ uint32_t publish_tile(const FrameParams &p, const FrameBuffers &b, uint32_t tile,
+                                                 uint32_t epoch, uint32_t agg) {
+    const uint32_t lane = lane_id();
+    uint32_t excl = 0;
+    if (tile == 0) {
+        if (lane == 0)
+            __hip_atomic_store(&b.tile_state[0], status_word(kFlagInclusive, epoch, agg), __ATOMIC_RELAXED,
+                               __HIP_MEMORY_SCOPE_AGENT);
+    } else {
+        if (lane == 0)
+            __hip_atomic_store(&b.tile_state[tile], status_word(kFlagAggregate, epoch, agg), __ATOMIC_RELAXED,
+                               __HIP_MEMORY_SCOPE_AGENT);
+        excl = look_back(p, b, tile, epoch);
+        if (lane == 0)
+            __hip_atomic_store(&b.tile_state[tile], status_word(kFlagInclusive, epoch, excl + agg), __ATOMIC_RELAXED,
+                               __HIP_MEMORY_SCOPE_AGENT);
+    }
+    return excl;
+}
+
 // THREADS x ITEMS counts per tile (kScanShapes); ITEMS is a multiple of 4.
 template <int THREADS, int ITEMS>
 __global__ __launch_bounds__(THREADS) void scan_kernel(FrameParams p, FrameBuffers b) {
@@ -1538,21 +1602,7 @@ __global__ __launch_bounds__(THREADS) void scan_kernel(FrameParams p, FrameBuffe
     }
 
     if (wave == 0) {
-        uint32_t excl = 0;
-        if (tile == 0) {
-            if (lane == 0)
-                __hip_atomic_store(&b.tile_state[0], status_word(kFlagInclusive, epoch, agg),
-                                   __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        } else {
-            if (lane == 0)
-                __hip_atomic_store(&b.tile_state[tile], status_word(kFlagAggregate, epoch, agg),
-                                   __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-            excl = look_back(p, b, tile, epoch);
-            if (lane == 0)
-                __hip_atomic_store(&b.tile_state[tile],
-                                   status_word(kFlagInclusive, epoch, excl + agg),
-                                   __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        }
+        const uint32_t excl = publish_tile(p, b, tile, epoch, agg);
         if (lane == 0) s_prefix = excl;
     }
     __syncthreads();
@@ -1579,7 +1629,7 @@ __global__ __launch_bounds__(THREADS) void scan_kernel(FrameParams p, FrameBuffe
     }
     if ((base & (kChunkCells - 1)) == 0 && base < p.ncell) {  // the chunk's first thread
         b.chunk_prefix[chunk] = out[0];
-        b.chunk_live[chunk] = live ? 1 : 0;
+        b.chunk_live[chunk] = live ? kChunkWhole : kChunkEmpty;
         b.chunk_next[chunk] = 0;  // every thread of the chunk read it before the barriers above
     }
     if (tile == 0 && tid == 0) {
@@ -1591,12 +1641,165 @@ __global__ __launch_bounds__(THREADS) void scan_kernel(FrameParams p, FrameBuffe
     if (tile == b.scan_tiles - 1 && tid == 0) b.idx[p.ncell + 1] = s_prefix + agg;
 }
 
+// The scan of large grids (relative_offsets), in two launches without a wait
+// between tiles of cells: every live chunk scanned by itself by one
+// wavefront, its offsets left counted from its own first cell, and then the
+// chunks' totals scanned (chunk_scan_kernel), which makes the chunks' first
+// offsets.  Readers add the two.  Counted so they fit 16 bits, which halves
+// what this kernel writes and what the scatter gathers; a chunk of more
+// particles than that has kWideOffset there and its offsets in idx.  The
+// counts are read and cleared past the caches (nontemporal): the offsets,
+// which the scatter reads next, stay in them.
+//
+// One pass over the cells (scan_kernel) holds its counts in registers until
+// its look-back ends, two tiles of 32k cells on a CU, one loading while the
+// other waits.  512 worlds of 227M cells, half the chunks live: 345 us in one
+// pass, 107 + 6 here (0.45 GB of counts read and 0.23 GB written), and with
+// 32-bit offsets 137 + 6.  4M particles on 16.8M cells: 49 us, 23 + 6 here,
+// and their scatter 54 and 45 (53 with the counts read through the caches).
+// The 2.1M cells of the 1M lattice take 7.4 us in one pass, hardly more than
+// two launches cost; hence the line at 2^23 cells, where the pass needed
+// larger tiles already.
+//
+// A wavefront looks after `per` consecutive chunks: as few as leave every
+// wavefront slot of the device one (kChipWaves), at most kWaveChunks (4, 16:
+// 144 and 168 us instead of 137 on the 227M cells: the chunks in flight lie
+// farther apart).
+constexpr uint32_t kWaveChunks = 2, kChipWaves = 8192;
+
+__device__ __forceinline__ uint4 load_past(const uint4 *p) {
+    typedef uint32_t u4 __attribute__((ext_vector_type(4)));
+    const u4 v = __builtin_nontemporal_load(reinterpret_cast<const u4 *>(p));
+    return make_uint4(v.x, v.y, v.z, v.w);
+}
+
+__device__ __forceinline__ void clear_past(uint4 *p) {
+    typedef uint32_t u4 __attribute__((ext_vector_type(4)));
+    const u4 zero = {0, 0, 0, 0};
+    __builtin_nontemporal_store(zero, reinterpret_cast<u4 *>(p));
+}
+
+__global__ __launch_bounds__(256) void cell_scan_kernel(FrameParams p, FrameBuffers b, uint32_t chunks, uint32_t per) {
+    const uint32_t lane = lane_id(), wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const uint32_t c0 = (blockIdx.x * 4 + wave) * per;
+    // The cell kernel of this frame has finished with the lists.
+    for (uint32_t i = blockIdx.x * 256 + threadIdx.x; i < (uint32_t)(kClasses * (kSlices + 1)); i += gridDim.x * 256)
+        b.class_ctr[i * kCtrStride] = 0;
+    if (c0 >= chunks) return;
+    const bool mine = lane < per && c0 + lane < chunks;
+    const uint32_t marked = mine ? b.chunk_next[c0 + lane] : 0u;
+    uint32_t total = 0;  // lane l: of chunk c0 + l
+    for (unsigned long long left = __ballot(marked != 0); left; left &= left - 1) {
+        const uint32_t which = (uint32_t)__builtin_ctzll(left), c = c0 + which;
+        const uint32_t base = c * kChunkCells + 4 * lane;  // cells base + 256u .. + 3
+        uint4 v[4], at[4];
+        if (c * kChunkCells + kChunkCells <= p.ncell) {
+            uint4 *q = reinterpret_cast<uint4 *>(b.cnt + base);
+#pragma unroll
+            for (int u = 0; u < 4; ++u) v[u] = load_past(q + 64 * u);
+            // Clear only what holds counts: most cells of a large grid are empty.
+#pragma unroll
+            for (int u = 0; u < 4; ++u)
+                if (v[u].x | v[u].y | v[u].z | v[u].w) clear_past(q + 64 * u);
+        } else {  // the grid's last chunk
+#pragma unroll
+            for (int u = 0; u < 4; ++u) {
+                uint32_t w[4];
+#pragma unroll
+                for (int e = 0; e < 4; ++e) {
+                    const uint32_t k = base + 256 * u + e;
+                    w[e] = k < p.ncell ? b.cnt[k] : 0u;
+                    if (k < p.ncell) b.cnt[k] = 0;
+                }
+                v[u] = make_uint4(w[0], w[1], w[2], w[3]);
+            }
+        }
+        uint32_t run = 0;
+#pragma unroll
+        for (int u = 0; u < 4; ++u) {
+            const uint32_t sum = v[u].x + v[u].y + v[u].z + v[u].w;
+            const uint32_t incl = wave_inclusive_dpp(sum);
+            at[u].x = run + incl - sum;
+            at[u].y = at[u].x + v[u].x;
+            at[u].z = at[u].y + v[u].y;
+            at[u].w = at[u].z + v[u].z;
+            run += __builtin_amdgcn_readlane(incl, 63);
+        }
+        uint2 *rel = reinterpret_cast<uint2 *>(b.rel + base);  // whole chunks long
+        const bool wide = run >= kWideOffset;
+#pragma unroll
+        for (int u = 0; u < 4; ++u)
+            rel[64 * u] = wide ? make_uint2(~0u, ~0u)
+                               : make_uint2(at[u].x | at[u].y << 16, at[u].z | at[u].w << 16);
+        if (wide || p.idx_read) {
+#pragma unroll
+            for (int u = 0; u < 4; ++u) {
+                const uint32_t w[4] = {at[u].x, at[u].y, at[u].z, at[u].w};
+#pragma unroll
+                for (int e = 0; e < 4; ++e)
+                    if (base + 256 * u + e < p.ncell) b.idx[1 + base + 256 * u + e] = w[e];
+            }
+        }
+        total = lane == which ? run : total;
+    }
+    if (mine) {
+        b.chunk_sum[c0 + lane] = total;
+        b.chunk_live[c0 + lane] = marked ? kChunkRelative : kChunkEmpty;
+        b.chunk_next[c0 + lane] = 0;
+    }
+}
+
+// Exclusive scan of the chunks' totals into chunk_prefix: the single-pass
+// scan of scan_kernel, a tile of kChunkTile chunks a block.
+__global__ __launch_bounds__(1024) void chunk_scan_kernel(FrameParams p, FrameBuffers b, uint32_t chunks) {
+    constexpr uint32_t kItems = kChunkTile / 1024;
+    __shared__ uint32_t s_prefix;
+    __shared__ uint32_t s_wave[16];
+    const uint32_t lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const uint32_t tile = blockIdx.x;
+    const uint32_t epoch = *b.epoch & kEpochMask;
+    const uint32_t base = tile * kChunkTile + threadIdx.x * kItems;
+    uint32_t v[kItems], mine = 0;
+#pragma unroll
+    for (uint32_t i = 0; i < kItems; ++i) {
+        v[i] = base + i < chunks ? b.chunk_sum[base + i] : 0u;
+        mine += v[i];
+    }
+    const uint32_t incl = wave_inclusive_dpp(mine);
+    if (lane == 63) s_wave[wave] = incl;
+    __syncthreads();
+    uint32_t wave_off = 0, agg = 0;
+#pragma unroll
+    for (uint32_t w = 0; w < 16; ++w) {
+        const uint32_t ws = s_wave[w];
+        if (w < wave) wave_off += ws;
+        agg += ws;
+    }
+    if (wave == 0) {
+        const uint32_t excl = publish_tile(p, b, tile, epoch, agg);
+        if (lane == 0) s_prefix = excl;
+    }
+    __syncthreads();
+    uint32_t run = s_prefix + wave_off + incl - mine;
+#pragma unroll
+    for (uint32_t i = 0; i < kItems; ++i) {
+        if (base + i < chunks) b.chunk_prefix[base + i] = run;
+        run += v[i];
+    }
+    if (tile == 0 && threadIdx.x == 0) b.idx[0] = 0;
+    if (tile == gridDim.x - 1 && threadIdx.x == 0) b.idx[p.ncell + 1] = s_prefix + agg;
+}
+
 // ---------------------------------------------------------------------------
 
 // PER particles per lane (kScatterPerLane), strided across the wavefront: every
 // load of the dependent chain (kslot -> start offset -> destination) is in
 // flight for all of them at once.
-template <int PER>
+// RELATIVE: the offsets are 16 bits from their chunk's prefix
+// (relative_offsets).  A template: with the choice made at run time 4M loose
+// particles took 57 us instead of 45 (whole offsets: 54), and the 1M lattice
+// 12.5 instead of 11.8 where one form of loads serves both.
+template <int PER, bool RELATIVE>
 __global__ __launch_bounds__(kScatterBlock) void scatter_kernel(FrameParams p, FrameBuffers b) {
     // Blocks go to the 8 XCDs in turn (block b to XCD b % 8): block b takes
     // tile (b % 8) * (grid / 8) + b / 8, so that each XCD scatters one
@@ -1609,7 +1812,7 @@ __global__ __launch_bounds__(kScatterBlock) void scatter_kernel(FrameParams p, F
     if (blockIdx.x == 0 && threadIdx.x == 0) *b.epoch = *b.epoch + 1;  // the frame's scan has finished
     uint2 ks[PER];
     float2 q[PER], v[PER];
-    uint32_t start[PER];
+    uint32_t start[PER], prefix[PER];
 #pragma unroll
     for (int j = 0; j < PER; ++j) {
         const uint32_t i = w0 + 64 * j + ln;
@@ -1625,13 +1828,24 @@ __global__ __launch_bounds__(kScatterBlock) void scatter_kernel(FrameParams p, F
     const uint32_t dead = b.error[lane_id() >> 6];
 #pragma unroll
     for (int j = 0; j < PER; ++j)
-        if (w0 + 64 * j + ln < p.n) start[j] = b.idx[ks[j].x + 1];
+        if (w0 + 64 * j + ln < p.n) {
+            if (RELATIVE) {
+                start[j] = reinterpret_cast<const uint16_t *>(b.off)[ks[j].x];
+                prefix[j] = b.chunk_prefix[ks[j].x >> kChunkShift];
+            } else {
+                start[j] = b.idx[ks[j].x + 1];
+            }
+        }
     if (__builtin_amdgcn_readfirstlane(dead)) return;
 #pragma unroll
     for (int j = 0; j < PER; ++j) {
         const uint32_t i = w0 + 64 * j + ln;
         if (i < p.n) {
-            const uint32_t dest = start[j] + (ks[j].y & kSrcMask);
+            uint32_t dest = start[j] + (ks[j].y & kSrcMask);
+            if (RELATIVE) {
+                if (start[j] == kWideOffset) dest = b.idx[ks[j].x + 1] + (ks[j].y & kSrcMask);
+                dest += prefix[j];
+            }
             if (dest < p.n) {  // always, with a consistent frame
                 b.pos[dest] = q[j];
                 b.vel[dest] = v[j];
@@ -1642,16 +1856,25 @@ __global__ __launch_bounds__(kScatterBlock) void scatter_kernel(FrameParams p, F
     }
 }
 
-// Offsets of the chunks the last scan found empty: every entry is the offset
-// at the chunk's first cell.
+// Whole offsets in idx everywhere: an empty chunk's entries become the offset
+// at its first cell, a relative chunk's theirs counted from 0, and it is whole
+// then.
 __global__ __launch_bounds__(256) void materialize_kernel(FrameParams p, FrameBuffers b) {
     const uint32_t chunk = blockIdx.x;
-    if (b.chunk_live[chunk]) return;
+    const uint32_t state = b.chunk_live[chunk];
+    if (state == kChunkWhole) return;
     const uint32_t v = b.chunk_prefix[chunk];
     for (uint32_t i = threadIdx.x; i < kChunkCells; i += 256) {
         const uint32_t c = chunk * kChunkCells + i;
-        if (c < p.ncell) b.idx[1 + c] = v;
+        uint32_t at = 0;
+        if (c < p.ncell && state == kChunkRelative) {
+            at = offset_entry(b, c, offset_word(b, c));
+            if (at == kWideOffset) at = b.idx[1 + c];
+        }
+        if (c < p.ncell) b.idx[1 + c] = v + at;
     }
+    __syncthreads();  // every thread has read the state
+    if (threadIdx.x == 0 && state == kChunkRelative) b.chunk_live[chunk] = kChunkWhole;
 }
 
 __global__ void copy32_kernel(uint32_t *dst, const uint32_t *src, size_t n) {
@@ -1844,7 +2067,9 @@ __global__ __launch_bounds__(256) void upload_scatter_kernel(UploadParams u, Fra
     if (i >= u.n) return;
     const uint2 ks = u.ks[i];
     if (ks.x == 0xffffffffu) return;
-    const uint32_t dest = b.idx[ks.x + 1] + ks.y;
+    uint32_t at = offset_entry(b, ks.x, offset_word(b, ks.x));  // the chunk is live
+    if (b.off_shift) at = wide_entry(b, ks.x, at, kChunkRelative) + b.chunk_prefix[ks.x >> kChunkShift];
+    const uint32_t dest = at + ks.y;
     if (dest >= u.cap) return;  // never, with a consistent scan
     b.pos[dest] = u.pos[i];
     b.vel[dest] = u.vel[i];
@@ -1962,11 +2187,11 @@ __device__ __forceinline__ void stencil_rows(const FrameParams &p, const FrameBu
         const uint32_t k = c[u] < p.ncell ? c[u] : p.ncell - 1;
         live[u] = b.chunk_live[k >> kChunkShift];
         pre[u] = b.chunk_prefix[k >> kChunkShift];
-        at[u] = b.idx[k + 1];
+        at[u] = b.idx[k + 1];  // also on large grids: FrameParams::idx_read
     }
 #pragma unroll
     for (int u = 0; u < 7; ++u) {
-        at[u] = live[u] ? at[u] : pre[u];
+        at[u] = offset_of(at[u], live[u], pre[u]);
         at[u] = c[u] < p.ncell && at[u] < p.n ? at[u] : p.n;
     }
 #pragma unroll
@@ -2743,11 +2968,11 @@ __global__ __launch_bounds__(256, 4) void learn_features_kernel(FrameParams p, F
             const uint32_t v = c[u] < p.ncell ? c[u] : p.ncell - 1;
             live[u] = b.chunk_live[v >> kChunkShift];
             pre[u] = b.chunk_prefix[v >> kChunkShift];
-            at[u] = b.idx[v + 1];
+            at[u] = b.idx[v + 1];  // also on large grids: FrameParams::idx_read
         }
 #pragma unroll
         for (int u = 0; u < 17; ++u) {
-            at[u] = live[u] ? at[u] : pre[u];
+            at[u] = offset_of(at[u], live[u], pre[u]);
             at[u] = c[u] < p.ncell && at[u] < p.n ? at[u] : p.n;
         }
         uint64_t tot5 = 0, tot3 = 0;
@@ -2961,6 +3186,10 @@ hipError_t launch_canonical(const FrameParams &p, const FrameBuffers &b, uint32_
     const uint32_t chunks = (p.ncell + kChunkCells - 1) / kChunkCells;
     const uint32_t blocks = (p.n + kCollideBlock - 1) / kCollideBlock;
     if (chunks + blocks == 0) return hipSuccess;
+    if (relative_offsets(p.ncell)) {  // the particles' blocks read the offsets that the others would make whole
+        const hipError_t e = launch_materialize(p, b, stream);
+        if (e != hipSuccess) return e;
+    }
     hipLaunchKernelGGL(canonical_kernel, dim3(chunks + blocks), dim3(kCollideBlock), 0, stream, p, b, idx_out);
     return hipGetLastError();
 }
@@ -2975,6 +3204,21 @@ static hipError_t launch_scan_as(const FrameParams &p, const FrameBuffers &b, hi
 
 hipError_t launch_scan(const FrameParams &p, const FrameBuffers &b, hipStream_t stream,
                        hipEvent_t start, hipEvent_t stop) {
+    if (relative_offsets(p.ncell)) {
+        const uint32_t chunks = (p.ncell + kChunkCells - 1) / kChunkCells;
+        const uint32_t per = std::min((chunks + kChipWaves - 1) / kChipWaves, kWaveChunks);
+        const uint32_t cells = (chunks + 4 * per - 1) / (4 * per);
+        const uint32_t tiles = (chunks + kChunkTile - 1) / kChunkTile;
+        if (start || stop) {
+            hipExtLaunchKernelGGL(cell_scan_kernel, dim3(cells), dim3(256), 0, stream, start, nullptr, 0, p, b, chunks,
+                                  per);
+            hipExtLaunchKernelGGL(chunk_scan_kernel, dim3(tiles), dim3(1024), 0, stream, nullptr, stop, 0, p, b, chunks);
+        } else {
+            hipLaunchKernelGGL(cell_scan_kernel, dim3(cells), dim3(256), 0, stream, p, b, chunks, per);
+            hipLaunchKernelGGL(chunk_scan_kernel, dim3(tiles), dim3(1024), 0, stream, p, b, chunks);
+        }
+        return hipGetLastError();
+    }
     static_assert(kNumScanShapes == 9, "one case per scan shape");
     switch (b.scan_shape) {
         case 8: return launch_scan_as<8>(p, b, stream, start, stop);
@@ -2995,7 +3239,8 @@ static hipError_t launch_scatter_as(const FrameParams &p, const FrameBuffers &b,
     constexpr int per = kScatterPerLane[S];
     constexpr uint32_t per_block = kScatterBlock * per;
     const uint32_t tiles = (p.n + per_block - 1) / per_block;
-    return launch(scatter_kernel<per>, (tiles + 7) / 8 * 8, kScatterBlock, stream, start, stop, p, b);
+    const auto kernel = relative_offsets(p.ncell) ? scatter_kernel<per, true> : scatter_kernel<per, false>;
+    return launch(kernel, (tiles + 7) / 8 * 8, kScatterBlock, stream, start, stop, p, b);
 }
 
 hipError_t launch_scatter(const FrameParams &p, const FrameBuffers &b, hipStream_t stream,
