@@ -195,3 +195,43 @@ def test_large_grid_with_a_chunk_past_16_bits(oracle, m):
         *ref, st = oracle.step_s(P, *ref, max_passes=1, nsteps=1)
         assert_packed(w.read(), ref, "passes after plain frames")
         assert w.solver_stats() == st
+
+
+@pytest.mark.parametrize("n", [0, 1, 4000, 180_000, 190_000])
+def test_read_through_host_memory_and_by_copies(oracle, n):
+    """Readbacks up to 4 MiB are stored to host memory by the kernel, larger
+    ones copied (here 1.2 MB of offsets, and the pairs of 180,000 and 190,000
+    particles just below and above): all of the triple, parts of it, again
+    without a frame between, and the device's own canonical arrays after it."""
+    rng = np.random.default_rng(n)
+    cfg = WrachConfig(dimensions=(600, 500), cell_size=1, gravity=(0.0, -0.02))
+    say(f"[readback] read of {n}")
+    with World(cfg) as w:
+        done = 0
+        for add in (n // 3, n - n // 3):  # a longer readback each time
+            pos, vel = f32(rng.uniform(0, 500, (add, 2))), f32(rng.uniform(-1, 1, (add, 2)))
+            w.add_particles(pos, vel)
+            done += add
+            got = w.read()
+            assert len(got[1]) == done and got[0][-1] == done
+        if n:
+            w.step(3)
+        first = w.read()
+        P = oracle.params(600, 500, 1, n, gravity=cfg.gravity)
+        want = got if n == 0 else oracle.step(P, *got, nsteps=3)
+        assert_packed(first, want, "read")
+        assert_packed(w.read(), want, "read again")
+        idx, pos, vel = np.zeros(len(want[0]), np.uint32), np.zeros((max(n, 1), 2), np.float32), np.zeros((max(n, 1), 2), np.float32)
+        L, count = _lib.load(), ctypes.c_uint32()
+        f32p, u32p = ctypes.POINTER(ctypes.c_float), ctypes.POINTER(ctypes.c_uint32)
+        assert L.wrach_read(w._h, None, vel.ctypes.data_as(f32p), max(n, 1), None, 0, ctypes.byref(count)) == 0
+        assert L.wrach_read(w._h, pos.ctypes.data_as(f32p), None, max(n, 1), idx.ctypes.data_as(u32p), len(idx), None) == 0
+        assert count.value == n
+        assert_packed((idx, pos[:n], vel[:n]), want, "parts")
+        hip = Hip()
+        view = w.device_state(canonical=True)
+        w.sync()
+        assert np.array_equal(hip.download(ctypes.c_void_p(view.indices), idx), want[0])
+        if n:
+            assert np.array_equal(hip.download(ctypes.c_void_p(view.positions), pos).view(np.uint32),
+                                  want[1].view(np.uint32))

@@ -158,6 +158,16 @@ __device__ __forceinline__ uint32_t cell_key(const FrameParams &p, const Grid &g
     return g.base + ky * g.gx + kx;
 }
 
+// Raises a kErr* bit, for the kernels that follow and for the host, which
+// looks at its words after every wait (they stay raised: the context is
+// dead).  The store is visible there once the kernel has ended.
+__device__ __forceinline__ void raise_error(const FrameBuffers &b, uint32_t bit) {
+    atomicOr(b.error, bit);
+    if (b.error_host)
+        __hip_atomic_store(&b.error_host[bit == kErrLookBack ? 0 : 1], 1u, __ATOMIC_RELAXED,
+                           __HIP_MEMORY_SCOPE_SYSTEM);
+}
+
 // Claims `count` consecutive slots in cell k.  The frame's first claim in a
 // chunk marks it, so that the scan visits only chunks that hold particles.
 __device__ __forceinline__ uint32_t claim(const FrameBuffers &b, uint32_t k, uint32_t count) {
@@ -651,7 +661,7 @@ __global__ __launch_bounds__(kCollideBlock) void collide_kernel(FrameParams p, F
         bad = bad || kbad;
     }
     if (__builtin_amdgcn_readfirstlane(dead)) return;
-    if (bad) atomicOr(b.error, kErrLayout);
+    if (bad) raise_error(b, kErrLayout);
     if (__ballot(work) == 0) return;  // every lane votes; nothing to handle or queue
 
     // Loads: the queued cells' ranges and the handled particles, all windows.
@@ -686,7 +696,7 @@ __global__ __launch_bounds__(kCollideBlock) void collide_kernel(FrameParams p, F
                 qn[j] = qen[j] - qst[j];
                 cls[j] = size_class(qn[j]);
             } else {
-                atomicOr(b.error, kErrLayout);
+                raise_error(b, kErrLayout);
             }
         }
     }
@@ -1475,7 +1485,7 @@ __device__ uint32_t look_back(const FrameParams &p, const FrameBuffers &b, uint3
     epoch = (epoch + p.epoch_skew) & kEpochMask;
     for (uint32_t round = 0;; ++round) {
         if (round >= p.wait_limit) {
-            if (lane == 0) atomicOr(b.error, kErrLookBack);
+            if (lane == 0) raise_error(b, kErrLookBack);
             return 0u;
         }
         unsigned long long w[kLookWindows];
