@@ -229,7 +229,8 @@ typedef struct wrach_tuning {
                                   above 2^23 cells scan without tiles of
                                   this shape; it is kept and reported) */
     uint32_t scatter_per_lane; /* particles per lane of the scatter: 2, 1 or 4 */
-    uint32_t cells_grid;       /* blocks of the queued-cell kernel, 1..4x the default */
+    uint32_t cells_grid;       /* blocks of the queued-cell kernel, 1..4x the default (at most
+                                  particles / 64 + 64 are started) */
     float frame_us;            /* wrach_autotune: the chosen shapes' frame time; else 0 */
 } wrach_tuning;
 

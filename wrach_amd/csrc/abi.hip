@@ -121,7 +121,8 @@ struct wrach_ctx {
     uint2 *srows2 = nullptr;
     uint32_t *sperm = nullptr;   // the separation kernels' lane order (capacity entries)
     // Host memory that kernels store to: buf.error's bits a word each, looked
-    // at after each wait, and a small readback's triple.
+    // at after each wait, and an upload's particles outside the grid
+    // (kOutsideWord); a small readback's triple (stage).
     uint32_t *err_host = nullptr;
     unsigned char *stage = nullptr, *stage_device = nullptr;
     size_t stage_bytes = 0;
@@ -152,6 +153,7 @@ struct wrach_ctx {
 namespace {
 
 constexpr uint32_t kFramesPerGraph = 16;
+constexpr uint32_t kOutsideWord = 2, kHostWords = 3;  // words of wrach_ctx::err_host
 
 void free_graphs(wrach_ctx *c) {
     if (c->graph_one) (void)hipGraphExecDestroy(c->graph_one);
@@ -638,13 +640,13 @@ int add_device_packed(wrach_ctx *c, const float *pos_xy, const float *vel_xy, ui
                                         (int)world, n, c->stream));
     }
     const wrach::UploadParams u = store_params(c, total);
-    uint32_t outside[wrach::kOutsideStripes * wrach::kCtrStride];
-    WRACH_HIP(hipMemsetAsync(c->doutside, 0, sizeof outside, c->stream));
+    WRACH_HIP(hipMemsetAsync(c->doutside, 0, (size_t)wrach::kOutsideStripes * wrach::kCtrStride * sizeof(uint32_t),
+                             c->stream));
     WRACH_HIP(wrach::launch_upload_bin(u, c->buf, c->stream));
-    WRACH_HIP(hipMemcpyAsync(outside, c->doutside, sizeof outside, hipMemcpyDeviceToHost, c->stream));
+    WRACH_HIP(wrach::launch_outside_sum(c->doutside, c->buf.error_host + kOutsideWord, c->stream));
     WRACH_SETTLE(c);
-    uint32_t packed = (uint32_t)total;
-    for (uint32_t t = 0; t < wrach::kOutsideStripes; ++t) packed -= outside[t * wrach::kCtrStride];
+    const volatile uint32_t *words = c->err_host;
+    const uint32_t packed = (uint32_t)total - words[kOutsideWord];
     if (packed > c->capacity) {
         // the counts are the only state touched: clear them for the next frame
         WRACH_HIP(hipMemsetAsync(c->buf.cnt, 0, (c->ncell + 16) * sizeof(uint32_t), c->stream));
@@ -847,8 +849,8 @@ int create_ctx(const wrach_config *cfg, uint32_t n_worlds, const wrach_config *w
     }
     WRACH_HIP_C(dmalloc(&b.epoch, 1));
     WRACH_HIP_C(dmalloc(&b.error, 1));
-    WRACH_HIP_C(hipHostMalloc((void **)&c->err_host, 2 * sizeof(uint32_t), hipHostMallocMapped | hipHostMallocCoherent));
-    c->err_host[0] = c->err_host[1] = 0;
+    WRACH_HIP_C(hipHostMalloc((void **)&c->err_host, kHostWords * sizeof(uint32_t), hipHostMallocMapped | hipHostMallocCoherent));
+    std::memset(c->err_host, 0, kHostWords * sizeof(uint32_t));
     {
         void *device = nullptr;
         WRACH_HIP_C(hipHostGetDevicePointer(&device, c->err_host, 0));

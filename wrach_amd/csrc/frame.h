@@ -247,6 +247,8 @@ struct UploadParams {
 // Cell and slot of every store particle, counts into b.cnt, those outside
 // the grid into u.outside (zeroed by the caller).
 hipError_t launch_upload_bin(const UploadParams &u, const FrameBuffers &b, hipStream_t stream);
+// Their sum, stored to host memory.
+hipError_t launch_outside_sum(const uint32_t *outside, uint32_t *host, hipStream_t stream);
 // The store's particles outside the grid in store order, copied to
 // dpos/dvel from index base on: counts[b] receives block b's number (blocks
 // of 256 store particles), and after the caller has turned them into

@@ -239,19 +239,10 @@ __device__ __forceinline__ unsigned long long lanemask_lt() {
     return (1ull << lane_id()) - 1;
 }
 
-__device__ __forceinline__ uint32_t wave_inclusive_sum(uint32_t v) {
-    const int lane = threadIdx.x & 63;
-#pragma unroll
-    for (int off = 1; off < 64; off <<= 1) {
-        const uint32_t u = __shfl_up(v, off, 64);
-        if (lane >= off) v += u;
-    }
-    return v;
-}
-
 // Inclusive sum over the wavefront by DPP moves (lanes without a source add
-// 0), one instruction a step.
-__device__ __forceinline__ uint32_t wave_inclusive_dpp(uint32_t v) {
+// 0), one instruction a step: it stands in the latency of the scan and of the
+// cell kernel's start, where six shuffles through LDS took 0.4 us a sum.
+__device__ __forceinline__ uint32_t wave_inclusive_sum(uint32_t v) {
 #define WRACH_DPP_ADD(ctrl, rows) \
     v += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, ctrl, rows, 0xf, false)
     WRACH_DPP_ADD(0x111, 0xf);  // row_shr:1, :2, :4, :8
@@ -1070,10 +1061,12 @@ __device__ __forceinline__ void wide_rest(const FrameParams &p, const FrameBuffe
     uint32_t count[9];
 #pragma unroll
     for (int d = 0; d < 9; ++d) count[d] = 0;
+    uint32_t next = kMaxInCell + lane < n ? code[kMaxInCell + lane] : 0u;
 #pragma unroll 1
     for (uint32_t r0 = kMaxInCell; r0 < n; r0 += 64) {
         const uint32_t r = r0 + lane;
-        const uint32_t w = r < n ? code[r] : 0u;
+        const uint32_t w = next;
+        next = r + 64 < n ? code[r + 64] : 0u;
         const uint32_t dir = (w & kRunFlag) ? (w >> 27) & 15u : 10u;
         uint32_t rin = 0;
 #pragma unroll
@@ -1195,9 +1188,18 @@ __host__ __device__ constexpr uint32_t cells_per_item(int k) {
     return k < kGroupClasses ? (32u >> k) : k == kWaveClass ? (uint32_t)kWideCells : 1u;
 }
 
-// Fills the map: wave w takes classes w and w + 4, lane l slice l.
+// Fills the map: wave w takes classes w and w + 4, lane l slice l.  Every
+// block waits for it before its first item, so both classes' counters, their
+// overflow lists' too, are loaded together, and the sums are DPP moves.
 __device__ __forceinline__ void build_item_map(const FrameBuffers &b, ItemMap &m) {
     const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = lane_id();
+    uint32_t fill[2], over[2];
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+        const int k = (int)wave + 4 * h;
+        fill[h] = b.class_ctr[ctr_index(k, (int)lane)];
+        over[h] = b.class_ctr[ctr_index(k, kSlices)];
+    }
 #pragma unroll
     for (int h = 0; h < 2; ++h) {
         const int k = (int)wave + 4 * h;
@@ -1211,12 +1213,12 @@ __device__ __forceinline__ void build_item_map(const FrameBuffers &b, ItemMap &m
             off = k == kk ? b.class_off[kk] : off;
         }
         const uint32_t per = cells_per_item(k);
-        const uint32_t f = min(b.class_ctr[ctr_index(k, (int)lane)], scap);
+        const uint32_t f = min(fill[h], scap);
         const uint32_t incl = wave_inclusive_sum((f + per - 1) / per);
         m.incl[k][lane] = incl;
         m.fill[k][lane] = f;
         if (lane == 63) {
-            const uint32_t fo = min(b.class_ctr[ctr_index(k, kSlices)], ccap);
+            const uint32_t fo = min(over[h], ccap);
             m.fill[k][kSlices] = fo;
             m.in_slices[k] = incl;
             m.items[k] = incl + (fo + per - 1) / per;
@@ -1728,7 +1730,7 @@ __global__ __launch_bounds__(256) void cell_scan_kernel(FrameParams p, FrameBuff
 #pragma unroll
         for (int u = 0; u < 4; ++u) {
             const uint32_t sum = v[u].x + v[u].y + v[u].z + v[u].w;
-            const uint32_t incl = wave_inclusive_dpp(sum);
+            const uint32_t incl = wave_inclusive_sum(sum);
             at[u].x = run + incl - sum;
             at[u].y = at[u].x + v[u].x;
             at[u].z = at[u].y + v[u].y;
@@ -1775,7 +1777,7 @@ __global__ __launch_bounds__(1024) void chunk_scan_kernel(FrameParams p, FrameBu
         v[i] = base + i < chunks ? b.chunk_sum[base + i] : 0u;
         mine += v[i];
     }
-    const uint32_t incl = wave_inclusive_dpp(mine);
+    const uint32_t incl = wave_inclusive_sum(mine);
     if (lane == 63) s_wave[wave] = incl;
     __syncthreads();
     uint32_t wave_off = 0, agg = 0;
@@ -2024,6 +2026,15 @@ __global__ __launch_bounds__(256) void upload_bin_kernel(UploadParams u, FrameBu
     const unsigned long long m = __ballot(i < u.n && !in);
     if (lane_id() == 0 && m != 0)
         atomicAdd(&u.outside[(blockIdx.x % kOutsideStripes) * kCtrStride], (uint32_t)__popcll(m));
+}
+
+// The striped counts' sum, to host memory (a copy of the counters would be
+// the upload's only one to the host).
+__global__ __launch_bounds__(64) void outside_sum_kernel(const uint32_t *outside, uint32_t *host) {
+    static_assert(kOutsideStripes <= 64, "a counter per lane");
+    const uint32_t t = threadIdx.x;
+    const uint32_t sum = wave_sum(t < kOutsideStripes ? outside[t * kCtrStride] : 0u);
+    if (t == 0) __hip_atomic_store(host, sum, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
 }
 
 // The store's particles outside the grid, appended at dpos/dvel[base + ...]
@@ -3173,7 +3184,11 @@ hipError_t launch_collide(const FrameParams &p, const FrameBuffers &b, hipStream
 
 hipError_t launch_cells(const FrameParams &p, const FrameBuffers &b, hipStream_t stream,
                         hipEvent_t start, hipEvent_t stop) {
-    return launch(cells_kernel, b.cells_grid, kCollideBlock, stream, start, stop, p, b);
+    // A small world's cells are few: at most n / 64 + 64 blocks, about what
+    // its particles could need with every list's last item partly filled (16k
+    // particles: 320 of the 1,024 that fit the device; 100 frames 2.33 ms with
+    // all of them, 2.29 with 64 to 320).
+    return launch(cells_kernel, std::min(b.cells_grid, p.n / 64 + 64), kCollideBlock, stream, start, stop, p, b);
 }
 
 // Asked once per device (a frame without a context asks on every call).
@@ -3303,6 +3318,11 @@ hipError_t launch_noalloc_init(const FrameParams &p, const FrameBuffers &b, cons
 hipError_t launch_upload_bin(const UploadParams &u, const FrameBuffers &b, hipStream_t stream) {
     if (u.n == 0) return hipSuccess;
     hipLaunchKernelGGL(upload_bin_kernel, dim3((u.n + 255) / 256), dim3(256), 0, stream, u, b);
+    return hipGetLastError();
+}
+
+hipError_t launch_outside_sum(const uint32_t *outside, uint32_t *host, hipStream_t stream) {
+    hipLaunchKernelGGL(outside_sum_kernel, dim3(1), dim3(64), 0, stream, outside, host);
     return hipGetLastError();
 }
 
