@@ -1,6 +1,6 @@
 // Frame kernels of the particle step, written for gfx950 (wave64).
 //
-// One frame is four launches:
+// One frame is four launches (five on a grid above 2^23 cells):
 //   collide_kernel     one packed particle per lane, 64 consecutive ones per
 //                      wavefront; `key` gives each particle's cell, so a
 //                      cell is a segment of equal keys.  A cell that lies
@@ -27,7 +27,9 @@
 //   scan_kernel        single-pass exclusive scan of the per-cell counts with
 //                      decoupled look-back; writes [0, start_0.., N] and clears
 //                      the counts for the next frame (prefix_sum.wgsl +
-//                      cell.rs:116-131).
+//                      cell.rs:116-131).  Large grids: cell_scan_kernel, each
+//                      chunk of 1,024 cells by itself, and chunk_scan_kernel,
+//                      the chunks' totals.
 //   scatter_kernel     one lane per particle: dest = start[key] + slot
 //                      (pack_new_particle_data.wgsl:39-44); records the source
 //                      index so the next collide pass can rebuild the stable
