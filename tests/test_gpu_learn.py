@@ -341,3 +341,30 @@ def test_features_of_crowds(oracle, crowd, n):
         bad = np.flatnonzero((rows != ref_rows).any(axis=1))
         assert bad.size == 0, f"crowd={crowd} n={n} cs={cs}: {bad.size} rows differ, first {bad[:5]}"
         assert sums == ref_sums, f"crowd={crowd} n={n} cs={cs}"
+
+
+@pytest.mark.parametrize("solver", ["R", "S"])
+def test_features_on_a_grid_above_the_large_scan(oracle, solver):
+    """Offsets counted from their chunks: the features after frames without
+    passes (which leave no 32-bit offsets) and with them, and a frame after."""
+    rng = np.random.default_rng(7)
+    W, H, n = 4098, 2052, 4000
+    say(f"[learn] features, {W + 1} x {H + 1} cells, solver {solver}")
+    pos = np.concatenate([rng.uniform((1, 1), (W - 1, 6), (n, 2)),
+                          rng.uniform((W - 8, H - 8), (W, H), (200, 2))]).astype(np.float32)
+    vel = rng.uniform(-1, 1, pos.shape).astype(np.float32)
+    cfg = WrachConfig(dimensions=(W, H), cell_size=1, gravity=(0.0, -0.1))
+    P = oracle.params(W, H, 1, len(pos), gravity=cfg.gravity)
+    with World(cfg) as w:
+        w.add_particles(pos, vel)
+        if solver == "S":
+            w.set_solver("S", 1)
+        w.step(2)
+        rows, sums = w.learn_features()
+        idx, p, v = w.read()
+        ref_rows, ref_sums = ol.features(P, idx, p, v)
+        assert np.array_equal(rows, ref_rows) and sums == ref_sums
+        w.step(1)
+        want = oracle.step(P, idx, p, v, nsteps=1) if solver == "R" else oracle.step_s(P, idx, p, v, max_passes=1)[:3]
+        for a, b in zip(w.read(), want):
+            assert np.array_equal(a.view(np.uint32), b.view(np.uint32))
