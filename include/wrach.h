@@ -228,7 +228,8 @@ typedef struct wrach_tuning {
                                   cells and at (256, 128) above 2^26 (grids
                                   above 2^23 cells scan without tiles of
                                   this shape; it is kept and reported) */
-    uint32_t scatter_per_lane; /* particles per lane of the scatter: 2, 1 or 4 */
+    uint32_t scatter_per_lane; /* particles per lane of the scatter: 2, 1 or 4; a context starts at
+                                  2, at 1 above 2^23 cells */
     uint32_t cells_grid;       /* blocks of the queued-cell kernel, 1..4x the default (at most
                                   particles / 64 + 64 are started) */
     float frame_us;            /* wrach_autotune: the chosen shapes' frame time; else 0 */

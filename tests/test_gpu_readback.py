@@ -133,6 +133,11 @@ def test_grids_just_above_the_large_scan(oracle, cells):
     with World(cfg) as w:
         w.add_particles(pos, vel)
         assert_packed(w.read(), ref, "upload")
+        for per_lane in (4, 2, 1):  # every scatter of such a grid; 1 is the default
+            w.set_tuning(scatter_per_lane=per_lane)
+            w.step(1)
+            ref = oracle.step(P, *ref, nsteps=1)
+            assert_packed(w.read(), ref, f"{per_lane} a lane")
         for frames in (1, 5):
             w.step(frames)
             assert w.world_settings(0).particles_in_frame_count == len(ref[1])

@@ -783,7 +783,7 @@ int create_ctx(const wrach_config *cfg, uint32_t n_worlds, const wrach_config *w
 
     wrach::FrameBuffers &b = c->buf;
     b.scan_shape = wrach::default_scan_shape(ncell);
-    b.scatter_shape = 0;
+    b.scatter_shape = wrach::default_scatter_shape(ncell);
     b.scan_tiles = wrach::scan_tiles_for((uint32_t)ncell, b.scan_shape);
     // Queued-cell regions: a class of cells holding at least m particles has
     // at most capacity / m cells.  Each class: kSlices slices sharing that

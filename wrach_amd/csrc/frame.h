@@ -160,6 +160,12 @@ constexpr uint32_t kMinScanTile = 4096;  // smallest threads x items above (size
 constexpr int kScatterBlock = 256;
 constexpr int kScatterPerLane[] = {2, 1, 4};
 constexpr int kNumScatterShapes = 3;
+// The scatter shape a context starts with: two particles a lane up to
+// kLargeScanGrid cells, where they have each other's latency to hide, one
+// above, where more wavefronts than fit follow one another.  1,000 frames of
+// the 1M lattice at 1, 2, 4 a lane: 54.2, 53.6, 53.8 ms; 200 frames of the 4M
+// blobs (16.8M cells) 38.9, 39.7, 40.4; 100 of the 512 worlds 61.7, 62.6, 64.1.
+constexpr uint32_t default_scatter_shape(uint64_t ncell) { return relative_offsets(ncell) ? 1u : 0u; }
 constexpr int kMaxInCell = 9;            // cell.rs:29-30
 constexpr int kLdsSort = 2048;           // keys per LDS bitonic sort (block path)
 constexpr int kWavesPerBlock = kCollideBlock / 64;
