@@ -167,14 +167,19 @@ void free_graphs(wrach_ctx *c) {
 // particles on 19k cells after a frame: 53 us with copies, 28 without, of
 // 100,000 (2.1 MB) 150 and 127; of 300,000 479 and 437, not enough for as
 // much memory a world.
-constexpr size_t kStageMost = 4u << 20;
+// Allocated are kStageLeast at least (4 KiB take as long).  New particles of up
+// to that many bytes take the same way in: as fast as copies from pageable
+// memory, without the 6 to 8 ms that the first of those, and now and then a
+// later one, take.  (For 65,000, 1 MB, touching the memory first takes longer
+// than the copies.)
+constexpr size_t kStageMost = 4u << 20, kStageLeast = 1u << 18;
 
 size_t stage_part(size_t bytes) { return (bytes + 255) & ~(size_t)255; }
 
 // At least `bytes` in c->stage (the stream has nothing that writes there).
 int ensure_stage(wrach_ctx *c, size_t bytes) {
     if (c->stage_bytes >= bytes) return WRACH_OK;
-    size_t want = 4096;
+    size_t want = kStageLeast;
     while (want < bytes) want *= 2;
     unsigned char *host = nullptr;
     void *device = nullptr;
@@ -631,10 +636,22 @@ int add_device_packed(wrach_ctx *c, const float *pos_xy, const float *vel_xy, ui
         if (rc) return rc;
     }
     if (n) {
-        WRACH_HIP(hipMemcpyAsync(c->dstore_pos + c->dstore_n, pos_xy, (size_t)n * sizeof(float2),
-                                 hipMemcpyHostToDevice, c->stream));
-        WRACH_HIP(hipMemcpyAsync(c->dstore_vel + c->dstore_n, vel_xy, (size_t)n * sizeof(float2),
-                                 hipMemcpyHostToDevice, c->stream));
+        const size_t bytes = (size_t)n * sizeof(float2), at_vel = stage_part(bytes);
+        if (at_vel + bytes <= kStageLeast) {  // through the readback's host memory (the stream is idle: add_to_world)
+            const int rc = ensure_stage(c, at_vel + bytes);
+            if (rc) return rc;
+            std::memcpy(c->stage, pos_xy, bytes);
+            std::memcpy(c->stage + at_vel, vel_xy, bytes);
+            WRACH_HIP(wrach::launch_copy32(reinterpret_cast<uint32_t *>(c->dstore_pos + c->dstore_n),
+                                           reinterpret_cast<const uint32_t *>(c->stage_device), 2 * (size_t)n,
+                                           c->stream));
+            WRACH_HIP(wrach::launch_copy32(reinterpret_cast<uint32_t *>(c->dstore_vel + c->dstore_n),
+                                           reinterpret_cast<const uint32_t *>(c->stage_device + at_vel), 2 * (size_t)n,
+                                           c->stream));
+        } else {
+            WRACH_HIP(hipMemcpyAsync(c->dstore_pos + c->dstore_n, pos_xy, bytes, hipMemcpyHostToDevice, c->stream));
+            WRACH_HIP(hipMemcpyAsync(c->dstore_vel + c->dstore_n, vel_xy, bytes, hipMemcpyHostToDevice, c->stream));
+        }
         if (c->worlds > 1)
             WRACH_HIP(hipMemsetD32Async(reinterpret_cast<hipDeviceptr_t>(c->dstore_world + c->dstore_n),
                                         (int)world, n, c->stream));
