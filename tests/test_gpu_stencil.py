@@ -419,3 +419,45 @@ def test_stencil_tolerance_at_every_pass(oracle, passes, quiet):
             assert got[0] == st[0] and got[2] == st[2] and got[3][:2] == st[3][:2], f"{got} against {st}"
             if not quiet:
                 assert got == st, f"{got} against {st}"
+
+
+def displaced_triple(oracle, cs, axis, seed):
+    """A packed triple of a sparse world with every third particle moved one
+    cell along `axis`, up and down in turn, inside the grid, its index range
+    left as it was (wrach_load_packed takes each index range as that cell's
+    particles, wherever they lie)."""
+    rng = np.random.default_rng(seed)
+    W, H = 40 * cs, 32 * cs
+    n = 700
+    pos = f32(rng.uniform(1.5 * cs, (W - 1.5 * cs, H - 1.5 * cs), (n, 2)))
+    vel = f32(rng.normal(0, 0.1, (n, 2)))
+    cfg = WrachConfig(dimensions=(W, H), cell_size=cs, gravity=(0.0, -0.1))
+    idx, p, v = oracle.pack(pos, vel, (0, 0, W, H), cs)
+    p = p.copy()
+    p[::6, axis] += np.float32(cs)
+    p[3::6, axis] -= np.float32(cs)
+    return cfg, oracle.params(W, H, cs, n, gravity=cfg.gravity), (idx, p, v)
+
+
+@pytest.mark.parametrize("cs", [1, 3])
+@pytest.mark.parametrize("axis", [0, 1])
+@pytest.mark.parametrize("solver,tol", [("S", 0.0), ("S", 0.2), ("L", 0.0)])
+def test_stencil_particles_beside_their_cell(oracle, cs, axis, solver, tol):
+    """A particle that lies in another row or column than the index range
+    that holds it is met in that range's row by its neighbours and not by
+    itself: the passes, the overlaps before them and the passes that run."""
+    cfg, P, ref = displaced_triple(oracle, cs, axis, 90 + cs)
+    say(f"[stencil] beside their cell: cs={cs} axis={axis} {solver} tol={tol}")
+    with World(cfg) as w:
+        if solver == "L":  # zero weights: no warm start
+            w.learn_set_params(np.zeros(_lib.WRACH_LEARN_PARAMS, np.float32))
+        w.load_packed(*ref)
+        w.set_solver(solver, 3, tol, quiet=True)
+        for frame in range(2):  # the second frame starts with every particle in its cell
+            w.step(1)
+            *ref, st = oracle.step_s(P, *ref, max_passes=3, overlap_tol=tol, nsteps=1)
+            assert_same_state(w.read(), tuple(ref), f"frame {frame}")
+            before, _, ran, sums = w.solver_stats()
+            assert sums[:2] == st[3][:2], f"frame {frame}: {sums} against {st}"
+            if solver == "S":
+                assert (before, ran) == (st[0], st[2]), f"frame {frame}: {before}, {ran} against {st}"

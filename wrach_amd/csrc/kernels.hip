@@ -2496,7 +2496,11 @@ __device__ __forceinline__ PairSums stencil_particle(const float2 *pin, uint32_t
         r.len[1] -= r.half;
     }
     PairSums s;
-    if (__ballot(max(max(r.len[0], r.len[1]), r.len[2]) > kShortRow) == 0) {
+    // The short path leaves out particle i in its own cell's row alone.  Where
+    // a particle lies beside the cell that holds it (a loaded triple may say
+    // so), it is met in another: stencil_long tests every row.
+    const bool beside = (i - r.rs[0] < r.len[0]) | (i - r.rs[2] < r.len[2]);
+    if (__ballot((max(max(r.len[0], r.len[1]), r.len[2]) > kShortRow) | beside) == 0) {
         stencil_short<MOVE, SUMS, HALF>(pin, i, xi, yi, r, list, s);
         return s;
     }
