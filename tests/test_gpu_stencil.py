@@ -461,3 +461,25 @@ def test_stencil_particles_beside_their_cell(oracle, cs, axis, solver, tol):
             assert sums[:2] == st[3][:2], f"frame {frame}: {sums} against {st}"
             if solver == "S":
                 assert (before, ran) == (st[0], st[2]), f"frame {frame}: {before}, {ran} against {st}"
+
+
+@pytest.mark.parametrize("cs", [1, 3])
+@pytest.mark.parametrize("axis", [0, 1])
+@pytest.mark.parametrize("solver", ["S", "L"])
+def test_stencil_closing_measure_beside_their_cell(oracle, cs, axis, solver):
+    """Where a particle lies beside the cell that holds it, a pair need not be
+    met from both sides: the closing measure of such a frame counts each side
+    by itself, and the next frame's each pair once again."""
+    cfg, P, ref = displaced_triple(oracle, cs, axis, 95 + cs)
+    say(f"[stencil] closing measure beside their cell: cs={cs} axis={axis} {solver}")
+    with World(cfg) as w:
+        if solver == "L":
+            w.learn_set_params(np.zeros(_lib.WRACH_LEARN_PARAMS, np.float32))
+        w.load_packed(*ref)
+        w.set_solver(solver, 2)
+        for frame in range(2):
+            w.step(1)
+            *ref, st = oracle.step_s(P, *ref, max_passes=2, nsteps=1)
+            assert_same_state(w.read(), tuple(ref), f"frame {frame}")
+            _, after, _, sums = w.solver_stats()
+            assert (after, sums) == (st[1], st[3]), f"frame {frame}: {after}, {sums} against {st}"

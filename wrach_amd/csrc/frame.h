@@ -294,11 +294,13 @@ constexpr uint32_t kStencilSumEntries = kStencilSumSets * kStencilSumSlots * kSt
 // frame-start positions (the warm start left more mean overlap than it
 // found), else 0.
 constexpr uint32_t kFallbackWord = kMaxStencilPasses + 1;
-// words[kOverBudgetWord]: nonzero once a stencil kernel of the frame has met
-// a particle whose 3x3 cells hold more than kStencilBudget particles (the
+// words[kOneSidedWord]: nonzero once a stencil kernel of the frame has met a
+// particle whose pairs need not be met from both sides: its 3x3 cells hold
+// more than kStencilBudget particles, or it lies beside the cell that holds it
+// (in a loaded triple; the frames leave every particle in its cell).  The
 // cells are the frame start's, so the frame's first pass or measure finds
-// every such particle).
-constexpr uint32_t kOverBudgetWord = kMaxStencilPasses + 2;
+// every such particle.
+constexpr uint32_t kOneSidedWord = kMaxStencilPasses + 2;
 constexpr float kOverlapScale = 16777216.0f;  // 2^24
 // Crowded cells (kCrowdMin..kCrowdMax particles): the separation kernels'
 // lanes take their particles in order of x (the lane order; the results
@@ -342,8 +344,9 @@ struct StencilArgs {
     // A measure after a pass or measure of the frame: each pair from one
     // side only (the particle's own cell past it, the cell to its right and
     // the three cells above), the pair count and overlap sum doubled, unless
-    // words[kOverBudgetWord] is set (a particle over the budget takes no
-    // pair from its own side, so the two sides differ).
+    // words[kOneSidedWord] is set (a particle over the budget takes no pair
+    // from its own side, one beside its cell is met where it is held and not
+    // where it lies, so the two sides differ).
     uint32_t half;
 };
 hipError_t launch_stencil_measure(const FrameParams &p, const FrameBuffers &b, const StencilArgs &a,

@@ -2605,11 +2605,13 @@ __device__ __forceinline__ StencilRows stencil_lane(const FrameParams &p, const 
     i = a.perm ? a.perm[t] : t;
     q = a.pin[i];
     const uint32_t k = a.rows_from == kRowsOfCell ? a.cell[i] : cell_key(p, particle_grid(p, b, i), q.x, q.y);
+    bool one_sided = a.rows_from == kRowsOfPosition && k != b.key[i];
     if (k < p.ncell) {
         bool over;
         r = stencil_rows_of(p, b, k, over);
-        if (over) atomicOr(&a.words[kOverBudgetWord], 1u);
+        one_sided |= over;
     }
+    if (one_sided) atomicOr(&a.words[kOneSidedWord], 1u);
     if (a.rows_from == kRowsOfPosition && !a.record) a.cell[i] = k;
     if (a.record) {
         a.rows[t] = make_uint4(r.rs[0], r.rs[1], r.rs[2], r.len[0] | (r.half << 16));
@@ -2683,7 +2685,7 @@ __global__ __launch_bounds__(256, 8) void stencil_measure_kernel(FrameParams p, 
     float2 q;
     const StencilRows r = stencil_lane(p, b, a, i, q);
     if (a.pout && a.pout != a.pin && i < p.n) a.pout[i] = q;
-    const bool half = a.half && a.words[kOverBudgetWord] == 0;  // the whole grid alike
+    const bool half = a.half && a.words[kOneSidedWord] == 0;  // the whole grid alike
     float2 *list = s_list + threadIdx.x;
     const PairSums s = half ? (a.stat ? stencil_particle<false, true, true>(a.pin, i, q.x, q.y, r, list)
                                       : stencil_particle<false, false, true>(a.pin, i, q.x, q.y, r, list))
@@ -3029,7 +3031,7 @@ __global__ __launch_bounds__(256, 4) void learn_features_kernel(FrameParams p, F
         r3.half = over ? 0u : min(max(r3.rs[1], at[16]), re1) - r3.rs[1];
         if (over) r3.len[0] = r3.len[1] = r3.len[2] = 0;
         // What the passes that follow need (stencil_lane).
-        if (a.words && over) atomicOr(&a.words[kOverBudgetWord], 1u);
+        if (a.words && (over || k != b.key[i])) atomicOr(&a.words[kOneSidedWord], 1u);
         if (a.rows) {
             a.rows[lane_t] = make_uint4(r3.rs[0], r3.rs[1], r3.rs[2], r3.len[0] | (r3.half << 16));
             a.rows2[lane_t] = make_uint2(r3.len[1] | (r3.len[2] << 16), i);
