@@ -10,6 +10,7 @@ positions and velocities bit for bit, and the overlap statistics equal.
 import numpy as np
 import pytest
 
+from oracle import learn as learn_oracle
 from wrach_amd import World, WrachConfig, WrachError, workloads
 from wrach_amd import _lib
 from tests.test_gpu_parity import _batch_worlds, assert_same_state, f32, oracle_world, say
@@ -476,6 +477,43 @@ def test_stencil_closing_measure_beside_their_cell(oracle, cs, axis, solver):
         if solver == "L":
             w.learn_set_params(np.zeros(_lib.WRACH_LEARN_PARAMS, np.float32))
         w.load_packed(*ref)
+        w.set_solver(solver, 2)
+        for frame in range(2):
+            w.step(1)
+            *ref, st = oracle.step_s(P, *ref, max_passes=2, nsteps=1)
+            assert_same_state(w.read(), tuple(ref), f"frame {frame}")
+            _, after, _, sums = w.solver_stats()
+            assert (after, sums) == (st[1], st[3]), f"frame {frame}: {after}, {sums} against {st}"
+
+
+@pytest.mark.parametrize("cs", [1, 3])
+@pytest.mark.parametrize("solver", ["S", "L"])
+def test_stencil_particles_outside_the_grid(oracle, cs, solver):
+    """Particles of a loaded triple that lie outside the grid, past each of
+    its sides: they have no cell and so no neighbours of their own (the pass
+    leaves them, their feature rows are empty), while the cell that holds them
+    counts them; the step's walls then bring them in."""
+    cfg, P, (idx, p, v) = displaced_triple(oracle, cs, 0, 97 + cs)
+    W, H = cfg.dimensions
+    # (An infinite feature makes a network of zeros answer NaN: 0 times infinity.)
+    infinite = [(np.inf, 6.5), (5.5, -np.inf)] if solver == "S" else []
+    p = p.copy()
+    for k, (x, y) in enumerate([(-0.25, 5.5), (-3.0 * cs, 9.5), (5.5, -0.25), (7.5, -2.5 * cs), (W + cs + 0.5, 3.5),
+                                (W + 9.0 * cs, 4.5), (6.5, H + cs + 0.5), (8.5, H + 8.0 * cs), (-0.5, -0.5),
+                                (W + 2.0 * cs, H + 2.0 * cs)] + infinite):
+        p[20 + 7 * k] = (x, y)
+        p[400 + 7 * k] = (x + 0.25, y + 0.25) if x > 0 and y > 0 else (x - 0.25, y - 0.25)
+    ref = (idx, p, v)
+    say(f"[stencil] outside the grid: cs={cs} {solver}")
+    with World(cfg) as w:
+        if solver == "L":
+            w.learn_set_params(np.zeros(_lib.WRACH_LEARN_PARAMS, np.float32))
+        w.load_packed(*ref)
+        rows, sums = w.learn_features()
+        ref_rows, ref_sums = learn_oracle.features(P, *ref)
+        bad = np.flatnonzero((rows != ref_rows).any(axis=1))
+        assert bad.size == 0, f"{bad.size} rows differ, first {bad[:5]}"
+        assert sums == ref_sums
         w.set_solver(solver, 2)
         for frame in range(2):
             w.step(1)

@@ -102,9 +102,7 @@ __device__ __forceinline__ void finish_particle(const FrameParams &p, const Grid
 // ax = 0 and x1 = W, and the division is monotonic, so the key lies in
 // [0, gx - 1] (gx - 1 = floor(W / cs) on the host, the same f32 division);
 // the max only maps a NaN position, which no upload lets in, to column 0.
-__device__ __forceinline__ void cell_xy(const FrameParams &p, float x, float y, uint32_t &kx,
-                                        uint32_t &ky) {
-    float fx, fy;
+__device__ __forceinline__ void cell_floor(const FrameParams &p, float x, float y, float &fx, float &fy) {
     if (p.cs == 1.0f) {  // x / 1 is exact: skip the division sequence
         fx = floorf(x - p.ax);
         fy = floorf(y - p.ay);
@@ -112,6 +110,12 @@ __device__ __forceinline__ void cell_xy(const FrameParams &p, float x, float y, 
         fx = floorf((x - p.ax) / p.cs);
         fy = floorf((y - p.ay) / p.cs);
     }
+}
+
+__device__ __forceinline__ void cell_xy(const FrameParams &p, float x, float y, uint32_t &kx,
+                                        uint32_t &ky) {
+    float fx, fy;
+    cell_floor(p, x, y, fx, fy);
     kx = (uint32_t)fmaxf(fx, 0.0f);
     ky = (uint32_t)fmaxf(fy, 0.0f);
 }
@@ -154,10 +158,15 @@ __device__ __forceinline__ void cell_coords(const Grid &g, uint32_t c, uint32_t 
     cx = l - cy * g.gx;
 }
 
-__device__ __forceinline__ uint32_t cell_key(const FrameParams &p, const Grid &g, float x, float y) {
-    uint32_t kx, ky;
-    cell_xy(p, x, y, kx, ky);
-    return g.base + ky * g.gx + kx;
+constexpr uint32_t kNoKey = 0xffffffffu;  // no cell; cell keys stay below 2^31
+
+// The cell of any position, kNoKey outside the grid: before a frame's step a
+// loaded triple's particles may lie anywhere.
+__device__ __forceinline__ uint32_t position_key(const FrameParams &p, const Grid &g, float x, float y) {
+    float fx, fy;
+    cell_floor(p, x, y, fx, fy);
+    if (!(fx >= 0.0f && fy >= 0.0f && fx < (float)g.gx && fy < (float)g.gy)) return kNoKey;
+    return g.base + (uint32_t)fy * g.gx + (uint32_t)fx;
 }
 
 // Raises a kErr* bit, for the kernels that follow and for the host, which
@@ -559,7 +568,6 @@ __device__ __forceinline__ void collide_group(float &x, float &y, uint32_t r, ui
 //    wavefront that queued it.  The kernel has no barrier: a wavefront with
 //    nothing to handle or queue returns after the keys, and queued cells go
 //    to their lists with one atomic each (slice = wavefront % kSlices).
-constexpr uint32_t kNoKey = 0xffffffffu;  // past the particles; cell keys stay below 2^31
 constexpr uint32_t kInWaveMax = 3;
 
 // Reductions of a wavefront into lane 63 by DPP moves (one instruction a
@@ -2604,7 +2612,7 @@ __device__ __forceinline__ StencilRows stencil_lane(const FrameParams &p, const 
     }
     i = a.perm ? a.perm[t] : t;
     q = a.pin[i];
-    const uint32_t k = a.rows_from == kRowsOfCell ? a.cell[i] : cell_key(p, particle_grid(p, b, i), q.x, q.y);
+    const uint32_t k = a.rows_from == kRowsOfCell ? a.cell[i] : position_key(p, particle_grid(p, b, i), q.x, q.y);
     bool one_sided = a.rows_from == kRowsOfPosition && k != b.key[i];
     if (k < p.ncell) {
         bool over;
@@ -2975,8 +2983,9 @@ __global__ __launch_bounds__(256, 4) void learn_features_kernel(FrameParams p, F
     if (on) {
         const Grid g = particle_grid(p, b, i);
         uint32_t ucx, ucy;
-        const uint32_t k = cell_key(p, g, q.x, q.y);
-        cell_coords(g, k, ucx, ucy);
+        const uint32_t k = position_key(p, g, q.x, q.y);
+        const bool cell = k != kNoKey;  // outside the grid: no candidates, a row of zeros
+        cell_coords(g, cell ? k : g.base, ucx, ucy);
         const int cx = (int)ucx, cy = (int)ucy;
         const int gx = (int)g.gx, gy = (int)g.gy;
         // Per row of the 5x5 cells, its first cell and the one past its last;
@@ -3013,7 +3022,7 @@ __global__ __launch_bounds__(256, 4) void learn_features_kernel(FrameParams p, F
 #pragma unroll
         for (int t = 0; t < 5; ++t) {
             const int y = cy + t - 2;
-            const bool in = y >= 0 && y < gy;  // the world's own rows only
+            const bool in = cell && y >= 0 && y < gy;  // the world's own rows only
             rs[t] = in ? at[2 * t] : 0u;
             const uint32_t re = in && at[2 * t + 1] > at[2 * t] ? at[2 * t + 1] : rs[t];
             cum[t] = (uint32_t)tot5;
