@@ -339,6 +339,11 @@ int wrach_prepare(wrach_ctx *ctx, uint32_t nframes);
  * frames that follow stay in bounds.  Production code never calls this. */
 int wrach_test_scan_wait(wrach_ctx *ctx, uint32_t wait_limit, uint32_t epoch_skew);
 
+/* Testing hook for small readbacks and uploads where no pinned host memory
+ * can be had (no counterpart in the reference): from here on the context
+ * gets none, and they copy.  Production code never calls this. */
+int wrach_test_no_staging(wrach_ctx *ctx);
+
 /* Self-check of the separation passes' pair arithmetic on one device (no
  * counterpart in the reference).  Modes S and L take the root of a squared
  * distance x in [2^-96, 1 + 2^-23] and the force (1 - d) * 2^29 / d for d

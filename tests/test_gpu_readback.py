@@ -240,3 +240,31 @@ def test_read_through_host_memory_and_by_copies(oracle, n):
         if n:
             assert np.array_equal(hip.download(ctypes.c_void_p(view.positions), pos).view(np.uint32),
                                   want[1].view(np.uint32))
+
+
+@pytest.mark.parametrize("n", [0, 1, 4000, 16384])
+def test_small_transfers_without_pinned_memory(oracle, n):
+    """Uploads and readbacks small enough for pinned host memory, where there
+    is none: before any, and after some was in use."""
+    rng = np.random.default_rng(50 + n)
+    cfg = WrachConfig(dimensions=(160, 128), cell_size=1, gravity=(0.0, -0.1))
+    pos, vel = f32(rng.uniform(0, (160, 128), (n, 2))), f32(rng.uniform(-1, 1, (n, 2)))
+    more, still = f32(rng.uniform(0, 100, (50, 2))), np.zeros((50, 2), np.float32)
+    P, ref = oracle_world(oracle, cfg, pos, vel)
+    say(f"[readback] without pinned memory, {n}")
+    for used in (False, True):
+        with World(cfg) as w:
+            if used:
+                w.add_particles(pos, vel)
+                assert_packed(w.read(), ref, "with pinned memory")
+                w.test_no_staging()
+            else:
+                w.test_no_staging()
+                w.add_particles(pos, vel)
+            assert_packed(w.read(), ref, f"used={used}")
+            if n:
+                w.step(2)
+                assert_packed(w.read(), oracle.step(P, *ref, nsteps=2), f"used={used}, after 2 frames")
+            w.add_particles(more, still)
+            assert_packed(w.read(), packed_by_the_oracle(oracle, cfg, np.concatenate([pos, more]),
+                                                         np.concatenate([vel, still])), f"used={used}, appended")

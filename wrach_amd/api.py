@@ -180,6 +180,11 @@ class World:
         an epoch skew that makes every look-back give up."""
         check(self._L.wrach_test_scan_wait(self._h, int(wait_limit), int(epoch_skew)))
 
+    def test_no_staging(self) -> None:
+        """Testing hook (wrach_test_no_staging): no pinned host memory for
+        readbacks and uploads from here on."""
+        check(self._L.wrach_test_no_staging(self._h))
+
     _TUNING = ("scan_threads", "scan_items", "scatter_per_lane", "cells_grid", "frame_us")
 
     def tuning(self) -> dict:

@@ -126,6 +126,7 @@ struct wrach_ctx {
     uint32_t *err_host = nullptr;
     unsigned char *stage = nullptr, *stage_device = nullptr;
     size_t stage_bytes = 0;
+    bool stage_refused = false;  // wrach_test_no_staging
     // The learned warm start (wrach_learn_*, WRACH_SOLVER_L): the network's
     // master parameters, gradient and Adam moments (f32, wrach::kParams
     // each), its packed weights, the frame's feature rows and a third
@@ -176,24 +177,26 @@ constexpr size_t kStageMost = 4u << 20, kStageLeast = 1u << 18;
 
 size_t stage_part(size_t bytes) { return (bytes + 255) & ~(size_t)255; }
 
-// At least `bytes` in c->stage (the stream has nothing that writes there).
-int ensure_stage(wrach_ctx *c, size_t bytes) {
-    if (c->stage_bytes >= bytes) return WRACH_OK;
+// Whether c->stage holds at least `bytes` (the stream has nothing that writes
+// there).  Where there is no such memory the callers copy.
+bool ensure_stage(wrach_ctx *c, size_t bytes) {
+    if (c->stage_bytes >= bytes) return true;
     size_t want = kStageLeast;
     while (want < bytes) want *= 2;
     unsigned char *host = nullptr;
     void *device = nullptr;
-    WRACH_HIP(hipHostMalloc((void **)&host, want, hipHostMallocMapped | hipHostMallocCoherent));
-    const hipError_t e = hipHostGetDevicePointer(&device, host, 0);
-    if (e != hipSuccess) {
-        (void)hipHostFree(host);
-        return fail(WRACH_E_DEVICE, std::string("staging memory: ") + hipGetErrorString(e));
+    if (c->stage_refused ||
+        hipHostMalloc((void **)&host, want, hipHostMallocMapped | hipHostMallocCoherent) != hipSuccess ||
+        hipHostGetDevicePointer(&device, host, 0) != hipSuccess) {
+        (void)hipGetLastError();
+        if (host) (void)hipHostFree(host);
+        return false;
     }
     if (c->stage) (void)hipHostFree(c->stage);
     c->stage = host;
     c->stage_device = static_cast<unsigned char *>(device);
     c->stage_bytes = want;
-    return WRACH_OK;
+    return true;
 }
 
 // Synchronises the stream and reports a wait a kernel gave up
@@ -637,9 +640,8 @@ int add_device_packed(wrach_ctx *c, const float *pos_xy, const float *vel_xy, ui
     }
     if (n) {
         const size_t bytes = (size_t)n * sizeof(float2), at_vel = stage_part(bytes);
-        if (at_vel + bytes <= kStageLeast) {  // through the readback's host memory (the stream is idle: add_to_world)
-            const int rc = ensure_stage(c, at_vel + bytes);
-            if (rc) return rc;
+        // Through the readback's host memory (the stream is idle: add_to_world).
+        if (at_vel + bytes <= kStageLeast && ensure_stage(c, at_vel + bytes)) {
             std::memcpy(c->stage, pos_xy, bytes);
             std::memcpy(c->stage + at_vel, vel_xy, bytes);
             WRACH_HIP(wrach::launch_copy32(reinterpret_cast<uint32_t *>(c->dstore_pos + c->dstore_n),
@@ -1013,6 +1015,17 @@ int wrach_test_scan_wait(wrach_ctx *c, uint32_t wait_limit, uint32_t epoch_skew)
     free_graphs(c);  // the graphs hold the frame parameters by value
     c->fp.wait_limit = wait_limit;
     c->fp.epoch_skew = epoch_skew;
+    return WRACH_OK;
+}
+
+int wrach_test_no_staging(wrach_ctx *c) {
+    if (!c) return fail(WRACH_E_INVALID, "null context");
+    WRACH_HIP(hipSetDevice(c->cfg.device));
+    WRACH_SETTLE(c);
+    if (c->stage) (void)hipHostFree(c->stage);
+    c->stage = c->stage_device = nullptr;
+    c->stage_bytes = 0;
+    c->stage_refused = true;
     return WRACH_OK;
 }
 
@@ -1709,10 +1722,8 @@ int wrach_read(wrach_ctx *c, float *pos_xy, float *vel_xy, size_t particle_cap,
     const size_t nidx = c->ncell + 2, at_pos = stage_part(nidx * sizeof(uint32_t));
     const size_t at_vel = at_pos + stage_part((size_t)n * sizeof(float2));
     const size_t staged = at_vel + (size_t)n * sizeof(float2);
-    if (staged <= kStageMost) {  // the state's own arrays stay as they are
-        WRACH_HIP(hipSetDevice(c->cfg.device));
-        const int rc = ensure_stage(c, staged);
-        if (rc) return rc;
+    WRACH_HIP(hipSetDevice(c->cfg.device));
+    if (staged <= kStageMost && ensure_stage(c, staged)) {  // the state's own arrays stay as they are
         wrach::FrameBuffers out = c->buf;
         out.pos_out = reinterpret_cast<float2 *>(c->stage_device + at_pos);
         out.vel_out = reinterpret_cast<float2 *>(c->stage_device + at_vel);
