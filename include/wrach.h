@@ -461,8 +461,9 @@ int wrach_learn_profile(wrach_ctx *ctx, uint32_t reps, double *ms);
  * triple the caller holds in device memory and that is replaced in place:
  * indices (grid cells + 2 offsets, the layout of wrach_read), pos_xy and
  * vel_xy (2n floats each).  ws gives the view, grid, cell size and
- * particles_in_frame_count (= n); gravity and dt as in wrach_config.  The
- * frames' other buffers live in one device array of
+ * particles_in_frame_count (= n); gravity and dt as in wrach_config.  A
+ * triple whose offsets do not ascend from indices[1] = 0 to n stays as it is
+ * (the call has returned by then).  The frames' other buffers live in one device array of
  * WRACH_NOALLOC_SCRATCH_BYTES per GPU that the library holds until the
  * process ends; a frame that needs more (about 8 bytes per cell plus 96 per
  * particle) returns WRACH_E_CAPACITY before any work.  Asynchronous on

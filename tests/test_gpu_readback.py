@@ -268,3 +268,56 @@ def test_small_transfers_without_pinned_memory(oracle, n):
             w.add_particles(more, still)
             assert_packed(w.read(), packed_by_the_oracle(oracle, cfg, np.concatenate([pos, more]),
                                                          np.concatenate([vel, still])), f"used={used}, appended")
+
+
+@pytest.mark.parametrize("offset", [0, 4])
+@pytest.mark.parametrize("fault", ["start", "end", "past", "descends", "alternates", "last cell", "none filled"])
+def test_noalloc_frame_leaves_a_bad_triple(oracle, fault, offset):
+    """Offsets that do not ascend from 0 to n: the call's kernels find it and
+    the caller's arrays stay as they were; the next call, on the good triple,
+    is the frame."""
+    hip = Hip()
+    rng = np.random.default_rng(60)
+    n, W, H = 5000, 90, 70
+    cfg = WrachConfig(dimensions=(W, H), cell_size=1, gravity=(0.0, -0.1))
+    pos = f32(np.concatenate([rng.uniform((3, 3), (3.99, 3.99), (1500, 2)), rng.uniform(0, (W, H), (n - 1500, 2))]))
+    vel = f32(rng.uniform(-1, 1, (n, 2)))
+    idx, pos, vel = packed_by_the_oracle(oracle, cfg, pos, vel)
+    ws = _lib.WorldSettingsC()
+    ws.view_dimensions[:] = [float(W), float(H)]
+    ws.view_anchor[:] = [0.0, 0.0]
+    ws.grid_dimensions[:] = [W + 1, H + 1]
+    ws.cell_size = 1
+    ws.particles_in_frame_count = n
+    bad = idx.copy()
+    if fault == "start":
+        bad[1] = 1
+    elif fault == "end":
+        bad[-1] = n - 1
+    elif fault == "past":
+        bad[-40:] = n + 7
+    elif fault == "descends":
+        bad[len(bad) // 2] = 0
+    elif fault == "alternates":  # every second cell's range is all of them
+        bad[1::2], bad[2::2] = 0, n
+    elif fault == "last cell":
+        bad[-2] = n + 1
+    else:
+        bad[:] = 0
+    g = (ctypes.c_float * 2)(*cfg.gravity)
+    skip = offset // 4
+    flat = [np.concatenate([np.zeros(skip, np.float32), a.ravel()]) for a in (pos, vel)]
+    say(f"[readback] noalloc, bad offsets: {fault}, offset {offset}")
+    for _ in range(2):
+        for offsets, want in ((bad, (bad, pos, vel)),
+                              (idx, oracle.step(oracle.params(W, H, 1, n, gravity=cfg.gravity), idx, pos, vel))):
+            di, dp, dv = (hip.upload(a) for a in (offsets, *flat))
+            try:
+                assert _lib.load().wrach_frame_noalloc(ctypes.byref(ws), g, 1.0, di, dp.value + offset,
+                                                       dv.value + offset, n, None) == 0
+                assert hip.h.hipDeviceSynchronize() == 0
+                got = (hip.download(di, offsets), hip.download(dp, flat[0])[skip:].reshape(-1, 2),
+                       hip.download(dv, flat[1])[skip:].reshape(-1, 2))
+                assert_packed(got, want, f"{fault} offset={offset} {'bad' if offsets is bad else 'good'}")
+            finally:
+                hip.free(di, dp, dv)

@@ -2318,6 +2318,9 @@ namespace {
 constexpr size_t kNoAllocBytes = WRACH_NOALLOC_SCRATCH_BYTES;
 constexpr int kNoAllocDevices = 64;
 static __device__ __align__(256) unsigned char scratch[kNoAllocBytes];
+// Every cell takes an offset and a count of it: no grid that fits scans by
+// chunks, whose buffers (rel, chunk_sum) carve_noalloc does not make.
+static_assert(kNoAllocBytes / (2 * sizeof(uint32_t)) <= wrach::kLargeScanGrid, "grids of the scratch array");
 
 std::mutex g_scratch_mu;
 void *g_scratch_ptr[kNoAllocDevices] = {};
@@ -2350,6 +2353,10 @@ size_t carve_noalloc(unsigned char *base, uint32_t n, uint64_t ncell, wrach::Fra
         return p;
     };
     const size_t np = n ? n : 1;
+    // First, so that they lie where the last call left them: zero, as they
+    // were loaded (see canonical_kernel).
+    b.error = reinterpret_cast<uint32_t *>(take(2 * sizeof(uint32_t)));
+    b.error_seen = b.error ? b.error + 1 : nullptr;
     b.idx = reinterpret_cast<uint32_t *>(take((ncell + 2 + 64) * sizeof(uint32_t)));
     if (b.idx) b.idx += 3;  // &idx[1] on a 16-byte boundary
     b.off = b.idx ? b.idx + 1 : nullptr;
@@ -2371,7 +2378,6 @@ size_t carve_noalloc(unsigned char *base, uint32_t n, uint64_t ncell, wrach::Fra
     b.chunk_live = take(chunks);
     b.chunk_prefix = reinterpret_cast<uint32_t *>(take(chunks * sizeof(uint32_t)));
     b.epoch = reinterpret_cast<uint32_t *>(take(sizeof(uint32_t)));
-    b.error = reinterpret_cast<uint32_t *>(take(sizeof(uint32_t)));
     b.class_ctr = reinterpret_cast<uint32_t *>(take(wrach::kCtrWords * sizeof(uint32_t)));
     ncells_total = 0;
     for (int k = 0; k < wrach::kClasses; ++k) {
@@ -2454,6 +2460,7 @@ int wrach_frame_noalloc(const wrach_world_settings *ws, const float gravity[2], 
     wrach::FrameBuffers in = b, out = b;
     in.idx = indices;
     in.off = indices + 1;
+    out.keep_dead = aligned ? 0u : 1u;  // the copies out replace the caller's pairs either way
     if (aligned) {
         in.pos = out.pos_out = reinterpret_cast<float2 *>(pos_xy);
         in.vel = out.vel_out = reinterpret_cast<float2 *>(vel_xy);

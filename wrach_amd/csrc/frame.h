@@ -96,6 +96,10 @@ struct FrameBuffers {
     uint32_t *epoch;      // frame counter tagging the scan's status words; the scatter advances it
     uint32_t *error;      // kErr* bits raised by a kernel that gave up a wait; zero otherwise
     uint32_t *error_host; // host memory: set to 1 with kErrLookBack, kErrLayout (null: nobody looks)
+    // A frame without a context (else null): the error ends with it.  A count
+    // of the canonical kernel's blocks that have seen it; the last clears both.
+    uint32_t *error_seen;
+    uint32_t keep_dead;   // such a frame: with an error, its output is its input's copy (pos, vel)
     uint4 *cells;         // queued cells (s, n, cell, 0), one region per size class
     uint32_t *class_ctr;  // fill of every slice and overflow list (ctr_index); reset by the scan
     uint32_t class_off[8];  // first entry of each class's region in `cells`

@@ -1403,6 +1403,20 @@ __global__ __launch_bounds__(kCollideBlock) void canonical_kernel(FrameParams p,
     __shared__ unsigned long long sk[kLdsSort];
     __shared__ uint2 s_big;
     const uint32_t blocks = (p.n + kCollideBlock - 1) / kCollideBlock;
+    if (*b.error) {  // raised before this kernel, if at all: no offsets are read, none are written
+        if (!b.error_seen) return;
+        const uint32_t i = blockIdx.x * kCollideBlock + threadIdx.x;
+        if (b.keep_dead && i < p.n) {
+            b.pos_out[i] = b.pos[i];
+            b.vel_out[i] = b.vel[i];
+        }
+        __syncthreads();
+        if (threadIdx.x == 0 && atomicAdd(b.error_seen, 1u) == gridDim.x - 1) {
+            *b.error_seen = 0;
+            *b.error = 0;
+        }
+        return;
+    }
     if (blockIdx.x >= blocks) {
         const uint32_t chunk = blockIdx.x - blocks;
         const bool live = b.chunk_live[chunk] != 0;
@@ -1420,7 +1434,6 @@ __global__ __launch_bounds__(kCollideBlock) void canonical_kernel(FrameParams p,
         }
         return;
     }
-    if (*b.error) return;  // a dead context's offsets are not read
     if (threadIdx.x == 0) s_big = make_uint2(0, 0);
     __syncthreads();
     const uint32_t lane = lane_id();
@@ -1947,13 +1960,28 @@ __global__ void keys_from_offsets_kernel(const uint32_t *idx, uint32_t ncell, ui
 // the buffers that a context keeps clean between frames, cleared, and each
 // particle's source index and cell from the caller's offsets.  One thread
 // per cell, a cell of more than kOwnCells particles by its whole wavefront.
+// Offsets that do not ascend from 0 to n are an error: the kernels that follow
+// do nothing and the caller's arrays stay as they are.  (b.error is clear: the
+// canonical kernel clears what a call raised.)  Such ranges may overlap, so
+// one of more than kLongCell particles looks now and then whether another
+// thread has found them wrong.
 // One launch in place of 12 (nine fills, a copy, an iota and a binary search
 // per particle), each 1.3 to 7 us and 2.7 us of the host's time.
 __global__ __launch_bounds__(256) void noalloc_init_kernel(FrameParams p, FrameBuffers b,
                                                            const uint32_t *indices, uint32_t tiles,
                                                            uint32_t chunks) {
-    constexpr uint32_t kOwnCells = 8;
+    constexpr uint32_t kOwnCells = 8, kLongCell = 1024;
     const uint32_t t = blockIdx.x * 256 + threadIdx.x, all = gridDim.x * 256;
+    uint32_t s = 0, e = 0;
+    bool bad = false;
+    if (t < p.ncell) {  // the grid covers the cells
+        s = indices[1 + t];
+        e = indices[2 + t];
+        bad = e < s || e > p.n || (t == 0 && s != 0) || (t == p.ncell - 1 && e != p.n);
+    }
+    const unsigned long long any = __ballot(bad);
+    if (any && lane_id() == (uint32_t)__builtin_ctzll(any)) raise_error(b, kErrLayout);
+    const uint32_t n = bad ? 0u : e - s;
     for (uint32_t i = t; i < p.ncell + 16; i += all) b.cnt[i] = 0;
     for (uint32_t i = t; i < tiles; i += all) b.tile_state[i] = 0;
     for (uint32_t i = t; i < chunks; i += all) {
@@ -1963,13 +1991,6 @@ __global__ __launch_bounds__(256) void noalloc_init_kernel(FrameParams p, FrameB
     for (uint32_t i = t; i < (uint32_t)(kClasses * (kSlices + 1)); i += all) b.class_ctr[i * kCtrStride] = 0;
     if (t == 0) {
         *b.epoch = 1;  // status words start at 0, never valid
-        *b.error = 0;
-    }
-    uint32_t s = 0, n = 0;
-    if (t < p.ncell) {  // the grid covers the cells
-        s = min(indices[1 + t], p.n);
-        const uint32_t e = min(indices[2 + t], p.n);
-        n = e > s ? e - s : 0u;
     }
     if (n <= kOwnCells)
         for (uint32_t j = s; j < s + n; ++j) {
@@ -1982,9 +2003,12 @@ __global__ __launch_bounds__(256) void noalloc_init_kernel(FrameParams p, FrameB
         big &= big - 1;
         const uint32_t s0 = (uint32_t)__shfl((int)s, l, 64), n0 = (uint32_t)__shfl((int)n, l, 64);
         const uint32_t c0 = (uint32_t)__shfl((int)t, l, 64);
-        for (uint32_t j = s0 + lane_id(); j < s0 + n0; j += 64) {
-            b.src[j] = j;
-            b.key[j] = c0;
+        for (uint32_t r = 0; r < n0; r += kLongCell) {
+            if (r && __hip_atomic_load(b.error, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) return;
+            for (uint32_t j = s0 + r + lane_id(); j < s0 + min(n0, r + kLongCell); j += 64) {
+                b.src[j] = j;
+                b.key[j] = c0;
+            }
         }
     }
 }
