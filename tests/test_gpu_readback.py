@@ -321,3 +321,23 @@ def test_noalloc_frame_leaves_a_bad_triple(oracle, fault, offset):
                 assert_packed(got, want, f"{fault} offset={offset} {'bad' if offsets is bad else 'good'}")
             finally:
                 hip.free(di, dp, dv)
+
+
+def test_autotune_leaves_what_changes_no_launch():
+    """A grid that scans by chunks has no scan shape to choose, and a small
+    world's grids of queued cells launch the same blocks: the autotuner keeps
+    them, whichever trial a clock finds the shortest."""
+    rng = np.random.default_rng(70)
+    say("[readback] autotune")
+    with World(WrachConfig(dimensions=(4096, 2048), cell_size=1)) as w:
+        w.add_particles(f32(rng.uniform(0, (4096, 100), (3000, 2))), f32(rng.uniform(-1, 1, (3000, 2))))
+        for shape in ((1024, 8), (512, 16), (1024, 64)):
+            w.set_tuning(scan_threads=shape[0], scan_items=shape[1])
+            got = w.autotune(2)
+            assert (got["scan_threads"], got["scan_items"]) == shape
+    with World(WrachConfig(dimensions=(512, 512), cell_size=1)) as w:
+        w.add_particles(f32(rng.uniform(0, 512, (6000, 2))), f32(rng.uniform(-1, 1, (6000, 2))))
+        grid = w.tuning()["cells_grid"]
+        assert grid // 2 >= 6000 // 64 + 64  # every candidate launches as many
+        for _ in range(4):
+            assert w.autotune(2)["cells_grid"] == grid

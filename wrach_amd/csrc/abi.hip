@@ -1524,11 +1524,14 @@ int wrach_load_packed(wrach_ctx *c, const uint32_t *indices, size_t n_indices, c
 
 namespace {
 
-// Candidate grids of the cells kernel around the creation default g0.
-void cells_grid_candidates(uint32_t g0, std::vector<uint32_t> &out) {
+// Candidate grids of the cells kernel around the creation default g0, the
+// first of those that launch alike for n particles.
+void cells_grid_candidates(uint32_t g0, uint32_t n, std::vector<uint32_t> &out) {
     out.clear();
-    for (const uint32_t g : {g0, std::max(1u, g0 * 3 / 4), std::max(1u, g0 / 2), g0 + g0 / 2})
-        if (std::find(out.begin(), out.end(), g) == out.end()) out.push_back(g);
+    for (const uint32_t g : {g0, std::max(1u, g0 * 3 / 4), std::max(1u, g0 / 2), g0 + g0 / 2}) {
+        const auto alike = [&](uint32_t o) { return wrach::cells_blocks(o, n) == wrach::cells_blocks(g, n); };
+        if (std::find_if(out.begin(), out.end(), alike) == out.end()) out.push_back(g);
+    }
 }
 
 wrach_tuning current_tuning(const wrach_ctx *c) {
@@ -1663,15 +1666,16 @@ int wrach_autotune(wrach_ctx *c, uint32_t frames, wrach_tuning *out) {
     uint32_t scan = c->buf.scan_shape, scatter = c->buf.scatter_shape, grid = c->buf.cells_grid;
     float best_us = 0.0f;
     int rc = WRACH_OK;
-    // One knob at a time, the others at their current best.
-    for (int knob = 0; knob < 3 && rc == WRACH_OK; ++knob) {
+    // One knob at a time, the others at their current best.  Large grids scan
+    // without tiles of the scan's shape: nothing to choose.
+    for (int knob = wrach::relative_offsets(c->ncell) ? 1 : 0; knob < 3 && rc == WRACH_OK; ++knob) {
         std::vector<uint32_t> cand;
         if (knob == 0)
             for (int i = 0; i < wrach::kNumScanShapes; ++i) cand.push_back((uint32_t)i);
         else if (knob == 1)
             for (int i = 0; i < wrach::kNumScatterShapes; ++i) cand.push_back((uint32_t)i);
         else
-            cells_grid_candidates(c->cells_grid0, cand);
+            cells_grid_candidates(c->cells_grid0, n, cand);
         uint32_t best = knob == 0 ? scan : knob == 1 ? scatter : grid;
         float best_here = -1.0f;
         for (const uint32_t v : cand) {

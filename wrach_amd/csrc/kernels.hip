@@ -3229,11 +3229,7 @@ hipError_t launch_collide(const FrameParams &p, const FrameBuffers &b, hipStream
 
 hipError_t launch_cells(const FrameParams &p, const FrameBuffers &b, hipStream_t stream,
                         hipEvent_t start, hipEvent_t stop) {
-    // A small world's cells are few: at most n / 64 + 64 blocks, about what
-    // its particles could need with every list's last item partly filled (16k
-    // particles: 320 of the 1,024 that fit the device; 100 frames 2.33 ms with
-    // all of them, 2.29 with 64 to 320).
-    return launch(cells_kernel, std::min(b.cells_grid, p.n / 64 + 64), kCollideBlock, stream, start, stop, p, b);
+    return launch(cells_kernel, cells_blocks(b.cells_grid, p.n), kCollideBlock, stream, start, stop, p, b);
 }
 
 // Asked once per device (a frame without a context asks on every call).
