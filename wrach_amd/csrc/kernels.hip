@@ -3138,7 +3138,12 @@ __global__ __launch_bounds__(256, 4) void learn_features_kernel(FrameParams p, F
     if (__ballot(tie || more) != 0) {  // every lane votes
         // Lanes with a tie from their first candidate on, lanes with more
         // than kKeyCands from there on; a candidate past the 16th in fixed
-        // point is past it exactly.
+        // point is past it exactly.  Two at a time, their loads in flight
+        // together: one by one, positions of few bits (ties in most wavefronts:
+        // 250k of 1/64 on a lattice 296 us, 225 so) and crowds (240k, 520
+        // candidates each: 724 us, 535) took longer than with every candidate's
+        // 64-bit key in the network (245, 561); four at a time 224 and 507, but
+        // loose worlds take 3% longer.
         const uint32_t last = ck[kNbrs - 1] >> kNumberBits;
         unsigned long long key[kNbrs];
 #pragma unroll
@@ -3147,13 +3152,20 @@ __global__ __launch_bounds__(256, 4) void learn_features_kernel(FrameParams p, F
                          ? ~0ull
                          : ((unsigned long long)__float_as_uint(squared_distance(a.pos[near[r]], q)) << 32) | near[r];
         const uint32_t begin = tie ? 0u : kKeyCands, end = tie || more ? m5 : 0u;
-        for (uint32_t u = __ballot(tie) != 0 ? 0u : kKeyCands; __ballot(u < end) != 0; ++u) {
-            if (u < begin || u >= end) continue;
-            const uint32_t j = WRACH_CAND(u);
-            if (j == i) continue;
-            const float sq = squared_distance(a.pos[j], q);
-            if ((uint32_t)fminf(sq * to_fixed, (float)kDistMax) > last) continue;
-            insert16(a.pos, a.vel, key, ((unsigned long long)__float_as_uint(sq) << 32) | j);
+        for (uint32_t u = __ballot(tie) != 0 ? 0u : kKeyCands; __ballot(u < end) != 0; u += 2) {
+            uint32_t j[2];
+            float sq[2];
+#pragma unroll
+            for (int v = 0; v < 2; ++v) {
+                j[v] = u + v >= begin && u + v < end ? WRACH_CAND(u + v) : i;
+                sq[v] = squared_distance(a.pos[j[v]], q);
+            }
+#pragma unroll
+            for (int v = 0; v < 2; ++v) {
+                if (j[v] == i) continue;
+                if ((uint32_t)fminf(sq[v] * to_fixed, (float)kDistMax) > last) continue;
+                insert16(a.pos, a.vel, key, ((unsigned long long)__float_as_uint(sq[v]) << 32) | j[v]);
+            }
         }
 #pragma unroll
         for (int r = 0; r < kNbrs; ++r)
