@@ -2390,8 +2390,14 @@ __device__ __forceinline__ void stencil_hit(float dx, float dy, PairSums &s) {
 // first particle and length, the lengths 0 over the budget.
 struct StencilRows {
     uint32_t rs[3], len[3];
-    uint32_t half;  // rs[1] + half: the particle's own cell's start
+    uint32_t half;  // rs[1] + half: the particle's own cell's start; kBeside: see below
 };
+
+// In StencilRows::half (at most kStencilBudget by itself): the particle lies
+// beside the cell that holds it, as a loaded triple may say.  It need not be in
+// the middle row then.
+constexpr uint32_t kBeside = 0x8000u;
+static_assert(kStencilBudget < kBeside, "half and its flag share 16 bits");
 
 // The rows of a particle in cell k.  More than kStencilBudget particles in
 // them: none, and `over` (a bound on the work of one lane).
@@ -2518,7 +2524,8 @@ __device__ __forceinline__ void stencil_long(const float2 *pin, uint32_t i, floa
 // terms, and with SUMS the sum of the overlaps.  (A lane without a particle
 // has empty rows.)  HALF: each pair once -- the later particles of its own
 // cell, the cell to its right and the three cells above; every other pair of
-// its 3x3 cells is one of these seen from the other particle.
+// its 3x3 cells is one of these seen from the other particle (no particle is
+// kBeside then).
 template <bool MOVE, bool SUMS, bool HALF>
 __device__ __forceinline__ PairSums stencil_particle(const float2 *pin, uint32_t i, float xi, float yi,
                                                      StencilRows r, float2 *list) {
@@ -2526,13 +2533,13 @@ __device__ __forceinline__ PairSums stencil_particle(const float2 *pin, uint32_t
         r.len[0] = 0;
         r.rs[1] += r.half;
         r.len[1] -= r.half;
+        r.half = 0;
     }
     PairSums s;
-    // The short path leaves out particle i in its own cell's row alone.  Where
-    // a particle lies beside the cell that holds it (a loaded triple may say
-    // so), it is met in another: stencil_long tests every row.
-    const bool beside = (i - r.rs[0] < r.len[0]) | (i - r.rs[2] < r.len[2]);
-    if (__ballot((max(max(r.len[0], r.len[1]), r.len[2]) > kShortRow) | beside) == 0) {
+    // The short path leaves out particle i in the middle row alone;
+    // stencil_long does in every row, and takes those that lie beside their
+    // cell.  (Without kBeside half is at most len[1].)
+    if (__ballot(max(max(r.len[0], r.len[1]), max(r.len[2], r.half)) > kShortRow) == 0) {
         stencil_short<MOVE, SUMS, HALF>(pin, i, xi, yi, r, list, s);
         return s;
     }
@@ -2636,14 +2643,13 @@ __device__ __forceinline__ StencilRows stencil_lane(const FrameParams &p, const 
     }
     i = a.perm ? a.perm[t] : t;
     q = a.pin[i];
+    const uint32_t held = b.key[i];
     const uint32_t k = a.rows_from == kRowsOfCell ? a.cell[i] : position_key(p, particle_grid(p, b, i), q.x, q.y);
-    bool one_sided = a.rows_from == kRowsOfPosition && k != b.key[i];
-    if (k < p.ncell) {
-        bool over;
-        r = stencil_rows_of(p, b, k, over);
-        one_sided |= over;
-    }
-    if (one_sided) atomicOr(&a.words[kOneSidedWord], 1u);
+    const bool beside = k != held;
+    bool over = false;
+    if (k < p.ncell) r = stencil_rows_of(p, b, k, over);
+    if (beside) r.half |= kBeside;
+    if (beside | over) atomicOr(&a.words[kOneSidedWord], 1u);
     if (a.rows_from == kRowsOfPosition && !a.record) a.cell[i] = k;
     if (a.record) {
         a.rows[t] = make_uint4(r.rs[0], r.rs[1], r.rs[2], r.len[0] | (r.half << 16));
@@ -2997,6 +3003,7 @@ __global__ __launch_bounds__(256, 4) void learn_features_kernel(FrameParams p, F
     uint32_t i = on ? lane_t : 0u;  // a lane past the particles reads particle 0 and writes nothing
     if (on && a.perm) i = a.perm[lane_t];
     const float2 q = a.pos[i], w = a.vel[i];
+    const uint32_t held = b.key[i];
     uint32_t rs[5], cum[5], m5 = 0;  // a row's first particle; candidates before its row
     StencilRows r3;
 #pragma unroll
@@ -3063,8 +3070,10 @@ __global__ __launch_bounds__(256, 4) void learn_features_kernel(FrameParams p, F
         const bool over = tot3 > kStencilBudget;
         r3.half = over ? 0u : min(max(r3.rs[1], at[16]), re1) - r3.rs[1];
         if (over) r3.len[0] = r3.len[1] = r3.len[2] = 0;
+        const bool beside = k != held;
+        if (beside) r3.half |= kBeside;
         // What the passes that follow need (stencil_lane).
-        if (a.words && (over || k != b.key[i])) atomicOr(&a.words[kOneSidedWord], 1u);
+        if (a.words && (beside | over)) atomicOr(&a.words[kOneSidedWord], 1u);
         if (a.rows) {
             a.rows[lane_t] = make_uint4(r3.rs[0], r3.rs[1], r3.rs[2], r3.len[0] | (r3.half << 16));
             a.rows2[lane_t] = make_uint2(r3.len[1] | (r3.len[2] << 16), i);
