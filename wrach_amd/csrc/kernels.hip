@@ -2987,7 +2987,7 @@ __device__ __forceinline__ uint32_t candidate(uint32_t u, uint32_t c1, uint32_t 
 // comparator, as it inserts those past the first 128.
 //
 // 1M particles: 181 us and 4,222 vector instructions a wavefront before, now
-// 122 (and 6.5 for learn_state_kernel) and 2,750.  What bounds it is the L1:
+// 118 (and 6.5 for learn_state_kernel) and 2,750.  What bounds it is the L1:
 // 2,700 accesses a wavefront, most of them the 16 neighbours' gathers, one of
 // 16 bytes each since positions and velocities lie side by side (two of 8
 // before), and the candidates'; rows stored from each lane were 450 more.
@@ -3149,10 +3149,10 @@ __global__ __launch_bounds__(256, 4) void learn_features_kernel(FrameParams p, F
         // than kKeyCands from there on; a candidate past the 16th in fixed
         // point is past it exactly.  Two at a time, their loads in flight
         // together: one by one, positions of few bits (ties in most wavefronts:
-        // 250k of 1/64 on a lattice 296 us, 225 so) and crowds (240k, 520
-        // candidates each: 724 us, 535) took longer than with every candidate's
-        // 64-bit key in the network (245, 561); four at a time 224 and 507, but
-        // loose worlds take 3% longer.
+        // 250k of 1/64 on a lattice 292 us, 229 so) and crowds (240k, 520
+        // candidates each: 702 us, 544) took longer than with every candidate's
+        // 64-bit key in the network (245, 562).  Four at a time spill registers
+        // (158 us instead of 118 for 1M loose particles).
         const uint32_t last = ck[kNbrs - 1] >> kNumberBits;
         unsigned long long key[kNbrs];
 #pragma unroll
@@ -3178,7 +3178,7 @@ __global__ __launch_bounds__(256, 4) void learn_features_kernel(FrameParams p, F
         }
 #pragma unroll
         for (int r = 0; r < kNbrs; ++r)
-            if (tie || more) near[r] = key[r] != ~0ull ? (uint32_t)key[r] : 0xffffffffu;
+            near[r] = (uint32_t)key[r];  // ~0 where there is none
     }
 #undef WRACH_CAND
     // The rows through LDS, half a row at a time, so that a wavefront stores
