@@ -1156,7 +1156,6 @@ int ensure_stencil(wrach_ctx *c) {
     return WRACH_OK;
 }
 
-// The learned frame's buffers: feature rows and a third position buffer.
 // The passes and features read idx; a large grid's frames leave offsets there
 // only with a solver that has them (FrameParams::idx_read).
 int offsets_for_passes(wrach_ctx *c) {
@@ -1165,6 +1164,7 @@ int offsets_for_passes(wrach_ctx *c) {
     return WRACH_OK;
 }
 
+// The learned frame's buffers: feature rows and a third position buffer.
 int ensure_learned_frame(wrach_ctx *c) {
     const int offsets = offsets_for_passes(c);
     if (offsets) return offsets;
